@@ -260,12 +260,10 @@ def run(state):
         return {"y": y, "mean": mean, "rstd": rstd, "dx": dx, "dgamma": dg, "dbeta": db}
     if kind == "batchnorm":
         x, g, b, rm, rv = (state[n] for n in ("x", "gamma", "beta", "running_mean", "running_var"))
-        y, mean, rstd = ops.batchnorm2d_fwd(x, g, b, 1e-5, 0.1, rm, rv, residual=state["res"], relu=True)
-        if case["residual"]:
-            dz = ops.relu_bwd(y, state["dy"])
-            dx, dg, db = ops.batchnorm2d_bwd(x, dz, mean, rstd, g)
-        else:
-            dx, dg, db = ops.batchnorm2d_bwd(x, state["dy"], mean, rstd, g, beta=b, relu=True)
+        # the branch's last BatchNorm takes the skip addition and the final ReLU,
+        # whose backward the next block's fork has already applied to dy
+        y, mean, rstd = ops.batchnorm2d_fwd(x, g, b, 1e-5, 0.1, rm, rv, residual=state["res"], relu=case["residual"])
+        dx, dg, db = ops.batchnorm2d_bwd(x, state["dy"], mean, rstd, g)
         return {"y": y, "mean": mean, "rstd": rstd, "running_mean": rm, "running_var": rv, "dx": dx, "dgamma": dg,
                 "dbeta": db}
     dl, loss = ops.softmax_xent_bwd(state["logits"], state["labels"], label_smoothing=case["smoothing"])
@@ -316,10 +314,11 @@ def work(case):
 def tolerance(case):
     kind = case["kind"]
     # A ReLU input within rounding of zero takes the other branch, and its
-    # channel's gradients change with it (as measured against 64 bits: up to
-    # 3e-4 of the small CNN's first layer's, 3e-3 of the ResNet's).
+    # channel's gradients change with it (as measured against 64 bits: 3e-4 of
+    # the small CNN's first layer's at batch 487, more at a smaller one; up to
+    # 3e-3 of the ResNet's).
     if kind == "small_cnn":
-        return {"rel": 2e-3, "max": 2e-2}
+        return {"rel": 1e-2, "max": 0.3}
     if kind == "resnet18":
         return {"rel": 2e-2, "max": 0.9}
     if case["dtype"] == "f32":
@@ -365,13 +364,12 @@ def exact(case, seed):
         var = (x - per(mean)).square().mean((0, 2, 3))
         rstd = (var + 1e-5).rsqrt()
         xh = (x - per(mean)) * per(rstd)
-        z = xh * per(s["gamma"]) + per(s["beta"])
+        z, dz = xh * per(s["gamma"]) + per(s["beta"]), s["dy"]
         if case["residual"]:
-            z = z + s["res"]
-        dz = s["dy"] * (z > 0)
+            z = (z + s["res"]).relu()
         dg, db = (dz * xh).sum((0, 2, 3)), dz.sum((0, 2, 3))
         dx = per(s["gamma"] * rstd) * (dz - per(db / count) - xh * per(dg / count))
-        return {"y": z.relu(), "mean": mean, "rstd": rstd, "running_mean": 0.1 * mean,
+        return {"y": z, "mean": mean, "rstd": rstd, "running_mean": 0.1 * mean,
                 "running_var": 0.9 + 0.1 * var * count / max(1, count - 1), "dx": dx, "dgamma": dg, "dbeta": db}
     logits, labels, eps = s["logits"], s["labels"], case["smoothing"]
     n, c = logits.shape
