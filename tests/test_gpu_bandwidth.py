@@ -1,6 +1,8 @@
 """GPU parity of the bandwidth-bound kernels against the CPU oracle, through
 the C ABI (thot_amd.ops -> libnott_hip.so).  Same seeded inputs on both sides;
 bf16 inputs are rounded once and the oracle sees the rounded values."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -475,6 +477,43 @@ def test_softmax_xent(ops, oracle, dt, n, c, eps, ignore):
     rows = np.nonzero(y != -100)[0]
     if eps == 0.0:
         assert (host(dl)[rows, y[rows]] < 0).all()
+
+
+# Rows that are not whole 16-byte groups, or longer than the vector path takes:
+# at the edges of what a thread holds (64 x 16, 256 x 32, 512 x 32, 512 x 64,
+# 512 x 104 and 1024 x 104 elements), past the last (the rest is streamed), and
+# below two groups with too many rows for one workgroup.
+XENT_ANY = [(4100, 7, 0.0), (4100, 17, 0.1), (4097, 33, 0.0), (70, 65, 0.1), (50, 1023, 0.0), (40, 1025, 0.1),
+            (20, 8191, 0.0), (20, 8193, 0.1), (9, 16383, 0.1), (9, 16385, 0.1), (7, 32767, 0.0), (7, 32776, 0.1),
+            (5, 53247, 0.1), (5, 53256, 0.0), (4, 106496, 0.1), (4, 106497, 0.0), (3, 128256, 0.1), (3, 250001, 0.1)]
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n,c,eps", XENT_ANY)
+@pytest.mark.parametrize("at", [(0, 0), (1, 1), (3, 2)], ids=lambda a: "off%d_%d" % a)
+def test_softmax_xent_any_row(ops, oracle, dt, n, c, eps, at):
+    """Any row length from any element offset of the buffers (the second number:
+    the gradient's), the elements around the rows left alone.  The oracle sums
+    in double, so the tolerance is that of the other cross-entropy tests."""
+    print(f"xent any {dt} {n}x{c} at {at}", flush=True)
+    g = rng(n + c)
+    z = host_input(g.standard_normal((n, c)) * 2.0, dt)
+    z[0, c // 2] = -9984.0                     # a masked class: probability 0 (−inf on the GPU)
+    y = g.integers(0, c, n).astype(np.int64)
+    y[0] = 0 if c // 2 else 1
+    y[1], y[2] = -100, c - 1
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    zb = torch.zeros(n * c + 8, dtype=tdt, device="cuda")
+    db = torch.full((n * c + 8,), 7.0, dtype=tdt, device="cuda")
+    zv, dv = zb[at[0]:at[0] + n * c].view(n, c), db[at[1]:at[1] + n * c].view(n, c)
+    zv.copy_(dev(z, dt))
+    if eps == 0.0:                             # (a smoothed loss of −inf is infinite)
+        zv[0, c // 2] = -math.inf
+    _, loss = ops.softmax_xent_bwd(zv, torch.from_numpy(y).cuda(), label_smoothing=eps, out=dv)
+    dle, losse = oracle.softmax_xent(z, y, eps)
+    check(host(dv), dle, dt, "xent dlogits")
+    check(loss.item(), losse, "f32", "xent loss", rtol=1e-5)
+    assert (db[:at[1]] == 7).all() and (db[at[1] + n * c:] == 7).all()
 
 
 @pytest.mark.parametrize("dt", DTYPES)

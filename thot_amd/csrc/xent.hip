@@ -73,12 +73,12 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
 // is kept in v, and the gradient is scale·(p/Σp − ε/C − (1 − ε)·[j = y])
 // (the label's term applied once, by the thread that holds it); the row sum
 // of the logits is formed only when label smoothing needs it.
-template <typename T, int NT, int EPT, bool VEC>
+template <typename T, int NT, int EPT>
 __device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int64_t y, const T* __restrict__ z,
                                               int64_t c, float smoothing, float grad_scale, int nv,
                                               T* __restrict__ dz, float* __restrict__ row_loss, float* red) {
     constexpr int NWAVES = NT / 64;
-    constexpr int G = VEC ? Pack16<T>::N : 1;
+    constexpr int G = Pack16<T>::N;
     constexpr int NG = EPT / G;
     constexpr float kLog2e = 1.4426950408889634f;
     const int ci = (int)c;
@@ -88,14 +88,10 @@ __device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int6
         for (int g = 0; g < NG; ++g) {
             const int j0 = (g * NT + (int)threadIdx.x) * G;
             if (j0 >= ci) continue;
-            if constexpr (VEC) {
-                float t[G];
+            float t[G];
 #pragma unroll
-                for (int e = 0; e < G; ++e) t[e] = 0.f;
-                Pack16<T>::template st<true>(dz + j0, t);
-            } else {
-                Io<T>::st(dz, j0, 0.f);
-            }
+            for (int e = 0; e < G; ++e) t[e] = 0.f;
+            Pack16<T>::template st<true>(dz + j0, t);
         }
         if (threadIdx.x == 0 && row_loss) row_loss[row] = 0.f;
         return;
@@ -135,8 +131,7 @@ __device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int6
             for (int e = 0; e < G; ++e)
                 if (j0 + e == yi) t[e] -= scale * hit;
         }
-        if constexpr (VEC) Pack16<T>::template st<true>(dz + j0, t);
-        else Io<T>::st(dz, j0, t[0]);
+        Pack16<T>::template st<true>(dz + j0, t);
     }
     if (threadIdx.x == 0 && row_loss) {
         const float zy = Io<T>::ld(z, y);
@@ -184,64 +179,231 @@ __global__ __launch_bounds__(NT) void xent_rows_vec_kernel(const T* __restrict__
         }
         const int64_t y = ny;
         if (row + gridDim.x < n) fetch(row + gridDim.x);
-        xent_row_body<T, NT, EPT, true>(v, row, y, logits + row * c, c, smoothing, grad_scale, nv,
+        xent_row_body<T, NT, EPT>(v, row, y, logits + row * c, c, smoothing, grad_scale, nv,
                                         dlogits + row * c, row_loss, red);
     }
 }
 
-// Element path (unaligned rows or c not a multiple of G): one workgroup per
-// row, single elements strided by NT.
-template <typename T, int NT, int EPT>
-__global__ __launch_bounds__(NT) void xent_row_kernel(const T* __restrict__ logits, const int64_t* __restrict__ labels,
-                                                      int64_t c, float smoothing, float grad_scale,
-                                                      const int* __restrict__ nvalid, T* __restrict__ dlogits,
-                                                      float* __restrict__ row_loss) {
-    __shared__ float red[2 * (NT / 64)];
-    const int64_t row = blockIdx.x;
-    const T* z = logits + row * c;
-    float v[EPT];
-#pragma unroll
-    for (int g = 0; g < EPT; ++g) {
-        const int64_t j0 = (int64_t)g * NT + threadIdx.x;
-        v[g] = j0 < c ? Io<T>::ld(z, j0) : -INFINITY;
+// Block-wide maximum / pair of sums with one LDS word per wave and a second
+// wave reduction (the unrolled reads of block_max and block_sum2 would cost the
+// wide rows their registers).  `red` is not reused by a later call.
+template <int NWAVES>
+__device__ __forceinline__ float row_max(float v, float* red) {
+    v = wave_max(v);
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return wave_max(lane < NWAVES ? red[lane] : -INFINITY);
+}
+template <int NWAVES>
+__device__ __forceinline__ void row_sum2(float& a, float& b, float* red) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) {
+        red[threadIdx.x >> 6] = a;
+        red[NWAVES + (threadIdx.x >> 6)] = b;
     }
-    xent_row_body<T, NT, EPT, false>(v, row, labels[row], z, c, smoothing, grad_scale, *nvalid, dlogits + row * c,
-                                     row_loss, red);
+    __syncthreads();
+    a = wave_sum(lane < NWAVES ? red[lane] : 0.f);
+    b = wave_sum(lane < NWAVES ? red[NWAVES + lane] : 0.f);
 }
 
-// Rows too long for registers: three passes over the row (the re-reads are
-// served from L2 / MALL for rows of a few hundred KiB).
+// A group of −inf.
 template <typename T>
-__global__ __launch_bounds__(256) void xent_long_kernel(const T* __restrict__ logits, const int64_t* __restrict__ labels,
-                                                        int64_t c, float smoothing, float grad_scale,
-                                                        const int* __restrict__ nvalid, T* __restrict__ dlogits,
-                                                        float* __restrict__ row_loss) {
-    __shared__ float red[8];
+__device__ __forceinline__ typename Pack16<T>::Raw minus_inf() {
+    if constexpr (sizeof(T) == 2) return u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+    else return f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+}
+
+// Rows of any length at any alignment: c not a multiple of the 16-byte group,
+// rows past the vector path's 32768, views that start off a 16-byte boundary.
+// Each row is taken as its own 16-byte aligned groups, every one a single
+// access, and the fewer than 2·G columns before the first and after the last
+// whole group, one per thread (an element each, by itself).
+//
+// The first NT·NG groups are held in registers: one HBM read and one write, as
+// in the vector path.  With REST the groups past them are streamed twice,
+// before the held ones are loaded (a running maximum and sum per thread) and
+// after they are stored, when their registers are free; the second read of a
+// row of a few hundred KiB comes from the caches.  104 elements are what a
+// thread holds at 4 waves per SIMD (128 VGPRs), which keeps two 512-thread rows
+// (up to 53248 columns) or one 1024-thread row on a CU.  Bound by memory: it
+// moves 4096 x 50257 fp32 at 5.1 TB/s (324 us), 8192 x 128256 bf16 at 5.4 TB/s
+// (780 us) and 2048 x 151936 fp32 at 5.2 TB/s (482 us); three passes of single
+// elements per row took 846, 3529 and 1247 us.
+// inf_counts: whether a logit of −inf enters the smoothed loss's Σ z_j.
+template <typename T, int NT, int EPT, bool REST>
+__global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
+    const T* __restrict__ logits, const int64_t* __restrict__ labels, int64_t c, float smoothing, float grad_scale,
+    const int* __restrict__ nvalid, T* __restrict__ dlogits, float* __restrict__ row_loss, int inf_counts) {
+    constexpr int G = Pack16<T>::N;
+    constexpr int NG = EPT / G;
+    constexpr int NWAVES = NT / 64;
+    constexpr int kUnroll = 4;       // streamed groups in flight per thread
+    constexpr float kLog2e = 1.4426950408889634f;
+    __shared__ float red[3 * NWAVES];
+    const int tid = (int)threadIdx.x;
+    const float off = smoothing / (float)c, hit = 1.f - smoothing;
     const int64_t row = blockIdx.x;
     const T* z = logits + row * c;
     T* dz = dlogits + row * c;
     const int64_t y = labels[row];
+    // [0, s0) and [s0 + groups·G, c) are the single columns; thread i
+    // holds the i-th of them (ej: its column, none for the other threads)
+    const int s0 = (int)min((int64_t)((G - ((uintptr_t)z / sizeof(T)) % G) % G), c);
+    const int64_t groups = (c - s0) / G, tail = s0 + groups * G;
+    const int64_t ej = tid < s0 ? tid : tid - s0 < (int)(c - tail) ? tail + (tid - s0) : -1;
+    const T* zb = z + s0;
+    T* db = dz + s0;
+    const bool vec_st = ((uintptr_t)db % 16) == 0;
+    // group g·NT + tid is held iff g·NT < rem
+    const int rem = (int)min(groups, (int64_t)NT * NG) - tid;
     if (!(y >= 0 && y < c)) {
-        for (int64_t j = threadIdx.x; j < c; j += 256) Io<T>::st(dz, j, 0.f);
-        if (threadIdx.x == 0 && row_loss) row_loss[row] = 0.f;
+        // Ignored (or out-of-range) row: zero gradient, no loss.
+        for (int64_t j = tid; j < c; j += NT) Io<T>::st(dz, j, 0.f);
+        if (tid == 0 && row_loss) row_loss[row] = 0.f;
         return;
     }
-    float mx = -INFINITY;
-    for (int64_t j = threadIdx.x; j < c; j += 256) mx = fmaxf(mx, Io<T>::ld(z, j));
-    mx = block_max<4>(mx, red);
+    float mx = ej >= 0 ? Io<T>::ld(z, ej) : -INFINITY;
+    const float ez = mx;
     float se = 0.f, sz = 0.f;
-    for (int64_t j = threadIdx.x; j < c; j += 256) {
-        const float t = Io<T>::ld(z, j);
-        se += __expf(t - mx);
-        sz += t;
+    if constexpr (REST) {
+        for (int64_t k = (int64_t)NT * NG + tid; k < groups; k += NT * kUnroll) {
+            float t[kUnroll][G];
+            float m = mx;
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                if (k + u * NT < groups) {
+                    Pack16<T>::ld(zb + (k + u * NT) * G, t[u]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < G; ++e) t[u][e] = -INFINITY;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+                for (int e = 0; e < G; ++e) m = fmaxf(m, t[u][e]);
+            // Nothing but −inf so far: no maximum to subtract (−inf − (−inf)
+            // is no exponent); a NaN still reaches the sum.
+            const bool none = m == -INFINITY;
+            const float ml = none ? 0.f : m * kLog2e;
+            se = none ? se : se * __builtin_amdgcn_exp2f((mx - m) * kLog2e);
+            mx = m;
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+                for (int e = 0; e < G; ++e) {
+                    se += __builtin_amdgcn_exp2f(fmaf(t[u][e], kLog2e, -ml));
+                    if (k + u * NT < groups && (inf_counts || t[u][e] != -INFINITY)) sz += t[u][e];
+                }
+        }
     }
-    block_sum2<4>(se, sz, red);
-    const float lse = mx + __logf(se);
+    // Every load is of a whole group of the row (past the last held one, that
+    // one again); a row of fewer than 2·G columns may have none.
+    typename Pack16<T>::Raw raw[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) raw[g] = minus_inf<T>();
+    if (groups > 0) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+            raw[g] = Pack16<T>::template raw<true>(zb + (unsigned)(tid + min(g * NT, rem - 1)) * G);
+    }
+    float m = mx;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        raw[g] = g * NT < rem ? raw[g] : minus_inf<T>();
+        float t[G];
+        Pack16<T>::unpack(raw[g], t);
+#pragma unroll
+        for (int e = 0; e < G; ++e) m = fmaxf(m, t[e]);
+        // unpacked again below: held packed until then, not as EPT floats more
+        asm volatile("" : "+v"(raw[g]));
+    }
+    m = row_max<NWAVES>(m, red);
+    const float ml = m * kLog2e;
+    const float ep = __builtin_amdgcn_exp2f(fmaf(ez, kLog2e, -ml));
+    const float zy = Io<T>::ld(z, y);   // (before the stores: dlogits may be logits)
+    if constexpr (REST) se = mx == -INFINITY ? se : se * __builtin_amdgcn_exp2f((mx - m) * kLog2e);
+    se += ej >= 0 ? ep : 0.f;
+    if (smoothing != 0.f) {
+        if (ej >= 0 && (inf_counts || ez != -INFINITY)) sz += ez;
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+            if (g * NT < rem) {
+                float t[G];
+                Pack16<T>::unpack(raw[g], t);
+#pragma unroll
+                for (int e = 0; e < G; ++e)
+                    if (inf_counts || t[e] != -INFINITY) sz += t[e];
+                asm volatile("" : "+v"(raw[g]));
+            }
+    }
+    float v[EPT];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        float t[G];
+        Pack16<T>::unpack(raw[g], t);
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            v[g * G + e] = __builtin_amdgcn_exp2f(fmaf(t[e], kLog2e, -ml));
+            se += v[g * G + e];
+        }
+    }
+    row_sum2<NWAVES>(se, sz, red + NWAVES);
+    const float lse = m + __logf(se);
     const float scale = grad_scale / (float)(*nvalid);
-    const float off = smoothing / (float)c, hit = 1.f - smoothing;
-    for (int64_t j = threadIdx.x; j < c; j += 256)
-        Io<T>::st(dz, j, scale * (__expf(Io<T>::ld(z, j) - lse) - off - (j == y ? hit : 0.f)));
-    if (threadIdx.x == 0 && row_loss) row_loss[row] = hit * (lse - Io<T>::ld(z, y)) + off * ((float)c * lse - sz);
+    const float ga = scale / se, gb = -scale * off;
+    // The label's group, counted from this thread's first, and its element there.
+    const int64_t yk = y >= s0 && y < tail ? (y - s0) / G - tid : -1;
+    const int ye = yk >= 0 ? (int)((y - s0) % G) : 0;
+    const int yh = yk < NT * NG ? (int)yk : -1;
+    auto grad = [&](bool mine, float (&t)[G]) {
+#pragma unroll
+        for (int e = 0; e < G; ++e) t[e] = fmaf(t[e], ga, gb);
+        if (mine) {
+#pragma unroll
+            for (int e = 0; e < G; ++e)
+                if (e == ye) t[e] -= scale * hit;
+        }
+    };
+    auto put = [&](T* p, const float (&t)[G]) {
+        if (vec_st) {
+            Pack16<T>::template st<true>(p, t);
+        } else {
+#pragma unroll
+            for (int e = 0; e < G; ++e) Io<T>::st(p, e, t[e]);
+        }
+    };
+    if (ej >= 0) Io<T>::st(dz, ej, fmaf(ep, ga, gb) - (ej == y ? scale * hit : 0.f));
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g * NT >= rem) continue;
+        float t[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) t[e] = v[g * G + e];
+        grad(g * NT == yh, t);
+        put(db + g * NT * G + (unsigned)(tid * G), t);
+    }
+    if constexpr (REST) {
+        for (int64_t k = (int64_t)NT * NG + tid; k < groups; k += NT * kUnroll) {
+            float t[kUnroll][G];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+                if (k + u * NT < groups) Pack16<T>::ld(zb + (k + u * NT) * G, t[u]);
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                if (k + u * NT >= groups) break;
+#pragma unroll
+                for (int e = 0; e < G; ++e) t[u][e] = __builtin_amdgcn_exp2f(fmaf(t[u][e], kLog2e, -ml));
+                grad(k + u * NT - tid == yk, t[u]);
+                put(db + (k + u * NT) * G, t[u]);
+            }
+        }
+    }
+    if (tid == 0 && row_loss)
+        row_loss[row] = hit * (lse - zy) + (smoothing != 0.f ? off * ((float)c * lse - sz) : 0.f);
 }
 
 __global__ __launch_bounds__(1024) void xent_loss_kernel(const float* __restrict__ row_loss, int64_t n,
@@ -255,15 +417,64 @@ __global__ __launch_bounds__(1024) void xent_loss_kernel(const float* __restrict
 
 __global__ void xent_nan_kernel(float* __restrict__ loss) { *loss = __builtin_nanf(""); }
 
+// One row of c <= 64 columns per wave, lane j holding column j: writes the
+// gradient and returns the row's loss (0 for an ignored row).
+template <typename T>
+__device__ __forceinline__ float xent_wave_row(const T* __restrict__ z, int64_t y, int64_t c, float smoothing,
+                                               float grad_scale, int nv, T* __restrict__ dz) {
+    constexpr float kLog2e = 1.4426950408889634f;
+    const int lane = threadIdx.x & 63, ci = (int)c;
+    const float v = lane < ci ? Io<T>::ld(z, lane) : -INFINITY;
+    if (!(y >= 0 && y < c)) {
+        if (lane < ci) Io<T>::st(dz, lane, 0.f);
+        return 0.f;
+    }
+    const float zy = Io<T>::ld(z, y);
+    const float mx = wave_max(v);
+    const float sz = smoothing != 0.f ? wave_sum(v == -INFINITY ? 0.f : v) : 0.f;
+    const float pe = __builtin_amdgcn_exp2f(fmaf(v, kLog2e, -mx * kLog2e));
+    const float se = wave_sum(pe);
+    const float lse = mx + __logf(se);
+    const float scale = grad_scale / (float)nv;
+    const float off = smoothing / (float)c;
+    const float hit = 1.f - smoothing;
+    if (lane < ci) {
+        float g = fmaf(pe, scale / se, -scale * off);
+        if (lane == (int)y) {
+            // not contracted, whatever a caller's loop hoists: both kernels give the same bits
+#pragma clang fp contract(off)
+            g = g - scale * hit;
+        }
+        Io<T>::st(dz, lane, g);
+    }
+    return hit * (lse - zy) + off * ((float)c * lse - sz);
+}
+
+// Rows of c <= 64 columns that are not whole 16-byte groups, when there are
+// too many for the single-workgroup kernel below: one row per wave.
+template <typename T>
+__global__ __launch_bounds__(256) void xent_wave_kernel(const T* __restrict__ logits,
+                                                        const int64_t* __restrict__ labels, int64_t n, int64_t c,
+                                                        float smoothing, float grad_scale,
+                                                        const int* __restrict__ nvalid, T* __restrict__ dlogits,
+                                                        float* __restrict__ row_loss) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= n) return;
+    const float l =
+        xent_wave_row(logits + row * c, labels[row], c, smoothing, grad_scale, *nvalid, dlogits + row * c);
+    if ((threadIdx.x & 63) == 0 && row_loss) row_loss[row] = l;
+}
+
 // Small problems (c <= 64 classes, n <= kSmallRows rows; a classifier head at
 // a small batch): the label count, every row and the mean loss in one
 // 1024-thread workgroup, where the general path takes three launches.  A wave
-// owns rows wid, wid + 16, ... with lane j holding column j; the arithmetic
-// and the summation orders are those of xent_count_kernel, the element path
-// xent_row_kernel<T, 64, 16> and xent_loss_kernel, so where the general path
-// takes the element path (c not a multiple of the 16-byte group) both give
-// the same bits; its vector path sums each thread's group first.
-constexpr int64_t kSmallRows = 4096;
+// owns rows wid, wid + 16, ...; the arithmetic and the summation orders are
+// those of xent_count_kernel, xent_wave_kernel and xent_loss_kernel, so where
+// the general path takes that kernel (c not a multiple of the 16-byte group)
+// both give the same bits; its vector path sums each thread's group first.
+// (One row per wave at a time costs 40 ns a row, 167 us at 4096 x 10 fp32
+// against 17 us on the general path; the two meet near 250 rows.)
+constexpr int64_t kSmallRows = 256;
 template <typename T>
 __global__ __launch_bounds__(1024) void xent_small_kernel(const T* __restrict__ logits,
                                                           const int64_t* __restrict__ labels, int64_t n, int64_t c,
@@ -286,33 +497,10 @@ __global__ __launch_bounds__(1024) void xent_small_kernel(const T* __restrict__ 
     if (threadIdx.x == 0) nvs = (int)total;
     __syncthreads();
     const int nv = nvs;
-    constexpr float kLog2e = 1.4426950408889634f;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int ci = (int)c;
     for (int64_t row = wid; row < n; row += 16) {
-        const T* z = logits + row * c;
-        T* dz = dlogits + row * c;
-        const int64_t y = labels[row];
-        const float v = lane < ci ? Io<T>::ld(z, lane) : -INFINITY;
-        if (!(y >= 0 && y < c)) {
-            if (lane < ci) Io<T>::st(dz, lane, 0.f);
-            if (lane == 0) rl[row] = 0.f;
-            continue;
-        }
-        const float mx = wave_max(v);
-        const float sz = smoothing != 0.f ? wave_sum(v == -INFINITY ? 0.f : v) : 0.f;
-        const float pe = __builtin_amdgcn_exp2f(fmaf(v, kLog2e, -mx * kLog2e));
-        const float se = wave_sum(pe);
-        const float lse = mx + __logf(se);
-        const float scale = grad_scale / (float)nv;
-        const float off = smoothing / (float)c;
-        const float hit = 1.f - smoothing;
-        if (lane < ci) {
-            float g = fmaf(pe, scale / se, -scale * off);
-            if (lane == (int)y) g -= scale * hit;
-            Io<T>::st(dz, lane, g);
-        }
-        if (lane == 0) rl[row] = hit * (lse - Io<T>::ld(z, y)) + off * ((float)c * lse - sz);
+        const float l = xent_wave_row(logits + row * c, labels[row], c, smoothing, grad_scale, nv, dlogits + row * c);
+        if (lane == 0) rl[row] = l;
     }
     if (!loss) return;
     __syncthreads();
@@ -322,49 +510,67 @@ __global__ __launch_bounds__(1024) void xent_small_kernel(const T* __restrict__ 
     if (threadIdx.x == 0) *loss = nv > 0 ? acc / (float)nv : __builtin_nanf("");
 }
 
-template <typename T, int NT, int EPT, bool VEC>
-void launch_rows(nott_ctx ctx, int64_t n, int64_t c, const void* logits, const int64_t* labels, float eps,
-                 float scale, const int* nvalid, void* dl, float* row_loss) {
-    if constexpr (VEC) {
-        // Persistent grid: as many workgroups as are resident at once, at
-        // most one per row.
-        static int per_cu = 0;
-        if (per_cu == 0 &&
-            (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, xent_rows_vec_kernel<T, NT, EPT>, NT, 0) !=
-                 hipSuccess ||
-             per_cu < 1))
-            per_cu = 1;
-        const int64_t grid = std::min<int64_t>(n, (int64_t)ctx->num_cu * per_cu);
-        hipLaunchKernelGGL((xent_rows_vec_kernel<T, NT, EPT>), dim3((unsigned)grid), dim3(NT), 0, ctx->stream,
-                           static_cast<const T*>(logits), labels, n, c, eps, scale, nvalid, static_cast<T*>(dl),
-                           row_loss);
-    } else {
-        hipLaunchKernelGGL((xent_row_kernel<T, NT, EPT>), dim3((unsigned)n), dim3(NT), 0, ctx->stream,
-                           static_cast<const T*>(logits), labels, c, eps, scale, nvalid, static_cast<T*>(dl), row_loss);
-    }
+// As many workgroups as are resident at once, at most one per row.
+template <class K>
+unsigned resident_grid(nott_ctx ctx, K kernel, int threads, int64_t n, int& per_cu) {
+    if (per_cu == 0 &&
+        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || per_cu < 1))
+        per_cu = 1;
+    return (unsigned)std::min<int64_t>(n, (int64_t)ctx->num_cu * per_cu);
 }
 
 template <typename T>
-void dispatch(nott_ctx ctx, int64_t n, int64_t c, const void* logits, const int64_t* labels, float eps, float scale,
-              const int* nvalid, void* dl, float* row_loss) {
-    const bool vec = (c % Pack16<T>::N == 0) && ((uintptr_t)logits % 16 == 0) && ((uintptr_t)dl % 16 == 0);
-    if (vec && c <= 64 * 16)
-        launch_rows<T, 64, 16, true>(ctx, n, c, logits, labels, eps, scale, nvalid, dl, row_loss);
-    else if (vec && c <= 256 * 32)
-        launch_rows<T, 256, 32, true>(ctx, n, c, logits, labels, eps, scale, nvalid, dl, row_loss);
-    else if (vec && sizeof(T) == 2 && c <= 512 * 64)
-        // bf16 rows of up to 32768: two 512-thread workgroups per CU, so that
-        // two rows (plus the two prefetched ones) are in flight per CU.
-        launch_rows<T, 512, 64, true>(ctx, n, c, logits, labels, eps, scale, nvalid, dl, row_loss);
-    else if (vec && c <= 1024 * 32)
-        launch_rows<T, 1024, 32, true>(ctx, n, c, logits, labels, eps, scale, nvalid, dl, row_loss);
-    else if (c <= 64 * 16)
-        launch_rows<T, 64, 16, false>(ctx, n, c, logits, labels, eps, scale, nvalid, dl, row_loss);
-    else if (c <= 512 * 32)
-        launch_rows<T, 512, 32, false>(ctx, n, c, logits, labels, eps, scale, nvalid, dl, row_loss);
-    else
-        hipLaunchKernelGGL(xent_long_kernel<T>, dim3((unsigned)n), dim3(256), 0, ctx->stream,
-                           static_cast<const T*>(logits), labels, c, eps, scale, nvalid, static_cast<T*>(dl), row_loss);
+struct RowArgs {
+    int64_t n, c;
+    const T* logits;
+    const int64_t* labels;
+    float eps, scale;
+    const int* nvalid;
+    T* dl;
+    float* row_loss;
+};
+
+template <typename T, int NT, int EPT>
+void launch_vec(nott_ctx ctx, const RowArgs<T>& a) {
+    static int per_cu = 0;
+    const unsigned grid = resident_grid(ctx, xent_rows_vec_kernel<T, NT, EPT>, NT, a.n, per_cu);
+    hipLaunchKernelGGL((xent_rows_vec_kernel<T, NT, EPT>), dim3(grid), dim3(NT), 0, ctx->stream, a.logits, a.labels,
+                       a.n, a.c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
+}
+
+template <typename T, int NT, int EPT, bool REST>
+void launch_any(nott_ctx ctx, const RowArgs<T>& a, int inf_counts) {
+    hipLaunchKernelGGL((xent_any_kernel<T, NT, EPT, REST>), dim3((unsigned)a.n), dim3(NT), 0, ctx->stream, a.logits,
+                       a.labels, a.c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss, inf_counts);
+}
+
+template <typename T>
+void dispatch(nott_ctx ctx, const RowArgs<T>& a) {
+    constexpr int G = Pack16<T>::N;
+    // Whole aligned groups of up to 32768 columns: the persistent kernel, whose
+    // next row is in flight during the reductions (5.7 TB/s at 16384 x 32000
+    // fp32).  Everything else: the kernel for any row, in the smallest shape
+    // that holds it (the single-column rows of up to 64 one wave each).
+    const int64_t c = a.c;
+    const bool vec = (c % G == 0) && ((uintptr_t)a.logits % 16 == 0) && ((uintptr_t)a.dl % 16 == 0);
+    if (vec && c <= 64 * 16) return launch_vec<T, 64, 16>(ctx, a);
+    if (vec && c <= 256 * 32) return launch_vec<T, 256, 32>(ctx, a);
+    // bf16 rows of up to 32768: two 512-thread workgroups per CU, so that
+    // two rows (plus the two prefetched ones) are in flight per CU.
+    if (vec && sizeof(T) == 2 && c <= 512 * 64) return launch_vec<T, 512, 64>(ctx, a);
+    if (vec && c <= 1024 * 32) return launch_vec<T, 1024, 32>(ctx, a);
+    if (c <= 64) {
+        hipLaunchKernelGGL(xent_wave_kernel<T>, dim3((unsigned)nott::ceil_div(a.n, 4)), dim3(256), 0, ctx->stream,
+                           a.logits, a.labels, a.n, c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
+        return;
+    }
+    if (c <= 64 * 16) return launch_any<T, 64, 16, false>(ctx, a, 0);
+    if (c <= 256 * 32) return launch_any<T, 256, 32, false>(ctx, a, 0);
+    if (c <= 512 * 32) return launch_any<T, 512, 32, false>(ctx, a, 0);
+    if (c <= 512 * 64) return launch_any<T, 512, 64, false>(ctx, a, 1);
+    if (c <= 512 * 104) return launch_any<T, 512, 104, false>(ctx, a, 1);
+    if (c <= 1024 * 104) return launch_any<T, 1024, 104, false>(ctx, a, 1);
+    return launch_any<T, 1024, 104, true>(ctx, a, 1);
 }
 
 }  // namespace
@@ -402,9 +608,11 @@ extern "C" int nott_softmax_xent_bwd(nott_ctx ctx, nott_dtype dtype, int64_t n, 
     float* row_loss = loss ? reinterpret_cast<float*>(ws + 256) : nullptr;
     hipLaunchKernelGGL(xent_count_kernel, dim3(1), dim3(1024), 0, ctx->stream, labels, n, c, nvalid, ctx->err_word);
     if (dtype == NOTT_F32)
-        dispatch<float>(ctx, n, c, logits, labels, eps, scale, nvalid, dlogits, row_loss);
+        dispatch<float>(ctx, {n, c, static_cast<const float*>(logits), labels, eps, scale, nvalid,
+                              static_cast<float*>(dlogits), row_loss});
     else
-        dispatch<bf16_t>(ctx, n, c, logits, labels, eps, scale, nvalid, dlogits, row_loss);
+        dispatch<bf16_t>(ctx, {n, c, static_cast<const bf16_t*>(logits), labels, eps, scale, nvalid,
+                               static_cast<bf16_t*>(dlogits), row_loss});
     if (loss) hipLaunchKernelGGL(xent_loss_kernel, dim3(1), dim3(1024), 0, ctx->stream, row_loss, n, nvalid, loss);
     return nott::launch_status(ctx, "softmax_xent");
 }
