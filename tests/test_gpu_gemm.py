@@ -64,6 +64,11 @@ def test_linear(ops, oracle, dt, m, kin, nout):
 # dW unsplit over three tile columns (the bias gradient is summed once);
 # (4100, 2048, 4104) forward on unsplit 256x256 tiles (17 x 17, K = 2048).
 DMA_LIN = [(4104, 192, 2056), (2048, 1288, 1544), (1024, 200, 320), (256, 384, 256), (4100, 2048, 4104)]
+# k extents that end inside a 64-deep stage (their last stage is zero-filled):
+# odd token counts in dW, whole 8s in the forward and dX; a single partial
+# stage, one step past a stage, 8 short of one; 256x128 (8200 rows), 128x128
+# with two workgroups per CU (1576 -> 3072) and split dW (4001 tokens).
+DMA_LIN += [(129, 136, 128), (1576, 768, 3072), (8200, 328, 264), (4001, 152, 200), (257, 2040, 136)]
 
 
 def _edge(idx, n):

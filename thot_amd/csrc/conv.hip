@@ -532,7 +532,7 @@ int col_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, con
                        (int32_t)d->k, (int32_t)CRS, (int32_t)CRSp, wp);
     hipLaunchKernelGGL(to_kn_kernel<bf16_t>, dim3((unsigned)ceil_div(d->k * (NPQ / 8), 256)), dim3(256), 0, ctx->stream,
                        dy, g, (int32_t)NPQ, (int)((p * q) % 8 == 0 && ((uintptr_t)dy % 16) == 0), dyt);
-    RowMajorStore<bf16_t> ep{dcol, NPQ, CRSp, NPQ, nullptr, 0};
+    RowMajorStore<bf16_t> ep{dcol, NPQ, CRSp, NPQ, nullptr};
     const int st = fast::run<true, true>(ctx, wp, CRSp, dyt, NPQ, ep, CRSp, NPQ, d->k, 0,
                                          reinterpret_cast<float*>(ws + o_part));
     if (st != NOTT_OK) return st;

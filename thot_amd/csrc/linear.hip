@@ -9,10 +9,10 @@
 //   dw = dyᵀ·x            (TN: both k-strided; split-K over rows)
 //   db = Σ_rows dy        (folded into the dw GEMM as an extra all-ones column;
 //                          bf16 fast path: a two-phase column sum)
-// bf16 operands whose k extent is a multiple of 64 take the direct-to-LDS
-// GEMM (gemm_dma.hpp) when both output extents are at least 128, else the
-// register-staged fast GEMM (gemm.hpp, namespace fast); everything else the
-// generic engine, on 64×64 tiles with split-K (run_small) where its 128×128
+// bf16 operands in whole 16-byte groups take the direct-to-LDS GEMM
+// (gemm_dma.hpp; any k extent) when both output extents are at least 128, else
+// with a k extent that is a multiple of 64 the register-staged fast GEMM
+// (gemm.hpp, namespace fast); everything else the generic engine, on 64×64 tiles with split-K (run_small) where its 128×128
 // grid would leave CUs idle (small batches, narrow outputs).  Every product runs on the kernels in this library; no
 // vendor GEMM is called.
 #include "gemm_dma.hpp"
@@ -198,7 +198,7 @@ template <typename T>
 int fwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* x, const void* w, const float* b, void* y,
         int relu) {
     if constexpr (sizeof(T) == 2) {
-        RowMajorStore<T> ep{static_cast<T*>(y), nout, m, nout, b, 0, relu};
+        RowMajorStore<T> ep{static_cast<T*>(y), nout, m, nout, b, relu};
         const int st = bf16_gemm<false, false>(ctx, static_cast<const T*>(x), kin, static_cast<const T*>(w), kin, ep,
                                                m, nout, kin);
         if (st != NOTT_ERR_UNSUPPORTED) return st;
@@ -207,7 +207,7 @@ int fwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* x, const
     const T* wp = static_cast<const T*>(w);
     RowKLoader<T> la{xp, kin, m, kin, vec16<T>(x, kin)};
     RowKLoader<T> lb{wp, kin, nout, kin, vec16<T>(w, kin)};
-    RowMajorStore<T> ep{static_cast<T*>(y), nout, m, nout, b, 0, relu};
+    RowMajorStore<T> ep{static_cast<T*>(y), nout, m, nout, b, relu};
     if (small_grid(ctx, m, nout)) return run_small<T>(ctx, la, lb, ep, m, nout, kin);
     return run<T>(ctx, la, lb, ep, m, nout, kin);
 }
@@ -228,39 +228,34 @@ int bwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* dy, cons
     if constexpr (sizeof(T) == 2) {
         // dx = dy·w: A = dy (k = o contiguous), B(i, o) = w[o·kin + i] (transposed)
         // dw = dyᵀ·x: A(o, r) = dy[r·nout + o], B(i, r) = x[r·kin + i] (both transposed)
-        const bool fx = !dx || (nout % fast::BK == 0 && kin % 8 == 0);
-        const bool fw = !dw || (m % fast::BK == 0 && nout % 8 == 0 && kin % 8 == 0);
-        if (fx && fw) {
-            if (dx) {
-                RowMajorStore<T> ep{static_cast<T*>(dx), kin, m, kin, nullptr, 0, 0, dx_mask};
-                const int st = bf16_gemm<false, true>(ctx, dyp, nout, static_cast<const T*>(w), kin, ep, m, kin, nout);
-                if (st != NOTT_ERR_UNSUPPORTED) {
-                    if (st != NOTT_OK) return st;
-                    dx = nullptr;
-                }
+        if (dx) {
+            RowMajorStore<T> ep{static_cast<T*>(dx), kin, m, kin, nullptr, 0, dx_mask};
+            const int st = bf16_gemm<false, true>(ctx, dyp, nout, static_cast<const T*>(w), kin, ep, m, kin, nout);
+            if (st != NOTT_ERR_UNSUPPORTED) {
+                if (st != NOTT_OK) return st;
+                dx = nullptr;
             }
-            if (dw && db) {
-                // db = Σ_rows dy summed from the dw GEMM's dy fragments.
-                DwRowsumStore ep{dw, db, nout, kin, accumulate};
-                const int st = dma::run<true, true, true>(ctx, dyp, nout, static_cast<const T*>(x), kin, ep, nout, kin,
-                                                          m);
-                if (st != NOTT_ERR_UNSUPPORTED) {
-                    if (st != NOTT_OK) return st;
-                    dw = nullptr;
+        }
+        if (dw && db) {
+            // db = Σ_rows dy summed from the dw GEMM's dy fragments.
+            DwRowsumStore ep{dw, db, nout, kin, accumulate};
+            const int st = dma::run<true, true, true>(ctx, dyp, nout, static_cast<const T*>(x), kin, ep, nout, kin, m);
+            if (st != NOTT_ERR_UNSUPPORTED) {
+                if (st != NOTT_OK) return st;
+                dw = nullptr;
+                db = nullptr;
+            }
+        }
+        if (dw) {
+            DwDbStore ep{dw, nullptr, nout, kin, accumulate};
+            const int st = bf16_gemm<true, true>(ctx, dyp, nout, static_cast<const T*>(x), kin, ep, nout, kin, m);
+            if (st != NOTT_ERR_UNSUPPORTED) {
+                if (st != NOTT_OK) return st;
+                dw = nullptr;
+                if (db) {
+                    const int st2 = launch_db<T>(ctx, dyp, m, nout, db, accumulate);
+                    if (st2 != NOTT_OK) return st2;
                     db = nullptr;
-                }
-            }
-            if (dw) {
-                DwDbStore ep{dw, nullptr, nout, kin, accumulate};
-                const int st = bf16_gemm<true, true>(ctx, dyp, nout, static_cast<const T*>(x), kin, ep, nout, kin, m);
-                if (st != NOTT_ERR_UNSUPPORTED) {
-                    if (st != NOTT_OK) return st;
-                    dw = nullptr;
-                    if (db) {
-                        const int st2 = launch_db<T>(ctx, dyp, m, nout, db, accumulate);
-                        if (st2 != NOTT_OK) return st2;
-                        db = nullptr;
-                    }
                 }
             }
         }
@@ -268,7 +263,7 @@ int bwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* dy, cons
     if (dx) {
         RowKLoader<T> la{dyp, nout, m, nout, vec16<T>(dy, nout)};
         ColKLoader<T> lb{static_cast<const T*>(w), kin, kin, nout};
-        RowMajorStore<T> ep{static_cast<T*>(dx), kin, m, kin, nullptr, 0, 0, dx_mask};
+        RowMajorStore<T> ep{static_cast<T*>(dx), kin, m, kin, nullptr, 0, dx_mask};
         const int st = small_grid(ctx, m, kin) ? run_small<T>(ctx, la, lb, ep, m, kin, nout)
                                                : run<T>(ctx, la, lb, ep, m, kin, nout);
         if (st != NOTT_OK) return st;
