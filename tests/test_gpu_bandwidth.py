@@ -412,8 +412,15 @@ def test_batchnorm_act(ops, oracle, dt, shape, with_res):
 
 # -------------------------------------------------------------- layernorm
 @pytest.mark.parametrize("dt", DTYPES)
+# beside the first line: rows that are not whole 16-byte groups (single-element
+# accesses) and rows shared by 2, 4, 8 and 16 waves at the edges of what they
+# hold (16 values a lane), with row counts that leave a block's last rows
+# without work; 16385 columns take the kernels of any length
 @pytest.mark.parametrize("rows,d", [(2048, 1024), (37, 256), (5, 1000), (3, 3000), (64, 4), (4099, 512), (257, 2048),
-                                    (1029, 64)])
+                                    (1029, 64),
+                                    (1001, 1), (515, 67), (2051, 333), (1100, 771), (1030, 1023), (1027, 1025),
+                                    (1029, 2050), (2049, 2056), (515, 4095), (515, 4104), (259, 8191), (259, 8200),
+                                    (259, 16384), (3, 16383), (2, 16385)])
 def test_layernorm(ops, oracle, dt, rows, d):
     g = rng(rows + d)
     x = host_input(g.standard_normal((rows, d)), dt)

@@ -7,10 +7,12 @@
 //   forward : x̂ = (x − μ)·rstd, rstd = 1/sqrt(var_biased + eps), y = x̂·γ + β
 //   backward: g = dy·γ; dx = rstd·(g − Σg/d − x̂·Σ(g·x̂)/d)
 //             dγ = Σ_rows dy·x̂, dβ = Σ_rows dy
-// One wavefront owns one row: the row's x and dy stay in VGPRs, the two row
-// sums are DPP/shuffle wave reductions, and every lane keeps running dγ / dβ
-// sums for its columns.  Blocks write per-block column partials; a second
-// kernel reduces them (deterministic order).
+// A row of up to 16384 columns belongs to WPR wavefronts (one up to 1024
+// columns, more for wider ones, so that a lane holds at most 16 values): its x
+// and dy stay in VGPRs, the row sums are DPP wave reductions (and one LDS
+// exchange where several waves share a row), and every lane keeps running
+// dγ / dβ sums for its columns over the rows it takes.  Blocks write per-block
+// column partials; a second kernel reduces them (deterministic order).
 #include "common.hpp"
 
 #include <mutex>
@@ -25,205 +27,248 @@ constexpr int kReduceThreads = 1024;   // column reduction: 16 waves split the p
 constexpr int kReduceWaves = kReduceThreads / 64;
 constexpr int kReduceUnroll = 32;  // 16 waves x 32 loads cover 512 partial rows in one round
 
-// Element e of a lane's DPL row values is column col(g, e) with g = e / G:
-// group g of lane `lane` covers the 16 bytes at columns [(g*64 + lane)*G, +G),
-// G = 4 (fp32) or 8 (bf16), so every wave access is a 1 KB coalesced run.
-template <typename T>
-__device__ __forceinline__ int64_t row_col(int lane, int e) {
-    constexpr int G = Pack16<T>::N;
-    return ((int64_t)(e / G) * 64 + lane) * G + e % G;
+// How a row's columns are dealt to the P = 64·WPR lanes that own it: group g of
+// lane t covers columns [(g·P + t)·G, +G).  G is the 16-byte group (4 fp32 / 8
+// bf16 elements: a wave access is a 1 KB coalesced run) where every row is
+// aligned and whole groups, else 1 (any d, any alignment).
+template <typename T, int G> struct Group {
+    typedef typename Pack16<T>::Raw Raw;
+    static_assert(G == Pack16<T>::N, "a 16-byte group");
+    template <bool NT> static __device__ __forceinline__ Raw raw(const T* p) { return Pack16<T>::template raw<NT>(p); }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&v)[G]) { Pack16<T>::unpack(r, v); }
+    static __device__ __forceinline__ void st(T* p, const float (&v)[G]) { Pack16<T>::template st<false>(p, v); }
+};
+template <typename T> struct Group<T, 1> {
+    typedef T Raw;
+    template <bool NT> static __device__ __forceinline__ Raw raw(const T* p) { return *p; }
+    static __device__ __forceinline__ void unpack(const Raw& r, float (&v)[1]) { v[0] = Io<T>::ld(&r, 0); }
+    static __device__ __forceinline__ void st(T* p, const float (&v)[1]) { Io<T>::st(p, 0, v[0]); }
+};
+
+template <int DPL, int G, int P>
+struct Row {
+    static constexpr int NG = DPL / G;
+    static __device__ __forceinline__ int64_t col(int t, int e) { return ((int64_t)(e / G) * P + t) * G + e % G; }
+    // Every lane issues all of its loads unconditionally (columns past d read
+    // column 0 and are zeroed by unpack), so a row's loads stay in flight
+    // together.
+    template <typename T, bool NT>
+    static __device__ __forceinline__ void load(const T* __restrict__ p, int64_t d, int t,
+                                                typename Group<T, G>::Raw (&raw)[NG]) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int64_t c0 = ((int64_t)g * P + t) * G;
+            raw[g] = Group<T, G>::template raw<NT>(p + (c0 < d ? c0 : 0));
+        }
+    }
+    template <typename T>
+    static __device__ __forceinline__ void unpack(const typename Group<T, G>::Raw (&raw)[NG], int64_t d, int t,
+                                                  float (&v)[DPL]) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int64_t c0 = ((int64_t)g * P + t) * G;
+            float x[G];
+            Group<T, G>::unpack(raw[g], x);
+#pragma unroll
+            for (int e = 0; e < G; ++e) v[G * g + e] = c0 < d ? x[e] : 0.f;
+        }
+    }
+    template <typename T, bool NT>
+    static __device__ __forceinline__ void load_all(const T* __restrict__ p, int64_t d, int t, float (&v)[DPL]) {
+        typename Group<T, G>::Raw raw[NG];
+        load<T, NT>(p, d, t, raw);
+        unpack<T>(raw, d, t, v);
+    }
+    template <typename T>
+    static __device__ __forceinline__ void store(T* __restrict__ p, int64_t d, int t, const float (&v)[DPL]) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int64_t c0 = ((int64_t)g * P + t) * G;
+            float x[G];
+#pragma unroll
+            for (int e = 0; e < G; ++e) x[e] = v[G * g + e];
+            if (c0 < d) Group<T, G>::st(p + c0, x);
+        }
+    }
+};
+
+// Sum over the WPR waves of a row of K values each lane holds.  `red` is this
+// use's own LDS, K·WPR floats per row of the block; every thread of the block
+// calls it.  Two uses that alternate between two buffers need no other barrier.
+template <int WPR, int K>
+__device__ __forceinline__ void row_sum(float (&v)[K], float* red) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
+    if constexpr (WPR > 1) {
+        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        float* mine = red + (wid / WPR) * (K * WPR);
+        if (lane == 0) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) mine[k * WPR + wid % WPR] = v[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            float s = 0.f;
+#pragma unroll
+            for (int w = 0; w < WPR; ++w) s += mine[k * WPR + w];
+            v[k] = s;
+        }
+    }
 }
 
-// Every lane issues all of its loads unconditionally (columns past d read
-// column 0 and are zeroed afterwards), so a row's loads stay in flight
-// together.
-template <typename T, int DPL, bool NT>
-__device__ __forceinline__ void load_row(const T* __restrict__ p, int64_t d, int lane, float (&v)[DPL]) {
-    constexpr int G = Pack16<T>::N;
-    typename Pack16<T>::Raw raw[DPL / G > 0 ? DPL / G : 1];
-#pragma unroll
-    for (int g = 0; g < DPL / G; ++g) {
-        const int64_t c0 = ((int64_t)g * 64 + lane) * G;
-        raw[g] = Pack16<T>::template raw<NT>(p + (c0 < d ? c0 : 0));
-    }
-#pragma unroll
-    for (int g = 0; g < DPL / G; ++g) {
-        const int64_t c0 = ((int64_t)g * 64 + lane) * G;
-        float t[G];
-        Pack16<T>::unpack(raw[g], t);
-#pragma unroll
-        for (int e = 0; e < G; ++e) v[G * g + e] = c0 < d ? t[e] : 0.f;
-    }
-}
-
-// load_row split in two: the raw 16-byte loads, and their conversion to
-// floats (columns past d read column 0 and become zero).
-template <typename T>
-__host__ __device__ constexpr int raw_groups(int dpl) { return dpl / Pack16<T>::N > 0 ? dpl / Pack16<T>::N : 1; }
-template <typename T, int DPL, bool NT>
-__device__ __forceinline__ void load_raw(const T* __restrict__ p, int64_t d, int lane,
-                                         typename Pack16<T>::Raw (&raw)[raw_groups<T>(DPL)]) {
-    constexpr int G = Pack16<T>::N;
-#pragma unroll
-    for (int g = 0; g < DPL / G; ++g) {
-        const int64_t c0 = ((int64_t)g * 64 + lane) * G;
-        raw[g] = Pack16<T>::template raw<NT>(p + (c0 < d ? c0 : 0));
-    }
-}
-template <typename T, int DPL>
-__device__ __forceinline__ void unpack_row(const typename Pack16<T>::Raw (&raw)[raw_groups<T>(DPL)], int64_t d,
-                                           int lane, float (&v)[DPL]) {
-    constexpr int G = Pack16<T>::N;
-#pragma unroll
-    for (int g = 0; g < DPL / G; ++g) {
-        const int64_t c0 = ((int64_t)g * 64 + lane) * G;
-        float t[G];
-        Pack16<T>::unpack(raw[g], t);
-#pragma unroll
-        for (int e = 0; e < G; ++e) v[G * g + e] = c0 < d ? t[e] : 0.f;
-    }
-}
-
-template <typename T, int DPL, bool NT>
-__device__ __forceinline__ void store_row(T* __restrict__ p, int64_t d, int lane, const float (&v)[DPL]) {
-    constexpr int G = Pack16<T>::N;
-#pragma unroll
-    for (int g = 0; g < DPL / G; ++g) {
-        const int64_t c0 = ((int64_t)g * 64 + lane) * G;
-        float t[G];
-#pragma unroll
-        for (int e = 0; e < G; ++e) t[e] = v[G * g + e];
-        if (c0 < d) Pack16<T>::template st<NT>(p + c0, t);
-    }
-}
-
-template <typename T, int DPL>
-__global__ __launch_bounds__(kThreads) void ln_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
-                                                          const T* __restrict__ beta, float eps, T* __restrict__ y,
-                                                          float* __restrict__ mean, float* __restrict__ rstd,
-                                                          int64_t rows, int64_t d) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+// GROUPS rows per block at a time, WPR waves each.  Bound by memory: a call of
+// 8192x8192 bf16 46 us (5.9 TB/s), 4096x4096 14.4 us, where three passes of
+// single elements per row took 109 and 28.
+template <typename T, int DPL, int G, int WPR, int GROUPS>
+__global__ __launch_bounds__(64 * WPR * GROUPS) void ln_fwd_kernel(const T* __restrict__ x,
+                                                                   const T* __restrict__ gamma,
+                                                                   const T* __restrict__ beta, float eps,
+                                                                   T* __restrict__ y, float* __restrict__ mean,
+                                                                   float* __restrict__ rstd, int64_t rows, int64_t d) {
+    constexpr int P = 64 * WPR;
+    typedef Row<DPL, G, P> R;
+    __shared__ float red[2][GROUPS * WPR];
+    const int t = threadIdx.x % P, grp = threadIdx.x / P;
     float gm[DPL], bt[DPL];
-    load_row<T, DPL, false>(gamma, d, lane, gm);
-    load_row<T, DPL, false>(beta, d, lane, bt);
+    R::template load_all<T, false>(gamma, d, t, gm);
+    R::template load_all<T, false>(beta, d, t, bt);
     const float inv_d = 1.f / (float)d;
-    for (int64_t r = (int64_t)blockIdx.x * kWaves + wid; r < rows; r += (int64_t)gridDim.x * kWaves) {
+    const int64_t stride = (int64_t)gridDim.x * GROUPS;
+    for (int64_t r0 = (int64_t)blockIdx.x * GROUPS; r0 < rows; r0 += stride) {
+        const int64_t r = r0 + grp;
+        if (WPR == 1 && r >= rows) break;
+        const bool in = WPR == 1 || r < rows;
         float v[DPL];
-        load_row<T, DPL, true>(x + r * d, d, lane, v);
-        float s = 0.f;
+        R::template load_all<T, true>(x + (in ? r : rows - 1) * d, d, t, v);
+        float s[1] = {0.f};
 #pragma unroll
-        for (int e = 0; e < DPL; ++e) s += v[e];
-        const float mu = wave_sum(s) * inv_d;
-        float ss = 0.f;
+        for (int e = 0; e < DPL; ++e) s[0] += v[e];
+        row_sum<WPR, 1>(s, red[0]);
+        const float mu = s[0] * inv_d;
+        s[0] = 0.f;
 #pragma unroll
         for (int e = 0; e < DPL; ++e) {
-            const float t = row_col<T>(lane, e) < d ? v[e] - mu : 0.f;
-            ss += t * t;
+            const float u = R::col(t, e) < d ? v[e] - mu : 0.f;
+            s[0] += u * u;
         }
-        const float rs = 1.f / sqrtf(wave_sum(ss) * inv_d + eps);
+        row_sum<WPR, 1>(s, red[1]);
+        const float rs = 1.f / sqrtf(s[0] * inv_d + eps);
 #pragma unroll
         for (int e = 0; e < DPL; ++e) v[e] = (v[e] - mu) * rs * gm[e] + bt[e];
-        store_row<T, DPL, false>(y + r * d, d, lane, v);
-        if (lane == 0) {
+        if (!in) continue;
+        R::template store<T>(y + r * d, d, t, v);
+        if (t == 0) {
             mean[r] = mu;
             rstd[r] = rs;
         }
     }
 }
 
-// WAVES waves per block, one block per CU (measured best for configs[2]a:
-// 8 waves of one row each, ordinary loads and stores, with the next row's
-// loads in flight while the current row is reduced).
-template <typename T, int DPL, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void ln_bwd_kernel(const T* __restrict__ x, const T* __restrict__ dy,
-                                                            const float* __restrict__ mean,
-                                                            const float* __restrict__ rstd,
-                                                            const T* __restrict__ gamma, T* __restrict__ dx,
-                                                            float* __restrict__ partial, int64_t rows, int64_t d) {
-    extern __shared__ float lds[];  // [WAVES][2][d]
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+// One block per CU, GROUPS rows at a time of WPR waves each, 8 waves in all (16
+// past 8192 columns): ordinary loads and stores, with the next row's loads in
+// flight while the current row is reduced (measured best at 16384x1024, where
+// it streams 5.8 TB/s fp32; wider rows keep the same bytes in flight per CU:
+// 4096x4096 bf16 24 us a call, 8192x8192 86 us).  A block per row whose dγ / dβ
+// partials were written for every row took 71 and 344 us, and 59 us for 5000x771
+// fp32 (19 now).
+template <typename T, int DPL, int G, int WPR, int GROUPS>
+__global__ __launch_bounds__(64 * WPR * GROUPS) void ln_bwd_kernel(const T* __restrict__ x, const T* __restrict__ dy,
+                                                                   const float* __restrict__ mean,
+                                                                   const float* __restrict__ rstd,
+                                                                   const T* __restrict__ gamma, T* __restrict__ dx,
+                                                                   float* __restrict__ partial, int64_t rows,
+                                                                   int64_t d) {
+    constexpr int P = 64 * WPR, NT = P * GROUPS;
+    typedef Row<DPL, G, P> R;
+    extern __shared__ float lds[];  // [GROUPS][2][d] (one group: unused)
+    __shared__ float red[2][GROUPS * WPR * 2];
+    const int t = threadIdx.x % P, grp = threadIdx.x / P;
     float gm[DPL];
-    load_row<T, DPL, false>(gamma, d, lane, gm);
+    R::template load_all<T, false>(gamma, d, t, gm);
     float dg[DPL], db[DPL];
 #pragma unroll
     for (int e = 0; e < DPL; ++e) dg[e] = db[e] = 0.f;
     const float inv_d = 1.f / (float)d;
-    constexpr int kRowsInFlight = 1;
-    constexpr int NG = raw_groups<T>(DPL);
-    const int64_t stride = (int64_t)gridDim.x * WAVES * kRowsInFlight;
-    // The next group of rows is loaded (raw) while the current one is
-    // reduced and stored: two groups' loads per wave stay in flight.
-    typename Pack16<T>::Raw rx[kRowsInFlight][NG], rd[kRowsInFlight][NG];
-    float nmu[kRowsInFlight], nrs[kRowsInFlight];
-    auto fetch = [&](int64_t r0) {
-#pragma unroll
-        for (int i = 0; i < kRowsInFlight; ++i) {
-            // Rows past the end re-read the last row (unconditional loads keep
-            // every row's loads in flight together); they are not stored.
-            const int64_t r = r0 + i < rows ? r0 + i : rows - 1;
-            load_raw<T, DPL, false>(x + r * d, d, lane, rx[i]);
-            load_raw<T, DPL, false>(dy + r * d, d, lane, rd[i]);
-            nmu[i] = mean[r];
-            nrs[i] = rstd[r];
-        }
+    const int64_t stride = (int64_t)gridDim.x * GROUPS;
+    // The next row is loaded (raw) while the current one is reduced and
+    // stored: two rows' loads per group stay in flight.
+    typename Group<T, G>::Raw rx[R::NG], rd[R::NG];
+    float nmu = 0.f, nrs = 0.f;
+    auto fetch = [&](int64_t r) {
+        r = r < rows ? r : rows - 1;   // (a group past the end re-reads the last row)
+        R::template load<T, false>(x + r * d, d, t, rx);
+        R::template load<T, false>(dy + r * d, d, t, rd);
+        nmu = mean[r];
+        nrs = rstd[r];
     };
-    const int64_t first = ((int64_t)blockIdx.x * WAVES + wid) * kRowsInFlight;
-    if (first < rows) fetch(first);
+    int buf = 0;
+    const int64_t first = (int64_t)blockIdx.x * GROUPS;
+    if (first < rows) fetch(first + grp);
     for (int64_t r0 = first; r0 < rows; r0 += stride) {
-        float xv[kRowsInFlight][DPL], gv[kRowsInFlight][DPL];
-        float mu[kRowsInFlight], rs[kRowsInFlight];
+        const int64_t r = r0 + grp;
+        if (WPR == 1 && r >= rows) break;
+        const bool in = WPR == 1 || r < rows;
+        float xv[DPL], gv[DPL];
+        R::template unpack<T>(rx, d, t, xv);
+        R::template unpack<T>(rd, d, t, gv);
+        const float mu = nmu, rs = nrs;
+        if (r0 + stride < rows) fetch(r + stride);
+        float s[2] = {0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < kRowsInFlight; ++i) {
-            unpack_row<T, DPL>(rx[i], d, lane, xv[i]);
-            unpack_row<T, DPL>(rd[i], d, lane, gv[i]);
-            mu[i] = nmu[i];
-            rs[i] = nrs[i];
-        }
-        if (r0 + stride < rows) fetch(r0 + stride);
-#pragma unroll
-        for (int i = 0; i < kRowsInFlight; ++i) {
-            const int64_t r = r0 + i;
-            if (r >= rows) break;
-            float sg = 0.f, sgx = 0.f;
-#pragma unroll
-            for (int e = 0; e < DPL; ++e) {
-                const float xh = (xv[i][e] - mu[i]) * rs[i];
-                const float dyv = gv[i][e];
+        for (int e = 0; e < DPL; ++e) {
+            const float xh = (xv[e] - mu) * rs;
+            const float dyv = gv[e];
+            if (in) {
                 dg[e] += dyv * xh;
                 db[e] += dyv;
-                const float g = dyv * gm[e];
-                sg += g;
-                sgx += g * xh;
-                xv[i][e] = xh;
-                gv[i][e] = g;
             }
-            sg = wave_sum(sg) * inv_d;
-            sgx = wave_sum(sgx) * inv_d;
-#pragma unroll
-            for (int e = 0; e < DPL; ++e) xv[i][e] = rs[i] * (gv[i][e] - sg - xv[i][e] * sgx);
-            store_row<T, DPL, false>(dx + r * d, d, lane, xv[i]);
+            const float g = dyv * gm[e];
+            s[0] += g;
+            s[1] += g * xh;
+            xv[e] = xh;
+            gv[e] = g;
         }
-    }
-    // Combine the waves' column sums and write this block's partial row.
+        row_sum<WPR, 2>(s, red[buf]);
+        buf ^= 1;
+        const float sg = s[0] * inv_d, sgx = s[1] * inv_d;
 #pragma unroll
-    for (int e = 0; e < DPL; ++e) {
-        const int64_t col = row_col<T>(lane, e);
-        if (col < d) {
-            lds[(wid * 2 + 0) * d + col] = dg[e];
-            lds[(wid * 2 + 1) * d + col] = db[e];
-        }
+        for (int e = 0; e < DPL; ++e) xv[e] = rs * (gv[e] - sg - xv[e] * sgx);
+        if (in) R::template store<T>(dx + r * d, d, t, xv);
     }
-    __syncthreads();
-    // Partial layout [which][16-column group][block][16]: the reduction reads
-    // each group's partials as one contiguous run.
+    // This block's partial row: layout [which][16-column group][block][16], so
+    // that the reduction reads each group's partials as one contiguous run.
     const int64_t ngroups = (d + 15) / 16;
-    for (int64_t j = threadIdx.x; j < 2 * d; j += 64 * WAVES) {
-        const int which = j >= d;
-        const int64_t col = j - which * d;
-        float s = 0.f;
+    auto put = [&](int which, int64_t col, float v) {
+        partial[((which * ngroups + col / 16) * gridDim.x + blockIdx.x) * 16 + col % 16] = v;
+    };
+    if constexpr (GROUPS == 1) {
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) s += lds[(w * 2 + which) * d + col];
-        partial[((which * ngroups + col / 16) * gridDim.x + blockIdx.x) * 16 + col % 16] = s;
+        for (int e = 0; e < DPL; ++e) {
+            const int64_t col = R::col(t, e);
+            if (col < d) {
+                put(0, col, dg[e]);
+                put(1, col, db[e]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < DPL; ++e) {
+            const int64_t col = R::col(t, e);
+            if (col < d) {
+                lds[(grp * 2 + 0) * d + col] = dg[e];
+                lds[(grp * 2 + 1) * d + col] = db[e];
+            }
+        }
+        __syncthreads();
+        for (int64_t j = threadIdx.x; j < 2 * d; j += NT) {
+            const int which = j >= d;
+            const int64_t col = j - which * d;
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < GROUPS; ++w) v += lds[(w * 2 + which) * d + col];
+            put(which, col, v);
+        }
     }
 }
 
@@ -317,7 +362,7 @@ __global__ __launch_bounds__(kReduceThreads) void col_reduce_kernel(const float*
     }
 }
 
-// Generic row kernels (any d): one block per row, three passes over the row.
+// Rows past 16384 columns: one block per row, three passes over the row.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void ln_fwd_generic(const T* __restrict__ x, const T* __restrict__ gamma,
                                                            const T* __restrict__ beta, float eps, T* __restrict__ y,
@@ -370,45 +415,63 @@ __global__ __launch_bounds__(kThreads) void ln_bwd_generic(const T* __restrict__
     }
 }
 
-// The vector kernels need 16-byte aligned rows of whole 16-byte groups.
+constexpr int64_t kMaxRegCols = 1024 * 16;   // the widest row held in registers (16 waves)
+
+// 16-byte accesses need 16-byte aligned rows of whole 16-byte groups.
 template <typename T>
 bool vec_ok(int64_t d, std::initializer_list<const void*> ptrs) {
-    if (d % Pack16<T>::N != 0 || d > 2048) return false;
+    if (d % Pack16<T>::N != 0) return false;
     for (const void* p : ptrs)
         if ((uintptr_t)p % 16 != 0) return false;
     return true;
 }
 
-// Row values per lane for the vector kernels: 4, 8, 16 or 32, at least one
-// 16-byte group.
-template <typename T>
-int dpl_for(int64_t d) {
-    const int dpl = d <= 256 ? 4 : d <= 512 ? 8 : d <= 1024 ? 16 : 32;
-    return dpl < Pack16<T>::N ? Pack16<T>::N : dpl;
+// The kernel shape of a row length, as f(DPL, G, WPR constants): the fewest
+// waves per row that leave a lane at most 16 values.
+template <typename T, int G, class F>
+void for_shape_g(int64_t d, F f) {
+    constexpr int kLeast = G > 4 ? G : 4;
+    if (kLeast == 4 && d <= 64 * 4) f.template operator()<kLeast == 4 ? 4 : 8, G, 1>();
+    else if (d <= 64 * 8) f.template operator()<8, G, 1>();
+    else if (d <= 64 * 16) f.template operator()<16, G, 1>();
+    else if (d <= 128 * 16) f.template operator()<16, G, 2>();
+    else if (d <= 256 * 16) f.template operator()<16, G, 4>();
+    else if (d <= 512 * 16) f.template operator()<16, G, 8>();
+    else f.template operator()<16, G, 16>();
 }
+template <typename T, class F>
+void for_shape(bool vec, int64_t d, F f) {
+    if (vec) for_shape_g<T, Pack16<T>::N>(d, f);
+    else for_shape_g<T, 1>(d, f);
+}
+
+template <typename T>
+struct FwdArgs {
+    nott_ctx ctx;
+    const T *x, *gamma, *beta;
+    float eps;
+    T* y;
+    float *mean, *rstd;
+    int64_t rows, d;
+    template <int DPL, int G, int WPR>
+    void operator()() const {
+        constexpr int GROUPS = WPR < kWaves ? kWaves / WPR : 1;
+        const int64_t blocks = std::min<int64_t>(nott::ceil_div(rows, GROUPS), (int64_t)ctx->num_cu * 8);
+        hipLaunchKernelGGL((ln_fwd_kernel<T, DPL, G, WPR, GROUPS>), dim3((unsigned)blocks), dim3(64 * WPR * GROUPS), 0,
+                           ctx->stream, x, gamma, beta, eps, y, mean, rstd, rows, d);
+    }
+};
 
 template <typename T>
 int fwd(nott_ctx ctx, int64_t rows, int64_t d, const void* x, const void* gamma, const void* beta, float eps, void* y,
         float* mean, float* rstd) {
-    const T* xx = static_cast<const T*>(x);
-    const T* gg = static_cast<const T*>(gamma);
-    const T* bb = static_cast<const T*>(beta);
-    T* yy = static_cast<T*>(y);
-    const bool vec = vec_ok<T>(d, {x, gamma, beta, y});
-    const int64_t blocks = std::min<int64_t>(nott::ceil_div(rows, kWaves), (int64_t)ctx->num_cu * 8);
-    const dim3 grid((unsigned)std::max<int64_t>(blocks, 1));
-    const int dpl = vec ? dpl_for<T>(d) : 0;
-    if (dpl == 4)
-        hipLaunchKernelGGL((ln_fwd_kernel<T, 4>), grid, dim3(kThreads), 0, ctx->stream, xx, gg, bb, eps, yy, mean, rstd, rows, d);
-    else if (dpl == 8)
-        hipLaunchKernelGGL((ln_fwd_kernel<T, 8>), grid, dim3(kThreads), 0, ctx->stream, xx, gg, bb, eps, yy, mean, rstd, rows, d);
-    else if (dpl == 16)
-        hipLaunchKernelGGL((ln_fwd_kernel<T, 16>), grid, dim3(kThreads), 0, ctx->stream, xx, gg, bb, eps, yy, mean, rstd, rows, d);
-    else if (dpl == 32)
-        hipLaunchKernelGGL((ln_fwd_kernel<T, 32>), grid, dim3(kThreads), 0, ctx->stream, xx, gg, bb, eps, yy, mean, rstd, rows, d);
+    const FwdArgs<T> a{ctx, static_cast<const T*>(x), static_cast<const T*>(gamma), static_cast<const T*>(beta), eps,
+                       static_cast<T*>(y), mean, rstd, rows, d};
+    if (d <= kMaxRegCols)
+        for_shape<T>(vec_ok<T>(d, {x, gamma, beta, y}), d, a);
     else
-        hipLaunchKernelGGL(ln_fwd_generic<T>, dim3((unsigned)rows), dim3(kThreads), 0, ctx->stream, xx, gg, bb, eps, yy,
-                           mean, rstd, d);
+        hipLaunchKernelGGL(ln_fwd_generic<T>, dim3((unsigned)rows), dim3(kThreads), 0, ctx->stream, a.x, a.gamma, a.beta,
+                           eps, a.y, mean, rstd, d);
     return nott::launch_status(ctx, "layernorm_fwd");
 }
 
@@ -419,33 +482,40 @@ int fwd(nott_ctx ctx, int64_t rows, int64_t d, const void* x, const void* gamma,
 constexpr size_t kScratchBytes = size_t(16) << 20;
 static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
 
-// Waves per block of the vector backward kernel: 8 while the block's LDS
-// column sums (waves × 2 × d floats) fit 64 KB, else 4.
-inline int bwd_waves(int64_t d) { return d <= 1024 ? 8 : 4; }
+// Rows a block of the backward takes at a time: 8 waves over the waves per row.
+constexpr int bwd_groups(int wpr) { return wpr < 8 ? 8 / wpr : 1; }
 
-// Partials need: 2 rows (dgamma, dbeta) of `pcols` columns per block.
 template <typename T>
-void partial_plan(nott_ctx ctx, int64_t rows, int64_t d, bool vec, int dpl, int64_t& nparts, size_t& pcols) {
-    (void)dpl;
-    if (vec) {
-        nparts = std::min<int64_t>(nott::ceil_div(rows, bwd_waves(d)), (int64_t)ctx->num_cu);
-        nparts = std::max<int64_t>(nparts, 1);
-    } else {
-        nparts = rows;
+struct BwdArgs {
+    nott_ctx ctx;
+    const T *x, *dy;
+    const float *mean, *rstd;
+    const T* gamma;
+    T* dx;
+    float* partial;
+    int64_t rows, d;
+    int64_t* nparts;   // in: at most this many blocks (0: plan only); out: blocks
+    template <int DPL, int G, int WPR>
+    void operator()() const {
+        constexpr int GROUPS = bwd_groups(WPR);
+        const int64_t most = std::max<int64_t>(
+            1, std::min<int64_t>(nott::ceil_div(rows, GROUPS), (int64_t)ctx->num_cu));
+        if (!partial) {
+            *nparts = most;
+            return;
+        }
+        // at most 64 KB, beside the kernel's own few words
+        const size_t lds = GROUPS > 1 ? sizeof(float) * GROUPS * 2 * (size_t)d : 0;
+        static bool attr = false;
+        if (GROUPS > 1 && !attr) {
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ln_bwd_kernel<T, DPL, G, WPR, GROUPS>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)(64 << 10));
+            attr = true;
+        }
+        hipLaunchKernelGGL((ln_bwd_kernel<T, DPL, G, WPR, GROUPS>), dim3((unsigned)*nparts), dim3(64 * WPR * GROUPS),
+                           lds, ctx->stream, x, dy, mean, rstd, gamma, dx, partial, rows, d);
     }
-    pcols = vec ? (size_t)nott::ceil_div(d, 16) * 16 : (size_t)d;
-}
-
-template <typename T, int DPL>
-void launch_bwd_vec(nott_ctx ctx, dim3 grid, const T* x, const T* dy, const float* mean, const float* rstd,
-                    const T* gamma, T* dx, float* partial, int64_t rows, int64_t d) {
-    if (bwd_waves(d) == 8)
-        hipLaunchKernelGGL((ln_bwd_kernel<T, DPL, 8>), grid, dim3(512), sizeof(float) * 8 * 2 * (size_t)d, ctx->stream,
-                           x, dy, mean, rstd, gamma, dx, partial, rows, d);
-    else
-        hipLaunchKernelGGL((ln_bwd_kernel<T, DPL, 4>), grid, dim3(256), sizeof(float) * 4 * 2 * (size_t)d, ctx->stream,
-                           x, dy, mean, rstd, gamma, dx, partial, rows, d);
-}
+};
 
 // `fixed` (nullable) replaces the context workspace for the partials;
 // `fixed_bytes` is its size.
@@ -453,45 +523,45 @@ template <typename T>
 int bwd(nott_ctx ctx, int64_t rows, int64_t d, const void* x, const void* dy, const float* mean, const float* rstd,
         const void* gamma, void* dx, float* dgamma, float* dbeta, int accumulate, float* fixed = nullptr,
         size_t fixed_bytes = 0) {
-    const T* xx = static_cast<const T*>(x);
-    const T* dd = static_cast<const T*>(dy);
-    const T* gg = static_cast<const T*>(gamma);
-    T* out = static_cast<T*>(dx);
-    const bool vec = vec_ok<T>(d, {x, dy, gamma, dx});
-    const int dpl = vec ? dpl_for<T>(d) : 0;
-    int64_t nparts;
-    size_t pcols;
-    partial_plan<T>(ctx, rows, d, vec, dpl, nparts, pcols);
-    const size_t need = sizeof(float) * 2 * pcols * (size_t)nparts;
-    float* partial;
+    int64_t nparts = 0;
+    BwdArgs<T> a{ctx, static_cast<const T*>(x), static_cast<const T*>(dy), mean, rstd, static_cast<const T*>(gamma),
+                 static_cast<T*>(dx), nullptr, rows, d, &nparts};
+    const bool vec = vec_ok<T>(d, {x, dy, gamma, dx}), reg = d <= kMaxRegCols;
+    // Partials: 2 rows (dgamma, dbeta) of `pcols` columns per block.
+    size_t pcols = (size_t)d;
+    if (reg) {
+        for_shape<T>(vec, d, a);   // the block count
+        pcols = (size_t)nott::ceil_div(d, 16) * 16;
+    } else {
+        nparts = rows;
+    }
     if (fixed) {
-        if (need > fixed_bytes)
+        // The entry point's bound is 8·d bytes a row outside aligned rows of up
+        // to 2048 columns; inside it the blocks' partials fit (fewer blocks where
+        // the columns' rounding to 16 would not).
+        const size_t bound = vec && d <= 2048 ? 0 : sizeof(float) * 2 * (size_t)d * (size_t)rows;
+        if (bound > fixed_bytes)
             return nott::fail(ctx, NOTT_ERR_UNSUPPORTED,
                               "nott_layernorm_bwd_noalloc: rows=" + std::to_string(rows) + ", d=" + std::to_string(d) +
-                                  " needs " + std::to_string(need) + " bytes of scratch; the static scratch holds " +
+                                  " needs " + std::to_string(bound) + " bytes of scratch; the static scratch holds " +
                                   std::to_string(fixed_bytes));
-        partial = fixed;
+        if (reg) nparts = std::min<int64_t>(nparts, (int64_t)(fixed_bytes / (sizeof(float) * 2 * pcols)));
+        a.partial = fixed;
     } else {
-        partial = static_cast<float*>(nott::workspace(ctx, need));
-        if (!partial) return NOTT_ERR_ALLOC;
+        a.partial = static_cast<float*>(nott::workspace(ctx, sizeof(float) * 2 * pcols * (size_t)nparts));
+        if (!a.partial) return NOTT_ERR_ALLOC;
     }
-    const dim3 grid((unsigned)nparts);
-    if (dpl == 4)
-        launch_bwd_vec<T, 4>(ctx, grid, xx, dd, mean, rstd, gg, out, partial, rows, d);
-    else if (dpl == 8)
-        launch_bwd_vec<T, 8>(ctx, grid, xx, dd, mean, rstd, gg, out, partial, rows, d);
-    else if (dpl == 16)
-        launch_bwd_vec<T, 16>(ctx, grid, xx, dd, mean, rstd, gg, out, partial, rows, d);
-    else if (dpl == 32)
-        launch_bwd_vec<T, 32>(ctx, grid, xx, dd, mean, rstd, gg, out, partial, rows, d);
+    if (reg)
+        for_shape<T>(vec, d, a);
     else
-        hipLaunchKernelGGL(ln_bwd_generic<T>, grid, dim3(kThreads), 0, ctx->stream, xx, dd, mean, rstd, gg, out, partial, d);
-    if ((dgamma || dbeta) && vec)
+        hipLaunchKernelGGL(ln_bwd_generic<T>, dim3((unsigned)nparts), dim3(kThreads), 0, ctx->stream, a.x, a.dy, mean,
+                           rstd, a.gamma, a.dx, a.partial, d);
+    if ((dgamma || dbeta) && reg)
         hipLaunchKernelGGL(col_reduce_grouped_kernel, dim3((unsigned)(2 * nott::ceil_div(d, 16))), dim3(256), 0,
-                           ctx->stream, partial, nparts, d, dgamma, dbeta, accumulate);
+                           ctx->stream, a.partial, nparts, d, dgamma, dbeta, accumulate);
     else if (dgamma || dbeta)
-        hipLaunchKernelGGL(col_reduce_kernel, dim3((unsigned)nott::ceil_div(d, 64), 2), dim3(kReduceThreads), 0, ctx->stream,
-                           partial, nparts, d, dgamma, dbeta, accumulate);
+        hipLaunchKernelGGL(col_reduce_kernel, dim3((unsigned)nott::ceil_div(d, 64), 2), dim3(kReduceThreads), 0,
+                           ctx->stream, a.partial, nparts, d, dgamma, dbeta, accumulate);
     return nott::launch_status(ctx, "layernorm_bwd");
 }
 
