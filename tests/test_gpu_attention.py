@@ -55,12 +55,25 @@ CASES = [
     (1, 2, 300, 300, 64, True),
     (1, 2, 200, 330, 64, False),
     (2, 1, 257, 129, 64, True),
+    # every padded head size of the 32x32 bf16 kernels (32, 64, 96, 128 columns;
+    # whole and partly zero), one short tile and ragged ends over several blocks
+    (1, 2, 140, 140, 8, True),
+    (2, 1, 40, 200, 32, False),
+    (1, 3, 161, 161, 40, False),
+    (1, 2, 300, 270, 72, False),
+    (2, 1, 190, 190, 80, True),
+    (1, 2, 129, 65, 96, True),
+    (1, 1, 260, 260, 104, False),
+    (1, 2, 300, 300, 128, True),
+    (1, 1, 1, 1, 128, True),
 ]
+CASES_F32 = [c for c in CASES if c[4] <= 64]   # (fp32 takes head sizes up to 64)
 
 
-@pytest.mark.parametrize("dt", ["f32", "bf16"])
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "b{}h{}t{}s{}d{}c{}".format(*c))
+@pytest.mark.parametrize("dt,case", [("f32", c) for c in CASES_F32] + [("bf16", c) for c in CASES],
+                         ids=lambda c: "b{}h{}t{}s{}d{}c{}".format(*c) if isinstance(c, tuple) else c)
 def test_attention_vs_oracle(ops, oracle, dt, case):
+    print(f"attention {dt} {case}", flush=True)
     b, h, t, s, dh, causal = case
     g = rng(sum(case) + len(dt))
     q = host_input(g.standard_normal((b, h, t, dh)), dt)
@@ -81,6 +94,25 @@ def test_attention_vs_oracle(ops, oracle, dt, case):
     check(host(dq), rdq, dt, "dq")
     check(host(dk), rdk, dt, "dk")
     check(host(dv), rdv, dt, "dv")
+
+
+@pytest.mark.parametrize("scale", [None, -0.3, 0.0])
+@pytest.mark.parametrize("case", [(1, 2, 200, 330, 64, False), (1, 1, 300, 300, 128, True), (1, 1, 150, 150, 32, True)])
+def test_attention_bf16_growing_scores(ops, oracle, case, scale):
+    """Scores of up to hundreds that grow along the keys, so that the running
+    maximum moves in most tiles; a negative and a zero scale."""
+    b, h, t, s, dh, causal = case
+    print(f"attention bf16 growing {case} scale {scale}", flush=True)
+    g = rng(t + s + dh)
+    q = host_input(g.standard_normal((b, h, t, dh)) * 3, "bf16")
+    k = host_input(g.standard_normal((b, h, s, dh)) * np.linspace(0.1, 3, s)[:, None], "bf16")
+    v = host_input(g.standard_normal((b, h, s, dh)), "bf16")
+    d = ops.attn_desc(b, h, t, s, dh, causal, scale=scale)
+    o, lse = ops.attention_fwd(dev(q, "bf16"), dev(k, "bf16"), dev(v, "bf16"), d)
+    ro, rlse = oracle.attention_fwd(d, q, k, v)
+    torch.cuda.synchronize()
+    check(host(o), ro, "bf16", "o")
+    check(host(lse), rlse, "bf16", "lse")
 
 
 def _torch_attention_fp32(q, k, v, dO, causal, scale):

@@ -681,40 +681,26 @@ __global__ __launch_bounds__(kThreads) void attn_dq_kernel(const T* __restrict__
 }
 
 // ===========================================================================
-// bf16 backward for head dim 64 on 32×32×16 MFMAs.
+// bf16 on 32×32×16 MFMAs, any head dim that is a multiple of 8 up to 128
+// (16-byte aligned rows), padded to ND = 1..4 blocks of 32.
 //
-// Two deterministic passes, each streaming 64-row tiles of the other side
-// through an LDS ring filled by direct-to-LDS loads:
-//   attn_dq64:   one workgroup per 128 query rows (4 waves × 32); forms
-//                D = rowsum(dO∘O) for its rows (written for the next pass),
-//                then per 64-key block: sᵀ = k·qᵀ, dpᵀ = v·dOᵀ, dsᵀ, and
-//                dq += ds·k.
-//   attn_dkdv64: one workgroup per 128 keys (4 waves × 32); per 64-query
-//                block: s = q·kᵀ, dp = dO·vᵀ, p, ds, dv += pᵀ·dO and
-//                dk += dsᵀ·q.
-// Each wave keeps its own 32 rows of the fixed side (q and dO, or k and v) as
-// MFMA B operands in registers for the whole pass.
+// A workgroup's 4 waves own 32 rows each of the fixed side (queries in the
+// forward), held in registers as MFMA B operands; 64-row tiles of the streamed
+// side go through an LDS ring filled by direct-to-LDS loads.  A tile is
+// [row][32·ND] bf16 in linear order, its 16-byte chunks permuted within a row
+// (swz below) so that both reads of it meet distinct banks: 16 rows of one
+// chunk (frag_rows), and 4 rows × 4 neighbouring chunks (frag_cols, transposing
+// reads).  Chunks past the head dim are filled with zeros.
 //
-// Precision.  p and ds enter the second-stage MFMAs as bf16.  Where a wave's
-// tile holds a probability of at least kLoTau (rows with few effective keys,
-// whose few large terms dominate their sums), the bf16 remainder
-// (x − bf16(x), rounded again) is multiplied as well, which carries ~16
-// mantissa bits; elsewhere a rounding error of 2^-9 relative on terms that
-// small stays far inside the bf16 tolerance.  D must be exact: D taken from
-// the bf16-rounded o is off by dO·δo, which shifts every ds of the row.  The
-// dq pass therefore uses D~ = rowsum(dO∘o_bf16) during its sweep, while it
-// accumulates the exact D = Σ_j p·dp and b = Σ_j p·k, and at the end sets
-// dq = scale·(Σ_j p(dp − D~)k − (D − D~)·b); the exact D is what it writes
-// for the dk/dv pass.  Score tiles are computed with
-// the fixed side as the B operand, so a lane's accumulator column is its own
-// row of the fixed side and its 16 registers are rows 8j + 4·(l/32) + e of
-// the streamed side; 8 consecutive registers are then exactly a 32×16 A
-// operand whose k-slots are streamed rows {4h..4h+3, 8+4h..8+4h+3} of a
-// 16-row slice, and the matching B operand is read from the streamed tile
-// with two transposing LDS reads (ds_read_b64_tr_b16, 4 rows each).
-// Tiles are [row][64] bf16 with 128-byte rows and 16-byte chunks swizzled by
-// (row>>1)&7, as in the direct-to-LDS GEMM.
-namespace a64 {
+// Bound by the exponentials and the products together (they share the issue
+// slots of two to four waves per SIMD).  Measured with inputs changing from
+// call to call, against the 16×16 kernels above (forward; backward outside head
+// dim 64, where D took a sweep of its own), b·h x t x dh:
+//   forward   128 x 1024 x 64 causal 61.7 -> 35.9 us, 32 x 4096 x 64 causal
+//             175 -> 103, 32 x 1000 x 128 full 52 -> 35.7 us;
+//   backward  32 x 1000 x 128 full 231 -> 137 us, 16 x 4096 x 128 full 1736 ->
+//             861, 64 x 1024 x 32 causal 80 -> 50, 32 x 777 x 80 full 181 -> 74.
+namespace fa {
 
 using nott::lds::barrier;
 using nott::lds::dma16;
@@ -724,60 +710,303 @@ using nott::lds::wait_vm_lgkm0;
 
 constexpr int NW = 4;                    // waves per workgroup, 32 fixed rows each
 constexpr int FIXED = 32 * NW;           // fixed rows per workgroup
-constexpr int TR = 64;                   // streamed rows per stage
-constexpr int TILE = TR * 128;           // one [64][64] bf16 tile
-constexpr int RING = 4;                  // stages in flight + 1
-constexpr float kLoTau = 1.f / 16;       // tile max of p above which the bf16 remainder is multiplied too
 
-__device__ __forceinline__ int toff64(int r, int c) { return r * 128 + ((c ^ ((r >> 1) & 7)) << 4); }
+static __device__ u32x4 zero_chunk;      // source of the padding columns
 
-// Fills a [64][64] tile with rows row0.. of `base` (row stride ld, rows past
-// nrows clamped to the last one): 8 blocks of 1 KB, two per wave.
-__device__ __forceinline__ void fill_tile(const bf16_t* base, int row0, int nrows, int ld, char NOTT_LDS* tile,
+// Where chunk c of row r sits in its row.  In 256 bytes of banks a row of 4·ND
+// chunks starts at chunk 4·ND·r mod 16; what is left of r's low 4 bits is
+// XORed in: all of a 16-chunk row's, 2 bits of a 4- or 12-chunk one's.
+template <int ND>
+__device__ __forceinline__ int swz(int r, int c) {
+    if constexpr (ND == 4) return c ^ (((r & 3) << 2) | ((r >> 2) & 3));
+    else if constexpr (ND == 2) return c ^ ((r >> 1) & 7);
+    else return c ^ ((r >> 2) & 3);
+}
+template <int ND>
+__device__ __forceinline__ int tile_off(int r, int c) { return r * (64 * ND) + (swz<ND>(r, c) << 4); }
+
+// Fills a [ROWS][32·ND] tile with rows row0.. of `base` (row stride ld, rows
+// past nrows clamped to the last): 1 KB blocks dealt to the waves.
+template <int ND, int ROWS>
+__device__ __forceinline__ void fill_tile(const bf16_t* base, int row0, int nrows, int dh, int ld, char NOTT_LDS* tile,
                                           int wid, int lane) {
+    constexpr int CH = 4 * ND, BLOCKS = ROWS * CH / 64;
+    static_assert(BLOCKS % NW == 0, "blocks split evenly over the waves");
 #pragma unroll
-    for (int qq = 0; qq < 8 / NW; ++qq) {
+    for (int qq = 0; qq < BLOCKS / NW; ++qq) {
         const int q = wid + NW * qq;
-        const int r = 8 * q + (lane >> 3);
-        const int c = (lane & 7) ^ ((r >> 1) & 7);
-        int gr = row0 + r;
-        gr = gr < nrows ? gr : nrows - 1;
-        dma16(base + (int64_t)gr * ld + 8 * c, lds_addr(tile) + 1024 * q);
+        const int i = 64 * q + lane, r = i / CH;
+        const int c = swz<ND>(r, i - r * CH);   // (an involution)
+        const int gr = min(row0 + r, nrows - 1);
+        const bf16_t* src = base + (int64_t)gr * ld + 8 * c;
+        dma16(8 * c < dh ? src : reinterpret_cast<const bf16_t*>(&zero_chunk), lds_addr(tile) + 1024 * q);
     }
 }
 
 // 32×16 operand of tile rows r0..r0+31, d slice s: lane l gets row r0 + l%32,
 // d = 16s + 8·(l/32) + 0..7.
+template <int ND>
 __device__ __forceinline__ bf16x8 frag_rows(const char NOTT_LDS* tile, int r0, int s, int lane) {
-    const int r = r0 + (lane & 31);
-    return __builtin_bit_cast(bf16x8,
-                              *reinterpret_cast<const u32x4 NOTT_LDS*>(tile + toff64(r, 2 * s + (lane >> 5))));
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 NOTT_LDS*>(
+                                          tile + tile_off<ND>(r0 + (lane & 31), 2 * s + (lane >> 5))));
 }
 
 typedef short v4i16s __attribute__((ext_vector_type(4)));
 
-// B operand over a 16-row slice starting at tile row rs: lane l gets column
-// d0 + l%32 and rows rs + 4h + 0..3, rs + 8 + 4h + 0..3 (h = l/32).
+// 32×16 operand of the transposed tile over the 16 rows from rs: lane l gets
+// column d0 + l%32 and, as its 8 k-slots, rows rs + 4h + 0..3, rs + 8 + 4h +
+// 0..3 (h = l/32): the rows that 8 consecutive registers of a 32×32
+// accumulator hold, so a score tile is the other operand as it is.
+template <int ND>
 __device__ __forceinline__ bf16x8 frag_cols(const char NOTT_LDS* tile, int rs, int d0, int lane) {
     const int j = lane & 15, g = lane >> 4;
     const int col = d0 + 16 * (g & 1) + 4 * (j & 3);
     const int r1 = rs + 4 * (g >> 1) + (j >> 2);
     const int byte = (col & 7) * 2;
-    const v4i16s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16s NOTT_LDS*)(tile + toff64(r1, col >> 3) + byte));
+    const v4i16s lo =
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16s NOTT_LDS*)(tile + tile_off<ND>(r1, col >> 3) + byte));
     const v4i16s hi =
-        __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16s NOTT_LDS*)(tile + toff64(r1 + 8, col >> 3) + byte));
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16s NOTT_LDS*)(tile + tile_off<ND>(r1 + 8, col >> 3) + byte));
     const v4i16s w[2] = {lo, hi};
     return __builtin_bit_cast(bf16x8, w);
 }
 
-// Registers base..base+7 of an accumulator tile as a bf16 A operand.
+// Registers base..base+7 of an accumulator tile as a bf16 operand.
 __device__ __forceinline__ bf16x8 pack8(const f32x16& t, int base) {
     const u32x4 w = {pack_bf16x2(t[base], t[base + 1]), pack_bf16x2(t[base + 2], t[base + 3]),
                      pack_bf16x2(t[base + 4], t[base + 5]), pack_bf16x2(t[base + 6], t[base + 7])};
     return __builtin_bit_cast(bf16x8, w);
 }
 
-// The remainder x − bf16(x) of the same 8 registers, rounded to bf16.
+__device__ __forceinline__ f32x16 mfma(const bf16x8& a, const bf16x8& b, const f32x16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Maximum over lanes l and l ^ 32 (permlane32_swap of a value with itself gives
+// the lower and the upper half's in every lane).
+__device__ __forceinline__ float max_halves(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x),
+                                                    false, false);
+    // through scalars: a bit-cast of a vector's element 1 reads element 0 (hipcc, ROCm 7.2)
+    const unsigned lo = r[0], hi = r[1];
+    return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+
+// A row's values as 2·ND B-operand slices: lane l holds d = 16s + 8·(l/32) + 0..7.
+template <int ND>
+__device__ __forceinline__ void load_fixed(const bf16_t* base, int row, int nrows, int dh, int ld, int lane,
+                                           u32x4 (&r)[2 * ND]) {
+    const bf16_t* pr = base + (int64_t)min(row, nrows - 1) * ld;
+#pragma unroll
+    for (int s = 0; s < 2 * ND; ++s) {
+        const int d = 16 * s + 8 * (lane >> 5);
+        r[s] = *reinterpret_cast<const u32x4*>(pr + (d < dh ? d : 0));
+        if (d >= dh) r[s] = u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// Forward: o and lse of 128 queries, 64 keys per stage.  Scores are formed
+// transposed (k·qᵀ), so a lane's accumulator column is its own query: the row
+// maximum and sum need one exchange between the two lanes of a query, and oᵀ +=
+// vᵀ·pᵀ keeps the output in the same lane, so the rescale by 2^(m − m') is a
+// lane's own.  It is skipped where no row's maximum grew (letting the maximum
+// lag behind by up to 2^8 saved more of them and 3 us of 36 at 128 x 1024 x 64, but
+// then the largest probability is no longer exactly 1, and its rounding to bf16
+// took the output's error at 1000 keys from 2.2e-3 to 2.3e-3).
+template <int ND, int RING>
+__global__ __launch_bounds__(64 * NW, 2) void attn_fwd32_kernel(const bf16_t* __restrict__ q,
+                                                                const bf16_t* __restrict__ k,
+                                                                const bf16_t* __restrict__ v, bf16_t* __restrict__ o,
+                                                                float* __restrict__ lse, AttnParams p) {
+    constexpr int TR = 64, TILE = TR * 64 * ND, STAGE = 2 * TILE;
+    constexpr int LOADS = 2 * (TR * 4 * ND / 64) / NW;   // per wave and stage
+    extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
+    char NOTT_LDS* smem = (char NOTT_LDS*)smem_raw;
+    const int bh = blockIdx.x;
+    const int nqb = (p.t + FIXED - 1) / FIXED;
+    const int q0 = (nqb - 1 - (int)blockIdx.y) * FIXED;   // heaviest (causal) blocks first
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int h = lane >> 5;
+    const int qw0 = q0 + 32 * wid;
+    const int my_q = qw0 + (lane & 31);
+    const int64_t qoff = bh_off(bh, p.nh, p.sbq, p.shq), koff = bh_off(bh, p.nh, p.sbk, p.shk);
+    const int64_t ooff = bh_off(bh, p.nh, p.sbo, p.sho);
+    const float sl2 = p.scale * 1.4426950408889634f;
+    const bool neg = sl2 < 0.f;
+    const float masked = neg ? INFINITY : -INFINITY;     // −inf once scaled
+
+    u32x4 qr[2 * ND];
+    load_fixed<ND>(q + qoff, my_q, p.t, p.dh, p.ldq, lane, qr);
+    int nk = p.nkb;   // 64-key blocks
+    if (p.causal) nk = min(nk, (q0 + FIXED - 1) / TR + 1);
+    auto issue = [&](int i, int slot) {
+        char NOTT_LDS* st = smem + slot * STAGE;
+        fill_tile<ND, TR>(k + koff, i * TR, p.s, p.dh, p.ldk, st, wid, lane);
+        fill_tile<ND, TR>(v + koff, i * TR, p.s, p.dh, p.ldk, st + TILE, wid, lane);
+    };
+#pragma unroll
+    for (int i = 0; i < RING - 1; ++i)
+        if (i < nk) issue(i, i);
+
+    f32x16 acc[ND];
+#pragma unroll
+    for (int f = 0; f < ND; ++f)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[f][e] = 0.f;
+    float m = -INFINITY, l = 0.f;   // l: this lane's keys only
+    int slot = 0, next = RING - 1;
+    for (int i = 0; i < nk; ++i) {
+        if (i + RING - 2 < nk) wait_vm_lgkm0<(RING - 2) * LOADS>();
+        else wait_vm_lgkm0<0>();
+        barrier();
+        if (i + RING - 1 < nk) issue(i + RING - 1, next);
+        const char NOTT_LDS* tk = smem + slot * STAGE;
+        const char NOTT_LDS* tv = tk + TILE;
+        slot = slot + 1 == RING ? 0 : slot + 1;
+        next = next + 1 == RING ? 0 : next + 1;
+        const int k0 = i * TR;
+        if ((p.causal && k0 > qw0 + 31) || qw0 >= p.t) continue;   // every key of the block masked for this wave
+        const bool full = k0 + TR <= p.s && (!p.causal || k0 + TR - 1 <= qw0);
+        const int rel = min(p.s, p.causal ? my_q + 1 : p.s) - k0 - 4 * h;
+        f32x16 st[2];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) st[f][e] = 0.f;
+#pragma unroll
+            for (int s = 0; s < 2 * ND; ++s)
+                st[f] = mfma(frag_rows<ND>(tk, 32 * f, s, lane), __builtin_bit_cast(bf16x8, qr[s]), st[f]);
+        }
+        // 32 keys at a time, so that one half's exponentials run beside the
+        // other half's products.
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            // Masking only on blocks that touch the diagonal or the end:
+            // element (f, r) is key k0 + 4h + c, c = 32f + 8(r/4) + r%4, kept
+            // iff c < rel.
+            if (!full) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (!(32 * f + 8 * (r >> 2) + (r & 3) < rel)) st[f][r] = masked;
+            }
+            float mx = st[f][0];
+            if (!neg) {
+#pragma unroll
+                for (int r = 1; r < 16; ++r) mx = fmaxf(mx, st[f][r]);
+            } else {
+#pragma unroll
+                for (int r = 1; r < 16; ++r) mx = fminf(mx, st[f][r]);
+            }
+            mx = max_halves(mx * sl2);   // log2 domain
+            if (__any(mx > m)) {
+                const float mn = fmaxf(m, mx);
+                const float alpha = __builtin_amdgcn_exp2f(mn == -INFINITY ? 0.f : m - mn);
+                l *= alpha;
+#pragma unroll
+                for (int df = 0; df < ND; ++df)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[df][e] *= alpha;
+                m = mn;
+            }
+            const float ms = m == -INFINITY ? 0.f : m;   // (a row with no unmasked key so far)
+            float rs = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                st[f][r] = __builtin_amdgcn_exp2f(fmaf(st[f][r], sl2, -ms));
+                rs += st[f][r];
+            }
+            l += rs;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const bf16x8 pb = pack8(st[f], 8 * s);
+#pragma unroll
+                for (int df = 0; df < ND; ++df)
+                    acc[df] = mfma(frag_cols<ND>(tv, 32 * f + 16 * s, 32 * df, lane), pb, acc[df]);
+            }
+        }
+    }
+    l += __shfl_xor(l, 32, 64);
+    if (my_q >= p.t) return;
+    const float inv = 1.f / l;
+    bf16_t* orow = o + ooff + (int64_t)my_q * p.ldo;
+#pragma unroll
+    for (int df = 0; df < ND; ++df)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int d = 32 * df + 8 * j + 4 * h;
+            if (d < p.dh)
+                *reinterpret_cast<u32x2*>(orow + d) = u32x2{pack_bf16x2(acc[df][4 * j] * inv, acc[df][4 * j + 1] * inv),
+                                                            pack_bf16x2(acc[df][4 * j + 2] * inv, acc[df][4 * j + 3] * inv)};
+        }
+    if (h == 0) lse[(int64_t)bh * p.t + my_q] = (m + log2f(l)) * 0.6931471805599453f;
+}
+
+template <int ND, int RING>
+int fwd_nd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* q, const void* k, const void* v,
+           void* o, float* lse) {
+    constexpr size_t lds = (size_t)RING * 2 * 64 * 64 * ND;
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd32_kernel<ND, RING>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        attr = true;
+    }
+    hipLaunchKernelGGL((attn_fwd32_kernel<ND, RING>), dim3((unsigned)(d->b * d->h), (unsigned)ceil_div(d->t, FIXED)),
+                       dim3(64 * NW), lds, ctx->stream, static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k),
+                       static_cast<const bf16_t*>(v), static_cast<bf16_t*>(o), lse, p);
+    return launch_status(ctx, "attention_fwd");
+}
+
+// Whether these kernels take a problem: 16-byte aligned bf16 rows in whole
+// 16-byte groups (the fills move 16-byte chunks), and a scale that a masked
+// score of ±inf survives.
+bool applies(const AttnParams& p, int elem) { return elem == 2 && p.vec && p.scale != 0.f; }
+
+int fwd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* q, const void* k, const void* v, void* o,
+        float* lse) {
+    // A 2-deep ring leaves room for four workgroups per CU at 64 columns (a 3-deep
+    // one is 13% slower at 128 x 1024 x 64 causal) and two at 128; with at most one
+    // per CU the ring is deeper instead.
+    const bool few = d->b * d->h * ceil_div(d->t, FIXED) <= ctx->num_cu;
+    if (d->dh <= 32) return fwd_nd<1, 2>(ctx, d, p, q, k, v, o, lse);
+    if (d->dh <= 64) return fwd_nd<2, 2>(ctx, d, p, q, k, v, o, lse);
+    if (d->dh <= 96) return fwd_nd<3, 2>(ctx, d, p, q, k, v, o, lse);
+    return few ? fwd_nd<4, 4>(ctx, d, p, q, k, v, o, lse) : fwd_nd<4, 2>(ctx, d, p, q, k, v, o, lse);
+}
+
+// ---- backward -------------------------------------------------------------
+// Two deterministic passes:
+//   attn_dq32:   one workgroup per 128 query rows; forms D = rowsum(dO∘O) for
+//                its rows (written for the next pass), then per step of 32·TF
+//                keys: sᵀ = k·qᵀ, dpᵀ = v·dOᵀ, dsᵀ, and dq += ds·k.
+//   attn_dkdv32: one workgroup per 128 keys; per step of 32·TF queries:
+//                s = q·kᵀ, dp = dO·vᵀ, p, ds, dv += pᵀ·dO and dk += dsᵀ·q.
+// Each wave keeps its own 32 rows of the fixed side (q and dO, or k and v) as
+// MFMA B operands in registers for the whole pass.  With 96 columns a step is
+// 32 rows (TF = 1), so that these, the two accumulators and the two score tiles
+// fit 256 registers (two waves per SIMD); 128 columns do not (49 registers
+// spilled: 237 us for 32 x 1000 x 128) and run one wave per SIMD with 64-row
+// steps (137 us; 149 with 32-row ones).  At head dim 64 32-row steps with three
+// waves per SIMD spilled and were slower (131 against 127 us for 128 x 1024).
+//
+// Precision.  p and ds enter the second-stage MFMAs as bf16 with the bf16
+// remainder (x − bf16(x), rounded again) multiplied as well, which carries ~16
+// mantissa bits; with TAU (head dim 64) only where a wave's tile holds a
+// probability of at least kLoTau (rows with few effective keys, whose few large
+// terms dominate their sums; elsewhere a rounding error of 2^-9 relative on
+// terms that small stays far inside the bf16 tolerance).  D must be exact: D
+// taken from the bf16-rounded o is off by dO·δo, which shifts every ds of the
+// row.  The dq pass therefore uses D~ = rowsum(dO∘o_bf16) during its sweep,
+// while it accumulates the exact D = Σ_j p·dp and b = Σ_j p·k, and at the end
+// sets dq = scale·(Σ_j p(dp − D~)k − (D − D~)·b); the exact D is what it writes
+// for the dk/dv pass.  Score tiles are computed with the fixed side as the B
+// operand, so a lane's accumulator column is its own row of the fixed side and
+// its 16 registers are rows 8j + 4·(l/32) + e of the streamed side; 8
+// consecutive registers are then exactly a 32×16 A operand whose k-slots are the
+// rows that frag_cols reads.
+constexpr float kLoTau = 1.f / 16;       // tile max of p above which the bf16 remainder is multiplied too
+
+// The remainder x − bf16(x) of registers base..base+7, rounded to bf16.
 __device__ __forceinline__ bf16x8 pack8_lo(const f32x16& t, int base, const bf16x8& hi) {
     const u32x4 h = __builtin_bit_cast(u32x4, hi);
     auto lo2 = [&](int i, uint32_t w) {
@@ -795,18 +1024,6 @@ __device__ __forceinline__ float wave_max(float x) {
     return x;
 }
 
-__device__ __forceinline__ f32x16 mfma(const bf16x8& a, const bf16x8& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// A row's 64 values as 4 B-operand slices: lane l holds d = 16s + 8·(l/32) + 0..7.
-__device__ __forceinline__ void load_fixed(const bf16_t* base, int row, int nrows, int ld, int lane, u32x4 (&r)[4]) {
-    const int rr = row < nrows ? row : nrows - 1;
-    const bf16_t* pr = base + (int64_t)rr * ld + 8 * (lane >> 5);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) r[s] = *reinterpret_cast<const u32x4*>(pr + 16 * s);
-}
-
 __device__ __forceinline__ float dot_bf16x8(const u32x4& a, const u32x4& b) {
     float s = 0.f;
 #pragma unroll
@@ -817,15 +1034,36 @@ __device__ __forceinline__ float dot_bf16x8(const u32x4& a, const u32x4& b) {
     return s;
 }
 
-__global__ __launch_bounds__(64 * NW, 2) void attn_dq64_kernel(const bf16_t* __restrict__ q,
-                                                                 const bf16_t* __restrict__ k,
-                                                                 const bf16_t* __restrict__ v,
-                                                                 const bf16_t* __restrict__ o,
-                                                                 const bf16_t* __restrict__ dO,
-                                                                 const float* __restrict__ lse,
-                                                                 float* __restrict__ dsum, float* __restrict__ lse2,
-                                                                 bf16_t* __restrict__ dq, AttnParams p) {
-    constexpr int STAGE = 2 * TILE;
+// Fills two [ROWS][32·ND] tiles, the second right behind the first, with rows
+// row0.. of a and b; their blocks are dealt to the waves together.
+template <int ND, int ROWS>
+__device__ __forceinline__ void fill_pair(const bf16_t* a, int lda, const bf16_t* b, int ldb, int row0, int nrows,
+                                          int dh, char NOTT_LDS* tile, int wid, int lane) {
+    constexpr int CH = 4 * ND, BLOCKS = ROWS * CH / 64;
+    static_assert(2 * BLOCKS % NW == 0, "blocks split evenly over the waves");
+#pragma unroll
+    for (int qq = 0; qq < 2 * BLOCKS / NW; ++qq) {
+        const int q = wid + NW * qq;
+        const bool second = BLOCKS % NW == 0 ? NW * qq >= BLOCKS : q >= BLOCKS;   // (mostly known at compile time)
+        const int i = 64 * (second ? q - BLOCKS : q) + lane, r = i / CH;
+        const int c = swz<ND>(r, i - r * CH);
+        const int gr = min(row0 + r, nrows - 1);
+        const bf16_t* src = (second ? b : a) + (int64_t)gr * (second ? ldb : lda) + 8 * c;
+        dma16(8 * c < dh ? src : reinterpret_cast<const bf16_t*>(&zero_chunk), lds_addr(tile) + 1024 * q);
+    }
+}
+
+template <int ND, int TF, int RING, bool TAU>
+__global__ __launch_bounds__(64 * NW, ND == 4 ? 1 : 2) void attn_dq32_kernel(const bf16_t* __restrict__ q,
+                                                               const bf16_t* __restrict__ k,
+                                                               const bf16_t* __restrict__ v,
+                                                               const bf16_t* __restrict__ o,
+                                                               const bf16_t* __restrict__ dO,
+                                                               const float* __restrict__ lse, float* __restrict__ dsum,
+                                                               float* __restrict__ lse2, bf16_t* __restrict__ dq,
+                                                               AttnParams p) {
+    constexpr int TR = 32 * TF, TILE = TR * 64 * ND, STAGE = 2 * TILE;
+    constexpr int LOADS = 2 * (TR * 4 * ND / 64) / NW;   // per wave and stage
     extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
     char NOTT_LDS* smem = (char NOTT_LDS*)smem_raw;
     const int bh = blockIdx.x;
@@ -838,42 +1076,41 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq64_kernel(const bf16_t* __r
     const int64_t qoff = bh_off(bh, p.nh, p.sbq, p.shq), koff = bh_off(bh, p.nh, p.sbk, p.shk);
     const int64_t ooff = bh_off(bh, p.nh, p.sbo, p.sho);
     const float sl2 = p.scale * 1.4426950408889634f;
+    const int dh = TAU ? 32 * ND : p.dh;
 
-    u32x4 qr[4], dr[4];
-    load_fixed(q + qoff, my_q, p.t, p.ldq, lane, qr);
-    load_fixed(dO + ooff, my_q, p.t, p.ldo, lane, dr);
+    u32x4 qr[2 * ND], dr[2 * ND];
+    load_fixed<ND>(q + qoff, my_q, p.t, dh, p.ldq, lane, qr);
+    load_fixed<ND>(dO + ooff, my_q, p.t, dh, p.ldo, lane, dr);
     float my_d;
     {
-        u32x4 orr[4];
-        load_fixed(o + ooff, my_q, p.t, p.ldo, lane, orr);
+        u32x4 orr[2 * ND];
+        load_fixed<ND>(o + ooff, my_q, p.t, dh, p.ldo, lane, orr);
         float s = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s += dot_bf16x8(dr[i], orr[i]);
+        for (int i = 0; i < 2 * ND; ++i) s += dot_bf16x8(dr[i], orr[i]);
         my_d = s + __shfl_xor(s, 32, 64);
     }
     const bool q_in = my_q < p.t;
     const float my_lse2 = lse[(int64_t)bh * p.t + (q_in ? my_q : p.t - 1)] * 1.4426950408889634f;
 
-    int nk = p.nkb;   // 64-key blocks
+    int nk = (p.s + TR - 1) / TR;
     if (p.causal) nk = min(nk, (q0 + FIXED - 1) / TR + 1);
     auto issue = [&](int i, int slot) {
-        char NOTT_LDS* st = smem + slot * STAGE;
-        fill_tile(k + koff, i * TR, p.s, p.ldk, st, wid, lane);
-        fill_tile(v + koff, i * TR, p.s, p.ldk, st + TILE, wid, lane);
+        fill_pair<ND, TR>(k + koff, p.ldk, v + koff, p.ldk, i * TR, p.s, dh, smem + slot * STAGE, wid, lane);
     };
 #pragma unroll
     for (int i = 0; i < RING - 1; ++i)
         if (i < nk) issue(i, i);
 
-    f32x16 adq[2], abv[2];
+    f32x16 adq[ND], abv[ND];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < ND; ++f)
 #pragma unroll
         for (int e = 0; e < 16; ++e) adq[f][e] = abv[f][e] = 0.f;
     float d_exact = 0.f;   // Σ p·dp over this lane's keys (its half of the row)
     int slot = 0, next = RING - 1;
     for (int i = 0; i < nk; ++i) {
-        if (i + RING - 2 < nk) wait_vm_lgkm0<(RING - 2) * 2 * (8 / NW)>();
+        if (i + RING - 2 < nk) wait_vm_lgkm0<(RING - 2) * LOADS>();
         else wait_vm_lgkm0<0>();
         barrier();
         if (i + RING - 1 < nk) issue(i + RING - 1, next);
@@ -883,62 +1120,66 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq64_kernel(const bf16_t* __r
         next = next + 1 == RING ? 0 : next + 1;
         const int k0 = i * TR;
         if ((p.causal && k0 > qw0 + 31) || qw0 >= p.t) continue;   // every key of the block masked for this wave
-        f32x16 st[2], dpt[2];
+        f32x16 st[TF], dpt[TF];
 #pragma unroll
-        for (int f = 0; f < 2; ++f) {
+        for (int f = 0; f < TF; ++f) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) st[f][e] = dpt[f][e] = 0.f;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                st[f] = mfma(frag_rows(tk, 32 * f, s, lane), __builtin_bit_cast(bf16x8, qr[s]), st[f]);
-                dpt[f] = mfma(frag_rows(tv, 32 * f, s, lane), __builtin_bit_cast(bf16x8, dr[s]), dpt[f]);
+            for (int s = 0; s < 2 * ND; ++s) {
+                st[f] = mfma(frag_rows<ND>(tk, 32 * f, s, lane), __builtin_bit_cast(bf16x8, qr[s]), st[f]);
+                dpt[f] = mfma(frag_rows<ND>(tv, 32 * f, s, lane), __builtin_bit_cast(bf16x8, dr[s]), dpt[f]);
             }
         }
         // exponent arguments (log2 domain) in place
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < TF; ++f)
 #pragma unroll
             for (int r = 0; r < 16; ++r) st[f][r] = fmaf(st[f][r], sl2, -my_lse2);
         // Masking only on blocks that touch the diagonal or the end (a
         // wave-uniform test).  Element (f, r) is key k0 + 4h + c with
-        // c = 32f + 8(r/4) + r%4 (0..59), kept iff c < rel: one compare against
-        // a constant, no per-element branches.
+        // c = 32f + 8(r/4) + r%4, kept iff c < rel: one compare against a
+        // constant, no per-element branches.
         if (!(qw0 + 32 <= p.t && k0 + TR <= p.s && (!p.causal || k0 + TR - 1 <= qw0))) {
             const int rel = q_in ? min(p.s, p.causal ? my_q + 1 : p.s) - k0 - 4 * h : -1;
 #pragma unroll
-            for (int f = 0; f < 2; ++f)
+            for (int f = 0; f < TF; ++f)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     if (!(32 * f + 8 * (r >> 2) + (r & 3) < rel)) st[f][r] = -INFINITY;
         }
+        // 32 keys at a time, so that one half's exponentials run beside the
+        // other half's products.
         float pmax = 0.f;
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < TF; ++f) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float pe = __builtin_amdgcn_exp2f(st[f][r]);
                 d_exact += pe * dpt[f][r];
-                pmax = fmaxf(pmax, pe);
+                if (TAU) pmax = fmaxf(pmax, pe);
                 st[f][r] = pe;
                 dpt[f][r] = pe * (dpt[f][r] - my_d);
             }
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const bf16x8 a = pack8(dpt[s >> 1], 8 * (s & 1));
-            const bf16x8 pa = pack8(st[s >> 1], 8 * (s & 1));
+            for (int s = 0; s < 2; ++s) {
+                const bf16x8 a = pack8(dpt[f], 8 * s);
+                const bf16x8 pa = pack8(st[f], 8 * s);
 #pragma unroll
-            for (int df = 0; df < 2; ++df) {
-                const bf16x8 b = frag_cols(tk, 16 * s, 32 * df, lane);
-                adq[df] = mfma(a, b, adq[df]);
-                abv[df] = mfma(pa, b, abv[df]);
+                for (int df = 0; df < ND; ++df) {
+                    const bf16x8 b = frag_cols<ND>(tk, 32 * f + 16 * s, 32 * df, lane);
+                    adq[df] = mfma(a, b, adq[df]);
+                    abv[df] = mfma(pa, b, abv[df]);
+                    if constexpr (!TAU) adq[df] = mfma(pack8_lo(dpt[f], 8 * s, a), b, adq[df]);
+                }
             }
         }
-        if (wave_max(pmax) >= kLoTau) {
+        if (TAU && wave_max(pmax) >= kLoTau) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < 2 * TF; ++s) {
                 const bf16x8 al = pack8_lo(dpt[s >> 1], 8 * (s & 1), pack8(dpt[s >> 1], 8 * (s & 1)));
 #pragma unroll
-                for (int df = 0; df < 2; ++df) adq[df] = mfma(al, frag_cols(tk, 16 * s, 32 * df, lane), adq[df]);
+                for (int df = 0; df < ND; ++df) adq[df] = mfma(al, frag_cols<ND>(tk, 16 * s, 32 * df, lane), adq[df]);
             }
         }
     }
@@ -958,22 +1199,26 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dq64_kernel(const bf16_t* __r
         const float c = __shfl(corr, rl, 64);
         const int row = qw0 + rl;
 #pragma unroll
-        for (int df = 0; df < 2; ++df)
-            if (row < p.t)
-                dq[qoff + (int64_t)row * p.ldq + 32 * df + (lane & 31)] =
-                    f32_to_bf16((adq[df][r] - c * abv[df][r]) * p.scale);
+        for (int df = 0; df < ND; ++df) {
+            const int d = 32 * df + (lane & 31);
+            if (row < p.t && d < dh)
+                dq[qoff + (int64_t)row * p.ldq + d] = f32_to_bf16((adq[df][r] - c * abv[df][r]) * p.scale);
+        }
     }
 }
 
-__global__ __launch_bounds__(64 * NW, 2) void attn_dkdv64_kernel(const bf16_t* __restrict__ q,
-                                                                   const bf16_t* __restrict__ k,
-                                                                   const bf16_t* __restrict__ v,
-                                                                   const bf16_t* __restrict__ dO,
-                                                                   const float* __restrict__ lse2,
-                                                                   const float* __restrict__ dsum,
-                                                                   bf16_t* __restrict__ dk, bf16_t* __restrict__ dv,
-                                                                   AttnParams p) {
-    constexpr int STAGE = 2 * TILE + 2 * TR * 4;   // q tile, dO tile, lse and D of its rows
+template <int ND, int TF, int RING, bool TAU>
+__global__ __launch_bounds__(64 * NW, ND == 4 ? 1 : 2) void attn_dkdv32_kernel(const bf16_t* __restrict__ q,
+                                                                 const bf16_t* __restrict__ k,
+                                                                 const bf16_t* __restrict__ v,
+                                                                 const bf16_t* __restrict__ dO,
+                                                                 const float* __restrict__ lse2,
+                                                                 const float* __restrict__ dsum,
+                                                                 bf16_t* __restrict__ dk, bf16_t* __restrict__ dv,
+                                                                 AttnParams p) {
+    // q tile, dO tile, lse and D of its rows (64 floats each)
+    constexpr int TR = 32 * TF, TILE = TR * 64 * ND, STAGE = 2 * TILE + 512;
+    constexpr int LOADS = 2 * (TR * 4 * ND / 64) / NW;   // per wave and stage, beside waves 0 and 1's statistics
     extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
     char NOTT_LDS* smem = (char NOTT_LDS*)smem_raw;
     const int bh = blockIdx.x;
@@ -985,64 +1230,61 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkdv64_kernel(const bf16_t* _
     const int64_t qoff = bh_off(bh, p.nh, p.sbq, p.shq), koff = bh_off(bh, p.nh, p.sbk, p.shk);
     const int64_t ooff = bh_off(bh, p.nh, p.sbo, p.sho);
     const float sl2 = p.scale * 1.4426950408889634f;
+    const int dh = TAU ? 32 * ND : p.dh;
     const float* lse_bh = lse2 + (int64_t)bh * p.t;   // lse·log2(e), written by the dq pass
     const float* d_bh = dsum + (int64_t)bh * p.t;
 
-    u32x4 kr[4], vr[4];
-    load_fixed(k + koff, my_k, p.s, p.ldk, lane, kr);
-    load_fixed(v + koff, my_k, p.s, p.ldk, lane, vr);
+    u32x4 kr[2 * ND], vr[2 * ND];
+    load_fixed<ND>(k + koff, my_k, p.s, dh, p.ldk, lane, kr);
+    load_fixed<ND>(v + koff, my_k, p.s, dh, p.ldk, lane, vr);
 
     const int qb0 = p.causal ? k0 / TR : 0;
-    const int nq = p.nqb - qb0;   // 64-query blocks
+    const int nq = (p.t + TR - 1) / TR - qb0;
     auto issue = [&](int i, int slot) {
         char NOTT_LDS* st = smem + slot * STAGE;
         const int q0 = (qb0 + i) * TR;
-        fill_tile(q + qoff, q0, p.t, p.ldq, st, wid, lane);
-        fill_tile(dO + ooff, q0, p.t, p.ldo, st + TILE, wid, lane);
-        if (wid < 2) {
-            const int row = q0 + lane < p.t ? q0 + lane : p.t - 1;
-            dma4((wid == 0 ? lse_bh : d_bh) + row, lds_addr(st + 2 * TILE) + 256 * wid);
-        }
+        fill_pair<ND, TR>(q + qoff, p.ldq, dO + ooff, p.ldo, q0, p.t, dh, st, wid, lane);
+        if (wid < 2) dma4((wid == 0 ? lse_bh : d_bh) + min(q0 + lane, p.t - 1), lds_addr(st + 2 * TILE) + 256 * wid);
     };
 #pragma unroll
     for (int i = 0; i < RING - 1; ++i)
         if (i < nq) issue(i, i);
 
-    f32x16 adk[2], adv[2];
+    f32x16 adk[ND], adv[ND];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < ND; ++f)
 #pragma unroll
         for (int e = 0; e < 16; ++e) adk[f][e] = adv[f][e] = 0.f;
     int slot = 0, next = RING - 1;
     for (int i = 0; i < nq; ++i) {
         // Waves 0 and 1 issue one more load per stage than 2 and 3; the count
         // of the latter is a safe bound for both.
-        if (i + RING - 2 < nq) wait_vm_lgkm0<(RING - 2) * 2 * (8 / NW)>();
+        if (i + RING - 2 < nq) wait_vm_lgkm0<(RING - 2) * LOADS>();
         else wait_vm_lgkm0<0>();
         barrier();
         if (i + RING - 1 < nq) issue(i + RING - 1, next);
         const char NOTT_LDS* tq = smem + slot * STAGE;
         const char NOTT_LDS* tdo = tq + TILE;
         const float NOTT_LDS* slse = reinterpret_cast<const float NOTT_LDS*>(tq + 2 * TILE);
-        const float NOTT_LDS* sd = slse + TR;
+        const float NOTT_LDS* sd = slse + 64;
         slot = slot + 1 == RING ? 0 : slot + 1;
         next = next + 1 == RING ? 0 : next + 1;
         const int q0 = (qb0 + i) * TR;
         if ((p.causal && kw0 > q0 + TR - 1) || kw0 >= p.s) continue;   // every query of the block masked
-        f32x16 sc[2], dp[2];
+        f32x16 sc[TF], dp[TF];
 #pragma unroll
-        for (int f = 0; f < 2; ++f) {
+        for (int f = 0; f < TF; ++f) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) sc[f][e] = dp[f][e] = 0.f;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                sc[f] = mfma(frag_rows(tq, 32 * f, s, lane), __builtin_bit_cast(bf16x8, kr[s]), sc[f]);
-                dp[f] = mfma(frag_rows(tdo, 32 * f, s, lane), __builtin_bit_cast(bf16x8, vr[s]), dp[f]);
+            for (int s = 0; s < 2 * ND; ++s) {
+                sc[f] = mfma(frag_rows<ND>(tq, 32 * f, s, lane), __builtin_bit_cast(bf16x8, kr[s]), sc[f]);
+                dp[f] = mfma(frag_rows<ND>(tdo, 32 * f, s, lane), __builtin_bit_cast(bf16x8, vr[s]), dp[f]);
             }
         }
         // exponent arguments (log2 domain; the ring holds lse·log2(e)) in place
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < TF; ++f)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const f32x4 l4 = *reinterpret_cast<const f32x4 NOTT_LDS*>(slse + 32 * f + 8 * j + 4 * h);
@@ -1051,12 +1293,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkdv64_kernel(const bf16_t* _
             }
         // Masking only on blocks that touch the diagonal or the end (a
         // wave-uniform test).  Element (f, 4j + e) is query q0 + 4h + c with
-        // c = 32f + 8j + e (0..59), kept iff lo <= c < hi.
+        // c = 32f + 8j + e, kept iff lo <= c < hi.
         if (!(q0 + TR <= p.t && kw0 + 32 <= p.s && (!p.causal || kw0 + 31 <= q0))) {
             const int hi = my_k < p.s ? p.t - q0 - 4 * h : -1;
             const int lo = p.causal ? my_k - q0 - 4 * h : 0;
 #pragma unroll
-            for (int f = 0; f < 2; ++f)
+            for (int f = 0; f < TF; ++f)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -1067,7 +1309,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkdv64_kernel(const bf16_t* _
         }
         float pmax = 0.f;
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < TF; ++f) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const f32x4 d4 = *reinterpret_cast<const f32x4 NOTT_LDS*>(sd + 32 * f + 8 * j + 4 * h);
@@ -1075,53 +1317,57 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_dkdv64_kernel(const bf16_t* _
                 for (int e = 0; e < 4; ++e) {
                     const int r = 4 * j + e;
                     const float pe = __builtin_amdgcn_exp2f(sc[f][r]);
-                    pmax = fmaxf(pmax, pe);
+                    if (TAU) pmax = fmaxf(pmax, pe);
                     sc[f][r] = pe;
                     dp[f][r] = pe * (dp[f][r] - d4[e]);
                 }
             }
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const bf16x8 pa = pack8(sc[s >> 1], 8 * (s & 1));
-            const bf16x8 da = pack8(dp[s >> 1], 8 * (s & 1));
+            for (int s = 0; s < 2; ++s) {
+                const bf16x8 pa = pack8(sc[f], 8 * s);
+                const bf16x8 da = pack8(dp[f], 8 * s);
 #pragma unroll
-            for (int df = 0; df < 2; ++df) {
-                adv[df] = mfma(pa, frag_cols(tdo, 16 * s, 32 * df, lane), adv[df]);
-                adk[df] = mfma(da, frag_cols(tq, 16 * s, 32 * df, lane), adk[df]);
+                for (int df = 0; df < ND; ++df) {
+                    const bf16x8 bo = frag_cols<ND>(tdo, 32 * f + 16 * s, 32 * df, lane);
+                    const bf16x8 bq = frag_cols<ND>(tq, 32 * f + 16 * s, 32 * df, lane);
+                    adv[df] = mfma(pa, bo, adv[df]);
+                    adk[df] = mfma(da, bq, adk[df]);
+                    if constexpr (!TAU) {
+                        adv[df] = mfma(pack8_lo(sc[f], 8 * s, pa), bo, adv[df]);
+                        adk[df] = mfma(pack8_lo(dp[f], 8 * s, da), bq, adk[df]);
+                    }
+                }
             }
         }
-        if (wave_max(pmax) >= kLoTau) {
+        if (TAU && wave_max(pmax) >= kLoTau) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < 2 * TF; ++s) {
                 const bf16x8 pl = pack8_lo(sc[s >> 1], 8 * (s & 1), pack8(sc[s >> 1], 8 * (s & 1)));
                 const bf16x8 dl = pack8_lo(dp[s >> 1], 8 * (s & 1), pack8(dp[s >> 1], 8 * (s & 1)));
 #pragma unroll
-                for (int df = 0; df < 2; ++df) {
-                    adv[df] = mfma(pl, frag_cols(tdo, 16 * s, 32 * df, lane), adv[df]);
-                    adk[df] = mfma(dl, frag_cols(tq, 16 * s, 32 * df, lane), adk[df]);
+                for (int df = 0; df < ND; ++df) {
+                    adv[df] = mfma(pl, frag_cols<ND>(tdo, 16 * s, 32 * df, lane), adv[df]);
+                    adk[df] = mfma(dl, frag_cols<ND>(tq, 16 * s, 32 * df, lane), adk[df]);
                 }
             }
         }
     }
 #pragma unroll
-    for (int df = 0; df < 2; ++df)
+    for (int df = 0; df < ND; ++df)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int key = kw0 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (key < p.s) {
-                const int64_t i = koff + (int64_t)key * p.ldk + 32 * df + (lane & 31);
+            const int key = kw0 + 8 * (r >> 2) + 4 * h + (r & 3), d = 32 * df + (lane & 31);
+            if (key < p.s && d < dh) {
+                const int64_t i = koff + (int64_t)key * p.ldk + d;
                 dk[i] = f32_to_bf16(adk[df][r] * p.scale);
                 dv[i] = f32_to_bf16(adv[df][r]);
             }
         }
 }
 
-// Whether the head-dim-64 kernels take this problem: bf16, dh = 64, 16-byte
-// aligned rows (the fills move 16-byte chunks).
-bool applies(const nott_attn_desc* d, const AttnParams& p, int elem) { return elem == 2 && d->dh == 64 && p.vec; }
-
-int bwd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* q, const void* k, const void* v,
-        const void* o, const void* dO, const float* lse, void* dq, void* dk, void* dv) {
+template <int ND, int TF, int RING, bool TAU>
+int bwd_nd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* q, const void* k, const void* v,
+           const void* o, const void* dO, const float* lse, void* dq, void* dk, void* dv) {
     const int64_t rows = d->b * d->h * d->t;
     // dsum (the exact rowsum(P∘dP)) and lse2 (lse·log2 e), both [b, h, t],
     // handed from the dq pass to the dk/dv pass
@@ -1129,27 +1375,38 @@ int bwd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* 
     if (!dsum) return NOTT_ERR_ALLOC;
     float* lse2 = dsum + std::max<int64_t>(rows, 1);
     const unsigned bh = (unsigned)(d->b * d->h);
-    const size_t lds_q = RING * 2 * TILE, lds_kv = RING * (2 * TILE + 2 * TR * 4);
+    constexpr size_t lds_q = (size_t)RING * 2 * (32 * TF) * 64 * ND, lds_kv = lds_q + RING * 512;
+    auto fq = &attn_dq32_kernel<ND, TF, RING, TAU>;
+    auto fkv = &attn_dkdv32_kernel<ND, TF, RING, TAU>;
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_dq64_kernel),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_q);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_dkdv64_kernel),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fq), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds_q);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fkv), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds_kv);
         attr = true;
     }
     const auto* qb = static_cast<const bf16_t*>(q);
     const auto* kb = static_cast<const bf16_t*>(k);
     const auto* vb = static_cast<const bf16_t*>(v);
     const auto* dob = static_cast<const bf16_t*>(dO);
-    hipLaunchKernelGGL(attn_dq64_kernel, dim3(bh, (unsigned)ceil_div(d->t, FIXED)), dim3(64 * NW), lds_q, ctx->stream,
-                       qb, kb, vb, static_cast<const bf16_t*>(o), dob, lse, dsum, lse2, static_cast<bf16_t*>(dq), p);
-    hipLaunchKernelGGL(attn_dkdv64_kernel, dim3(bh, (unsigned)ceil_div(d->s, FIXED)), dim3(64 * NW), lds_kv,
-                       ctx->stream, qb, kb, vb, dob, lse2, dsum, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), p);
+    hipLaunchKernelGGL(fq, dim3(bh, (unsigned)ceil_div(d->t, FIXED)), dim3(64 * NW), lds_q, ctx->stream, qb, kb, vb,
+                       static_cast<const bf16_t*>(o), dob, lse, dsum, lse2, static_cast<bf16_t*>(dq), p);
+    hipLaunchKernelGGL(fkv, dim3(bh, (unsigned)ceil_div(d->s, FIXED)), dim3(64 * NW), lds_kv, ctx->stream, qb, kb, vb,
+                       dob, lse2, dsum, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), p);
     return launch_status(ctx, "attention_bwd");
 }
 
-}  // namespace a64
+int bwd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* q, const void* k, const void* v,
+        const void* o, const void* dO, const float* lse, void* dq, void* dk, void* dv) {
+    if (d->dh <= 32) return bwd_nd<1, 2, 4, false>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+    if (d->dh == 64) return bwd_nd<2, 2, 4, true>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+    if (d->dh < 64) return bwd_nd<2, 2, 4, false>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+    if (d->dh <= 96) return bwd_nd<3, 1, 4, false>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+    return bwd_nd<4, 2, 2, false>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+}
+
+}  // namespace fa
 
 int check(nott_ctx ctx, const nott_attn_desc* d, AttnParams* p, int elem) {
     NOTT_REQUIRE(ctx, d != nullptr, "attention: null descriptor");
@@ -1308,6 +1565,8 @@ extern "C" int nott_attention_fwd(nott_ctx ctx, const nott_attn_desc* d, nott_dt
     NOTT_REQUIRE(ctx, q && k && v && o && lse, "nott_attention_fwd: null buffer");
     if (!(aligned16(q) && aligned16(k) && aligned16(v))) p.vec = 0;
     nott::DeviceScope scope(ctx->device);
+    if (d->s > 0 && aligned16(o) && fa::applies(p, (int)nott::dtype_size(dtype)))
+        return fa::fwd(ctx, d, p, q, k, v, o, lse);
     return dtype == NOTT_F32 ? fwd<float>(ctx, d, p, q, k, v, o, lse) : fwd<bf16_t>(ctx, d, p, q, k, v, o, lse);
 }
 
@@ -1333,7 +1592,7 @@ extern "C" int nott_attention_bwd(nott_ctx ctx, const nott_attn_desc* d, nott_dt
     NOTT_REQUIRE(ctx, q && k && v && o && dO && lse && dq && dk && dv, "nott_attention_bwd: null buffer");
     if (!(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(dO) && aligned16(o))) p.vec = 0;
     nott::DeviceScope scope(ctx->device);
-    if (a64::applies(d, p, (int)nott::dtype_size(dtype))) return a64::bwd(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+    if (fa::applies(p, (int)nott::dtype_size(dtype))) return fa::bwd(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
     return dtype == NOTT_F32 ? bwd<float>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv)
                              : bwd<bf16_t>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
 }
