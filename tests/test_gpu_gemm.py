@@ -265,6 +265,62 @@ def test_conv_nhwc(ops, oracle, dt, case):
     check(host(db), rdb, dt, "nhwc db")
 
 
+# n, c, h, w, k, (r, s), (stride), (pad), (dilation): bf16 convolutions that run
+# as implicit GEMMs over a channels-last copy.  A single output pixel, k = 8, a
+# K that is not whole 64s, images of 1 row under stride 2 (a parity class and
+# taps that no pixel takes), classes without taps (1×1 stride 2), strides above 2
+# (the data gradient stays on the general path), different strides per axis,
+# 25 taps, tiles on both sides of 64 and 128 rows and columns, rows over 64 wide.
+CONV_ROWS = [
+    (1, 8, 3, 3, 8, (3, 3), (1, 1), (0, 0), (1, 1)),
+    (2, 24, 9, 7, 40, (3, 3), (2, 2), (1, 1), (1, 1)),
+    (1, 16, 1, 130, 72, (3, 3), (2, 2), (1, 1), (1, 1)),
+    (3, 64, 8, 8, 64, (1, 1), (2, 2), (0, 0), (1, 1)),
+    (3, 72, 7, 9, 136, (1, 1), (1, 1), (0, 0), (1, 1)),
+    (2, 8, 11, 13, 16, (5, 5), (1, 1), (2, 2), (1, 1)),
+    (1, 32, 17, 10, 128, (3, 3), (3, 1), (2, 0), (1, 2)),
+    (2, 40, 12, 11, 56, (4, 2), (1, 2), (3, 1), (2, 1)),
+    (2, 64, 14, 14, 192, (3, 3), (2, 2), (1, 1), (1, 1)),
+]
+
+
+@pytest.mark.parametrize("case", CONV_ROWS, ids=[f"{c[1]}x{c[2]}x{c[3]}-{c[4]}-r{c[5][0]}{c[5][1]}s{c[6][0]}{c[6][1]}"
+                                                 for c in CONV_ROWS])
+def test_conv_channels_last_gemm(ops, oracle, case):
+    """Products of bf16 values are exact in fp32, so a sum of n terms is off by
+    at most n·2^-23·Σ|terms| (truncating adds); a bf16 result by 2^-8 of itself
+    on top.  Operands one element past a 16-byte boundary must do as well."""
+    n, c, h, w_, k, (r, s), st, pad, dil = case
+    d = ops.conv_desc((n, c, h, w_), (k, c, r, s), stride=st, padding=pad, dilation=dil)
+    p, q = conv_out(h, r, st[0], pad[0], dil[0]), conv_out(w_, s, st[1], pad[1], dil[1])
+    g = rng(77)
+    x, w, dy = (host_input(f32(g.standard_normal(v)), "bf16") for v in ((n, c, h, w_), (k, c, r, s), (n, k, p, q)))
+    b = f32(g.standard_normal(k))
+
+    def near(got, want, mag, terms, rel, what):
+        err = np.abs(host(got).astype(np.float64) - want) - (terms * 2.0 ** -23 * mag + rel * np.abs(want))
+        assert err.max() <= 0, f"{what}: over the bound by {err.max():.3g}"
+
+    def shifted(a):
+        t = torch.empty(a.size + 1, dtype=torch.bfloat16, device="cuda")[1:].view(a.shape)
+        return t.copy_(dev(a, "bf16"))
+
+    y_ref, y_mag = oracle.conv2d_fwd(d, x, w, b), oracle.conv2d_fwd(d, abs(x), abs(w), abs(b))
+    dx_ref, dx_mag = oracle.conv2d_bwd_data(d, dy, w), oracle.conv2d_bwd_data(d, abs(dy), abs(w))
+    dw_ref, dw_mag = oracle.conv2d_bwd_weight(d, x, dy)[0], oracle.conv2d_bwd_weight(d, abs(x), abs(dy))[0]
+    for put in (lambda a: dev(a, "bf16"), shifted):
+        X, Wt, DY = put(x), put(w), put(dy)
+        for relu in (False, True):
+            y = ops.conv2d_fwd(X, Wt, dev(b), d, relu=relu)
+            near(y, np.maximum(y_ref, 0) if relu else y_ref, y_mag, c * r * s + 1, 2.0 ** -8, "y")
+        near(ops.conv2d_bwd_data(DY, Wt, d), dx_ref, dx_mag, k * r * s, 2.0 ** -8, "dx")
+        dw, _ = ops.conv2d_bwd_weight(X, DY, d)
+        near(dw, dw_ref, dw_mag, n * p * q, 0.0, "dw")
+        again = dw.clone()
+        ops.conv2d_bwd_weight(X, DY, d, dw=again, accumulate=True)
+        assert torch.equal(again, dw + dw)
+
+
 @pytest.mark.parametrize("name", ["conv3x3_s1p1_bias", "conv3x3_s2p1", "conv7x7_s2p3", "conv1x1_s2",
                                   "conv3x3_dil2_rect"])
 def test_conv_golden(ops, name):

@@ -749,6 +749,13 @@ int fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const voi
     if (nott::conv_fast::stem_fwd_applies(ctx, d))
         return nott::conv_fast::stem_fwd<T>(ctx, d, static_cast<const T*>(x), static_cast<const T*>(w), b,
                                             static_cast<T*>(y), relu);
+    if constexpr (sizeof(T) == 2) {
+        if (nott::conv_fast::rows_fwd_applies(ctx, d)) {
+            const int st = nott::conv_fast::rows_fwd(ctx, d, p, q, static_cast<const T*>(x), static_cast<const T*>(w),
+                                                     b, static_cast<T*>(y), relu);
+            if (st != NOTT_ERR_ALLOC) return st;   // no room for the channels-last copy: the paths below
+        }
+    }
     if (nott::conv_fast::tap_fwd_applies(ctx, d, sizeof(T)))
         return nott::conv_fast::tap_fwd<T>(ctx, d, static_cast<const T*>(x), static_cast<const T*>(w), b,
                                            static_cast<T*>(y), relu);
@@ -761,6 +768,13 @@ template <typename T>
 int dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const void* dy, const void* w, void* dx) {
     if (nott::conv_fast::dgrad_applies(d, sizeof(T)))
         return nott::conv_fast::dgrad<T>(ctx, d, static_cast<const T*>(dy), static_cast<const T*>(w), static_cast<T*>(dx));
+    if constexpr (sizeof(T) == 2) {
+        if (nott::conv_fast::rows_dgrad_applies(ctx, d, p, q)) {
+            const int st = nott::conv_fast::rows_dgrad(ctx, d, p, q, static_cast<const T*>(dy),
+                                                       static_cast<const T*>(w), static_cast<T*>(dx));
+            if (st != NOTT_ERR_ALLOC) return st;
+        }
+    }
     if (nott::conv_fast::tap_dgrad_applies(ctx, d, sizeof(T)))
         return nott::conv_fast::tap_dgrad<T>(ctx, d, static_cast<const T*>(dy), static_cast<const T*>(w),
                                              static_cast<T*>(dx));
@@ -792,6 +806,9 @@ int wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const v
             // the bias gradient comes out of the same pass
             st = cin1_wgrad<T>(ctx, d, static_cast<const T*>(x), static_cast<const T*>(dy), dw, db, accumulate);
             db = nullptr;
+        } else if (sizeof(T) == 2 && nott::conv_fast::rows_wgrad_applies(ctx, d)) {
+            st = nott::conv_fast::rows_wgrad(ctx, d, p, q, reinterpret_cast<const bf16_t*>(x),
+                                             reinterpret_cast<const bf16_t*>(dy), dw, accumulate);
         } else if (sizeof(T) == 2 && col_applies(d, p, q, false)) {
             st = col_wgrad(ctx, d, p, q, reinterpret_cast<const bf16_t*>(x), reinterpret_cast<const bf16_t*>(dy), dw,
                            accumulate);
