@@ -281,6 +281,7 @@ CONV_ROWS = [
     (1, 32, 17, 10, 128, (3, 3), (3, 1), (2, 0), (1, 2)),
     (2, 40, 12, 11, 56, (4, 2), (1, 2), (3, 1), (2, 1)),
     (2, 64, 14, 14, 192, (3, 3), (2, 2), (1, 1), (1, 1)),
+    (2, 12, 9, 10, 20, (3, 3), (2, 2), (1, 1), (1, 1)),   # whole 4s: fp32 weight gradient only
 ]
 
 
@@ -308,6 +309,8 @@ def test_conv_channels_last_gemm(ops, oracle, case):
     y_ref, y_mag = oracle.conv2d_fwd(d, x, w, b), oracle.conv2d_fwd(d, abs(x), abs(w), abs(b))
     dx_ref, dx_mag = oracle.conv2d_bwd_data(d, dy, w), oracle.conv2d_bwd_data(d, abs(dy), abs(w))
     dw_ref, dw_mag = oracle.conv2d_bwd_weight(d, x, dy)[0], oracle.conv2d_bwd_weight(d, abs(x), abs(dy))[0]
+    dw, _ = ops.conv2d_bwd_weight(dev(x), dev(dy), d)   # the same products in fp32 tiles
+    near(dw, dw_ref, dw_mag, n * p * q, 0.0, "dw f32")
     for put in (lambda a: dev(a, "bf16"), shifted):
         X, Wt, DY = put(x), put(w), put(dy)
         for relu in (False, True):

@@ -806,9 +806,9 @@ int wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const v
             // the bias gradient comes out of the same pass
             st = cin1_wgrad<T>(ctx, d, static_cast<const T*>(x), static_cast<const T*>(dy), dw, db, accumulate);
             db = nullptr;
-        } else if (sizeof(T) == 2 && nott::conv_fast::rows_wgrad_applies(ctx, d)) {
-            st = nott::conv_fast::rows_wgrad(ctx, d, p, q, reinterpret_cast<const bf16_t*>(x),
-                                             reinterpret_cast<const bf16_t*>(dy), dw, accumulate);
+        } else if (nott::conv_fast::rows_wgrad_applies(ctx, d, sizeof(T))) {
+            st = nott::conv_fast::rows_wgrad<T>(ctx, d, p, q, static_cast<const T*>(x), static_cast<const T*>(dy), dw,
+                                                accumulate);
         } else if (sizeof(T) == 2 && col_applies(d, p, q, false)) {
             st = col_wgrad(ctx, d, p, q, reinterpret_cast<const bf16_t*>(x), reinterpret_cast<const bf16_t*>(dy), dw,
                            accumulate);

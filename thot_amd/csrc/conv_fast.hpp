@@ -34,17 +34,18 @@ int tap_fwd(nott_ctx ctx, const nott_conv2d_desc* d, const T* x, const T* w, con
 template <typename T>
 int tap_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, const T* dy, const T* w, T* dx);
 
-// bf16 implicit GEMMs over a channels-last copy, for the shapes without a kernel
+// Implicit GEMMs over a channels-last copy (the weight gradient in both types, the rest bf16), for the shapes without a kernel
 // of their own (conv_gemm.hip; NOTT_CONV_TAP=0 switches them off as well).
 bool rows_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d);
 bool rows_dgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q);
-bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d);
+bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, size_t elem);
 int rows_fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* x, const bf16_t* w,
              const float* b, bf16_t* y, int relu);
 int rows_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* dy, const bf16_t* w,
                bf16_t* dx);
-int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* x, const bf16_t* dy,
-               float* dw, int accumulate);
+template <typename T>
+int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const T* x, const T* dy, float* dw,
+               int accumulate);
 
 // Forward of the 3-channel 7x7 column-stride-2 stem (conv_stem.hip).
 bool stem_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d);

@@ -51,17 +51,17 @@ constexpr int BM = 128;
 // ------------------------------------------------------------------- prep
 // One tensor: xp[n][hp][wp][c] from x[n][c][h][w], position (i, j) holding pixel
 // (i·sh − pt, j·sw − pl) or zeros.
-struct PrepPart {
-    const bf16_t* x;
-    bf16_t* xp;
+template <typename T> struct PrepPart {
+    const T* x;
+    T* xp;
     int32_t c, h, w, pt, pl, sh, sw, cblocks, npos;
     FastDiv fij, fj, fcb;    // by hp·wp, wp and cblocks
 };
-struct PrepParams {
-    PrepPart part[2];        // the second may be empty (blocks[1] = blocks[0])
+template <typename T> struct PrepParams {
+    PrepPart<T> part[2];        // the second may be empty (blocks[1] = blocks[0])
     int32_t blocks[2];       // first block after each part
-    const bf16_t* wt;        // [k][cin][taps]
-    bf16_t* wp2;
+    const T* wt;        // [k][cin][taps]
+    T* wp2;
     int32_t k, cin, taps, by_cin;   // by_cin: rows are input channels (data gradient), columns output channels
     int32_t base[kMaxTaps], nt[kMaxTaps], t[kMaxTaps];   // by_cin, of a tap: its matrix, that matrix's taps, its place
 };
@@ -71,8 +71,9 @@ struct PrepParams {
 // counted through all rows and images, so that narrow images fill the lanes
 // too.  The blocks after the parts lay out the weights.  Bound by memory: the
 // 128 MB of x and dy of [64, 64, 56, 56] → 256, 1×1, take 46 µs, 5.5 TB/s.
-__global__ __launch_bounds__(256) void nhwc_prep_kernel(PrepParams p) {
-    __shared__ bf16_t tile[64][66];
+template <typename T> __global__ __launch_bounds__(256) void nhwc_prep_kernel(PrepParams<T> p) {
+    constexpr int E = 16 / sizeof(T), CH = 64 / E;   // elements of a chunk, chunks of 64 channels
+    __shared__ T tile[64][sizeof(T) == 2 ? 66 : 65];
     const int tid = threadIdx.x, b = (int)blockIdx.x;
     if (b >= p.blocks[1] && !p.by_cin) {
         // destination order: [row][tap][channel], a row's channels side by side
@@ -87,31 +88,31 @@ __global__ __launch_bounds__(256) void nhwc_prep_kernel(PrepParams p) {
         // [k][cin·taps] turned: 64 output channels × 64 (input channel, tap)
         const int32_t kb = (p.k + 63) / 64, ct = p.cin * p.taps, wb = b - p.blocks[1];
         const int32_t k0 = wb % kb * 64, j0 = wb / kb * 64, nk = min(64, p.k - k0), nj = min(64, ct - j0);
-        bf16_t v[16];
+        T v[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
             const int c = u * 4 + (tid >> 6);
-            v[u] = (tid & 63) < nj && c < nk ? p.wt[(int64_t)(k0 + c) * ct + j0 + (tid & 63)] : (bf16_t)0;
+            v[u] = (tid & 63) < nj && c < nk ? p.wt[(int64_t)(k0 + c) * ct + j0 + (tid & 63)] : T(0);
         }
 #pragma unroll
         for (int u = 0; u < 16; ++u) tile[u * 4 + (tid >> 6)][tid & 63] = v[u];
         __syncthreads();
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int n = u * 256 + tid, ch = n & 7, at = n >> 3;
-            if (at >= nj || ch * 8 >= nk) continue;
+        for (int u = 0; u < CH / 4; ++u) {
+            const int n = u * 256 + tid, ch = n % CH, at = n / CH;
+            if (at >= nj || ch * E >= nk) continue;
             const int32_t ci = (j0 + at) / p.taps, tap = j0 + at - ci * p.taps;
             if (!p.nt[tap]) continue;   // a tap that only pixels past the edge would take
-            bf16_t e[8];
+            T e[E];
 #pragma unroll
-            for (int z = 0; z < 8; ++z) e[z] = tile[ch * 8 + z][at];
-            *reinterpret_cast<u32x4*>(p.wp2 + p.base[tap] + (int64_t)(ci * p.nt[tap] + p.t[tap]) * p.k + k0 + ch * 8) =
-                gemm::Pack<bf16_t>::make(e);
+            for (int z = 0; z < E; ++z) e[z] = tile[ch * E + z][at];
+            *reinterpret_cast<u32x4*>(p.wp2 + p.base[tap] + (int64_t)(ci * p.nt[tap] + p.t[tap]) * p.k + k0 + ch * E) =
+                gemm::Pack<T>::make(e);
         }
         return;
     }
     const int second = b >= p.blocks[0];
-    const PrepPart& q = p.part[second];
+    const PrepPart<T>& q = p.part[second];
     uint32_t pb, cb, img, rest, i, j;
     q.fcb.divmod((uint32_t)(b - (second ? p.blocks[0] : 0)), pb, cb);
     const int32_t c0 = (int32_t)cb * 64, nc = min(64, q.c - c0), pos0 = (int32_t)pb * 64;
@@ -120,24 +121,24 @@ __global__ __launch_bounds__(256) void nhwc_prep_kernel(PrepParams p) {
     q.fj.divmod(rest, i, j);
     const int32_t hh = (int32_t)i * q.sh - q.pt, ww = (int32_t)j * q.sw - q.pl, hw = q.h * q.w;
     const bool in = hh >= 0 && hh < q.h && ww >= 0 && ww < q.w;
-    const bf16_t* src = q.x + ((int64_t)img * q.c + c0) * hw + (in ? hh * q.w + ww : 0);
-    bf16_t v[16];
+    const T* src = q.x + ((int64_t)img * q.c + c0) * hw + (in ? hh * q.w + ww : 0);
+    T v[16];
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
         const int c = u * 4 + (tid >> 6);
-        v[u] = in && c < nc ? src[(int64_t)c * hw] : (bf16_t)0;
+        v[u] = in && c < nc ? src[(int64_t)c * hw] : T(0);
     }
 #pragma unroll
     for (int u = 0; u < 16; ++u) tile[u * 4 + (tid >> 6)][tid & 63] = v[u];
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int n = u * 256 + tid, ch = n & 7, at = n >> 3;
-        if (pos0 + at >= q.npos || ch * 8 >= nc) continue;
-        bf16_t e[8];
+    for (int u = 0; u < CH / 4; ++u) {
+        const int n = u * 256 + tid, ch = n % CH, at = n / CH;
+        if (pos0 + at >= q.npos || ch * E >= nc) continue;
+        T e[E];
 #pragma unroll
-        for (int z = 0; z < 8; ++z) e[z] = tile[ch * 8 + z][at];
-        *reinterpret_cast<u32x4*>(q.xp + (int64_t)(pos0 + at) * q.c + c0 + ch * 8) = gemm::Pack<bf16_t>::make(e);
+        for (int z = 0; z < E; ++z) e[z] = tile[ch * E + z][at];
+        *reinterpret_cast<u32x4*>(q.xp + (int64_t)(pos0 + at) * q.c + c0 + ch * E) = gemm::Pack<T>::make(e);
     }
 }
 
@@ -344,8 +345,8 @@ __global__ __launch_bounds__(64 * NW) void conv_rows_kernel(RowParams p) {
 }
 
 // ---------------------------------------------------------- weight gradient
-struct WgradParams {
-    const bf16_t *dyt, *xp;   // [pixel][k], [n][hp][wp][c]
+template <typename T> struct WgradParams {
+    const T *dyt, *xp;   // [pixel][k], [n][hp][wp][c]
     int32_t M, N, K, kps, splits;   // M = k, N = taps · C, K = pixels
     FastDiv fij, fj, fc;
     int32_t sn, si, sj;
@@ -354,8 +355,37 @@ struct WgradParams {
 };
 constexpr int kMaxPixels = 14336;   // of a split: their offsets sit in LDS beside the ring
 
-__global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams p) {
+// The operand slices of one wave: 16 k of the stage's 64 (bf16), 8 of its 32
+// (fp32), for two 32-row fragments.
+template <typename T> struct Slices;
+template <> struct Slices<bf16_t> {
+    static constexpr int kStageK = 64;
+    FragAddr<true, 128, 2> at;
+    Frag<true> f[2][2];
+    __device__ __forceinline__ void init(int row0, int lane) { at.init(row0, lane); }
+    template <int SL> __device__ __forceinline__ void read(const char NOTT_LDS* tile) { read_all<SL>(f[SL & 1], at, tile); }
+};
+// fp32 tiles are [k][128 rows]; odd k hold their rows with bit 5 flipped, so
+// that the two halves of a wave (k and k + 1) read different banks.
+template <> struct Slices<float> {
+    static constexpr int kStageK = 32;
+    int at[2];
+    float f[2][2][4];
+    __device__ __forceinline__ void init(int row0, int lane) {
+        for (int i = 0; i < 2; ++i) at[i] = (lane >> 5) * 512 + 4 * ((row0 + 32 * i + (lane & 31)) ^ (lane & 32));
+    }
+    template <int SL> __device__ __forceinline__ void read(const char NOTT_LDS* tile) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                f[SL & 1][i][e] = *reinterpret_cast<const float NOTT_LDS*>(tile + at[i] + (SL * 4 + e) * 1024);
+    }
+};
+
+template <typename T> __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams<T> p) {
     constexpr int BN = 128, FM = 2, FN = 2, TILE = 128 * 128, STAGE = 2 * TILE, LOADS = 2 * 16 / NW;
+    constexpr int BK = Slices<T>::kStageK, E = 16 / sizeof(T), KPB = 1024 / (128 * (int)sizeof(T));   // k of a 1 KB block
     extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
     char NOTT_LDS* smem = (char NOTT_LDS*)smem_raw;
     int32_t NOTT_LDS* lpix = (int32_t NOTT_LDS*)(smem + S * STAGE);
@@ -371,10 +401,12 @@ __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams p)
         p.fj.divmod(rest, y, x);
         lpix[i] = (int32_t)img * p.sn + (int32_t)y * p.si + (int32_t)x * p.sj;
     }
-    // This lane's 8 columns of every B fill, (tap, channels), and its pixel in
-    // each 4-pixel block.
-    const int pix = lane >> 4;
-    const uint32_t col = (uint32_t)min(n0 + 8 * ((lane & 15) ^ (pix << 2)), p.N - 8);
+    // This lane's 16 bytes of columns of every fill (for B a tap and channels),
+    // and its pixel in each 1 KB block.
+    const int pix = lane / (128 / E);
+    const int crow = E * ((lane % (128 / E)) ^ (E == 8 ? pix << 2 : pix << 3));   // its columns within the tile
+    const uint32_t col = (uint32_t)min(n0 + crow, p.N - E);
+    const int64_t arow = min(m0 + crow, p.M - E);
     uint32_t tap, c;
     p.fc.divmod(col, tap, c);
     int32_t toff = (int32_t)c;
@@ -384,21 +416,13 @@ __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams p)
     auto issue = [&](int t, int slot) {
         char NOTT_LDS* st = smem + slot * STAGE;
         const int32_t k0 = kb + t * BK;
-        if (k0 + BK <= p.K) {
-#pragma unroll
-            for (int i = 0; i < 16 / NW; ++i)
-                fill_block<true, BM, NW, false>(i, p.dyt, p.M, m0, p.M, k0, p.K, st, wid, lane);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16 / NW; ++i)
-                fill_block<true, BM, NW, true>(i, p.dyt, p.M, m0, p.M, k0, p.K, st, wid, lane);
-        }
 #pragma unroll
         for (int i = 0; i < 16 / NW; ++i) {
-            const int k = 4 * (i * NW + wid) + pix;
-            const int32_t o = lpix[t * BK + k] + toff;
-            dma16(k0 + k < p.K ? p.xp + o : reinterpret_cast<const bf16_t*>(&zero_chunk),
-                  lds_addr(st + TILE) + 1024 * (i * NW + wid));
+            const int k = KPB * (i * NW + wid) + pix;
+            const bool in = k0 + k < p.K;
+            const T* zero = reinterpret_cast<const T*>(&zero_chunk);
+            dma16(in ? p.dyt + ((int64_t)(k0 + k) * p.M + arow) : zero, lds_addr(st) + 1024 * (i * NW + wid));
+            dma16(in ? p.xp + (lpix[t * BK + k] + toff) : zero, lds_addr(st + TILE) + 1024 * (i * NW + wid));
         }
     };
     f32x16 acc[FM][FN];
@@ -408,18 +432,24 @@ __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams p)
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    FragAddr<true, BM, FM> fa;
-    FragAddr<true, BN, FN> fb;
-    fa.init(wm * 64, lane);
-    fb.init(wn * 64, lane);
-    Frag<true> a[2][FM], b[2][FN];
+    Slices<T> a, b;
+    a.init(wm * 64, lane);
+    b.init(wn * 64, lane);
     auto mma = [&](int s) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                acc[i][j] =
-                    __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][i].get(), b[s][j].get(), acc[i][j], 0, 0, 0);
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (sizeof(T) == 2) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.f[s][i].get(), b.f[s][j].get(), acc[i][j], 0,
+                                                                        0, 0);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i][j] =
+                            __builtin_amdgcn_mfma_f32_32x32x2f32(a.f[s][i][e], b.f[s][j][e], acc[i][j], 0, 0, 0);
+                }
+            }
     };
 #pragma unroll
     for (int s = 0; s < S - 1; ++s)
@@ -428,23 +458,23 @@ __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams p)
         if (nk >= S - 1) wait_vm_lgkm0<(S - 2) * LOADS>();
         else wait_vm_lgkm0<0>();
         barrier();
-        read_all<0>(a[0], fa, smem);
-        read_all<0>(b[0], fb, smem + TILE);
+        a.template read<0>(smem);
+        b.template read<0>(smem + TILE);
     }
     int slot = 0, free = S - 1;
     for (int t = 0; t < nk; ++t) {
         const char NOTT_LDS* sa = smem + slot * STAGE;
         const char NOTT_LDS* sb = sa + TILE;
         const bool more = t + S - 1 < nk;
-        read_all<1>(a[1], fa, sa);
-        read_all<1>(b[1], fb, sb);
+        a.template read<1>(sa);
+        b.template read<1>(sb);
         if (more) issue(t + S - 1, free);
         mma(0);
-        read_all<2>(a[0], fa, sa);
-        read_all<2>(b[0], fb, sb);
+        a.template read<2>(sa);
+        b.template read<2>(sb);
         mma(1);
-        read_all<3>(a[1], fa, sa);
-        read_all<3>(b[1], fb, sb);
+        a.template read<3>(sa);
+        b.template read<3>(sb);
         mma(0);
         const int nslot = slot + 1 == S ? 0 : slot + 1;
         if (t + 1 < nk) {
@@ -452,8 +482,8 @@ __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows_kernel(WgradParams p)
             else wait_vm_lgkm0<0>();
             barrier();
             const char NOTT_LDS* na = smem + nslot * STAGE;
-            read_all<0>(a[0], fa, na);
-            read_all<0>(b[0], fb, na + TILE);
+            a.template read<0>(na);
+            b.template read<0>(na + TILE);
         }
         mma(1);
         free = slot;
@@ -489,9 +519,10 @@ struct TapMajorStore {
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-PrepPart part_of(const bf16_t* x, bf16_t* xp, int64_t n, int64_t c, int64_t h, int64_t w, int64_t hp, int64_t wp,
-                 int64_t pt, int64_t pl, int64_t sh = 1, int64_t sw = 1) {
-    PrepPart p{};
+template <typename T>
+PrepPart<T> part_of(const T* x, T* xp, int64_t n, int64_t c, int64_t h, int64_t w, int64_t hp, int64_t wp, int64_t pt,
+                    int64_t pl, int64_t sh = 1, int64_t sw = 1) {
+    PrepPart<T> p{};
     p.x = x; p.xp = xp;
     p.c = (int32_t)c; p.h = (int32_t)h; p.w = (int32_t)w;
     p.pt = (int32_t)pt; p.pl = (int32_t)pl; p.sh = (int32_t)sh; p.sw = (int32_t)sw;
@@ -501,7 +532,7 @@ PrepPart part_of(const bf16_t* x, bf16_t* xp, int64_t n, int64_t c, int64_t h, i
     return p;
 }
 
-int launch_prep(nott_ctx ctx, PrepParams& p) {
+template <typename T> int launch_prep(nott_ctx ctx, PrepParams<T>& p) {
     int64_t blocks = 0;
     for (int i = 0; i < 2; ++i) {
         blocks += ceil_div(p.part[i].npos, 64) * p.part[i].cblocks;
@@ -510,7 +541,7 @@ int launch_prep(nott_ctx ctx, PrepParams& p) {
     if (p.wt)
         blocks += p.by_cin ? ceil_div(p.k, 64) * ceil_div((int64_t)p.cin * p.taps, 64)
                            : ceil_div((int64_t)p.taps * p.k * p.cin, 256);
-    hipLaunchKernelGGL(nhwc_prep_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, p);
+    hipLaunchKernelGGL(nhwc_prep_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, p);
     return launch_status(ctx, "conv channels-last prep");
 }
 
@@ -602,8 +633,8 @@ void axis_padding(int64_t size, int64_t out, int64_t pad, int64_t taps, int64_t 
     padded = last - first + 1;
 }
 
-bool shape_ok(nott_ctx ctx, const nott_conv2d_desc* d) {
-    return ctx->conv_tap && d->layout == NOTT_NCHW && d->c % 8 == 0 && d->k % 8 == 0 && d->r * d->s <= kMaxTaps;
+bool shape_ok(nott_ctx ctx, const nott_conv2d_desc* d, int64_t chunk = 8) {
+    return ctx->conv_tap && d->layout == NOTT_NCHW && d->c % chunk == 0 && d->k % chunk == 0 && d->r * d->s <= kMaxTaps;
 }
 bool fits(int64_t elems) { return elems < (int64_t(1) << 31); }
 
@@ -612,7 +643,9 @@ bool fits(int64_t elems) { return elems < (int64_t(1) << 31); }
 bool rows_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d) {
     return shape_ok(ctx, d) && fits(d->n * (d->h + 2 * d->pad_h) * (d->w + 2 * d->pad_w) * d->c);
 }
-bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d) { return rows_fwd_applies(ctx, d); }
+bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, size_t elem) {
+    return shape_ok(ctx, d, 16 / (int64_t)elem) && fits(d->n * (d->h + 2 * d->pad_h) * (d->w + 2 * d->pad_w) * d->c);
+}
 bool rows_dgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q) {
     if (!shape_ok(ctx, d) || d->stride_h > 2 || d->stride_w > 2) return false;
     // A 1×1 kernel's gradient reads dy where it lies (conv_tap.hip): once, up to
@@ -636,7 +669,7 @@ int rows_fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, cons
     const int64_t xb = align256(2 * d->n * g.hp * g.wp * d->c);
     char* ws = static_cast<char*>(workspace(ctx, (size_t)(xb + 2 * d->k * d->c * taps)));
     if (!ws) return NOTT_ERR_ALLOC;
-    PrepParams pp{};
+    PrepParams<bf16_t> pp{};
     pp.part[0] = part_of(x, reinterpret_cast<bf16_t*>(ws), d->n, d->c, d->h, d->w, g.hp, g.wp, d->pad_h, d->pad_w,
                          g.sh, g.sw);
     pp.wt = w;
@@ -667,7 +700,7 @@ int rows_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
     const int64_t xb = align256(2 * d->n * hp * wp * d->k);
     char* ws = static_cast<char*>(workspace(ctx, (size_t)(xb + 2 * d->k * d->c * taps)));
     if (!ws) return NOTT_ERR_ALLOC;
-    PrepParams pp{};
+    PrepParams<bf16_t> pp{};
     pp.part[0] = part_of(dy, reinterpret_cast<bf16_t*>(ws), d->n, d->k, p, q, hp, wp, pt, pl);
     pp.wt = w;
     pp.wp2 = reinterpret_cast<bf16_t*>(ws + xb);
@@ -712,8 +745,10 @@ int rows_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
     return launch_rows(ctx, rp, products);
 }
 
-int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* x, const bf16_t* dy,
-               float* dw, int accumulate) {
+template <typename T>
+int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const T* x, const T* dy, float* dw,
+               int accumulate) {
+    constexpr int BK = Slices<T>::kStageK;
     const Gather g(d, p, q);
     const int64_t taps = d->r * d->s;
     const int64_t M = d->k, N = taps * d->c, K = d->n * p * q;
@@ -727,7 +762,7 @@ int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
         const int64_t per = ceil_div(nkb, s), n = ceil_div(nkb, per);
         if (per * BK > kMaxPixels) continue;
         const float fill = std::min(1.f, (float)(tiles * n) / (float)ctx->num_cu);
-        const float us = (float)ceil_div(tiles * n, ctx->num_cu) * ((float)per * (0.63f + 0.53f * fill) + 3.2f) +
+        const float us = (float)ceil_div(tiles * n, ctx->num_cu) * ((float)per * (sizeof(T) == 2 ? 0.63f + 0.53f * fill : 2.1f) + 3.2f) +
                          8.f * (float)(n * M * N) / 7.85e6f + 0.04f * (float)n;
         if (best == 0.f || us < best) {
             best = us;
@@ -735,18 +770,18 @@ int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
         }
     }
     const int64_t splits = ceil_div(nkb, stages);
-    const int64_t xb = align256(2 * d->n * g.hp * g.wp * d->c), yb = align256(2 * K * M);
+    const int64_t xb = align256((int64_t)sizeof(T) * d->n * g.hp * g.wp * d->c), yb = align256((int64_t)sizeof(T) * K * M);
     char* ws = static_cast<char*>(workspace(ctx, (size_t)(xb + yb + 4 * splits * M * N)));
     if (!ws) return NOTT_ERR_ALLOC;
-    PrepParams pp{};
-    pp.part[0] = part_of(x, reinterpret_cast<bf16_t*>(ws), d->n, d->c, d->h, d->w, g.hp, g.wp, d->pad_h, d->pad_w,
+    PrepParams<T> pp{};
+    pp.part[0] = part_of(x, reinterpret_cast<T*>(ws), d->n, d->c, d->h, d->w, g.hp, g.wp, d->pad_h, d->pad_w,
                          g.sh, g.sw);
-    pp.part[1] = part_of(dy, reinterpret_cast<bf16_t*>(ws + xb), d->n, d->k, p, q, p, q, 0, 0);
+    pp.part[1] = part_of(dy, reinterpret_cast<T*>(ws + xb), d->n, d->k, p, q, p, q, 0, 0);
     const int st = launch_prep(ctx, pp);
     if (st != NOTT_OK) return st;
-    WgradParams wg{};
-    wg.dyt = reinterpret_cast<const bf16_t*>(ws + xb);
-    wg.xp = reinterpret_cast<const bf16_t*>(ws);
+    WgradParams<T> wg{};
+    wg.dyt = reinterpret_cast<const T*>(ws + xb);
+    wg.xp = reinterpret_cast<const T*>(ws);
     wg.M = (int32_t)M; wg.N = (int32_t)N; wg.K = (int32_t)K;
     wg.kps = (int32_t)(stages * BK); wg.splits = (int32_t)splits;
     wg.fij = FastDiv((uint32_t)(p * q)); wg.fj = FastDiv((uint32_t)q); wg.fc = FastDiv((uint32_t)d->c);
@@ -759,16 +794,21 @@ int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
     const size_t lds = (size_t)S * 2 * 128 * 128 + 4 * (size_t)wg.kps;
     static bool attr = false;
     if (!attr) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_wgrad_rows_kernel),
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_wgrad_rows_kernel<T>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds) != hipSuccess)
             return fail(ctx, NOTT_ERR_HIP, "conv_gemm: cannot reserve LDS");
         attr = true;
     }
-    hipLaunchKernelGGL(conv_wgrad_rows_kernel, dim3((unsigned)(tiles * splits)), dim3(64 * NW), lds, ctx->stream, wg);
+    hipLaunchKernelGGL(conv_wgrad_rows_kernel<T>, dim3((unsigned)(tiles * splits)), dim3(64 * NW), lds, ctx->stream, wg);
     gemm::launch_splitk_reduce(ctx, wg.ws, splits, M, N,
                                TapMajorStore{dw, wg.fc, (int32_t)d->c, (int32_t)taps, accumulate});
     return launch_status(ctx, "conv_gemm wgrad");
 }
+
+template int rows_wgrad<float>(nott_ctx, const nott_conv2d_desc*, int64_t, int64_t, const float*, const float*, float*,
+                               int);
+template int rows_wgrad<bf16_t>(nott_ctx, const nott_conv2d_desc*, int64_t, int64_t, const bf16_t*, const bf16_t*,
+                                float*, int);
 
 }  // namespace conv_fast
 }  // namespace nott
