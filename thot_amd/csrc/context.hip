@@ -26,6 +26,7 @@ void* workspace(nott_ctx ctx, size_t bytes) {
     void* fresh = nullptr;
     hipError_t e = hipMalloc(&fresh, want);
     if (e != hipSuccess) {
+        (void)hipGetLastError();   // a caller that goes on without the workspace must not find this error at its launch
         fail(ctx, NOTT_ERR_ALLOC, std::string("workspace hipMalloc of ") + std::to_string(want) +
                                       " bytes failed: " + hipGetErrorString(e));
         return nullptr;

@@ -806,18 +806,22 @@ int wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const v
             // the bias gradient comes out of the same pass
             st = cin1_wgrad<T>(ctx, d, static_cast<const T*>(x), static_cast<const T*>(dy), dw, db, accumulate);
             db = nullptr;
-        } else if (nott::conv_fast::rows_wgrad_applies(ctx, d, sizeof(T))) {
-            st = nott::conv_fast::rows_wgrad<T>(ctx, d, p, q, static_cast<const T*>(x), static_cast<const T*>(dy), dw,
-                                                accumulate);
-        } else if (sizeof(T) == 2 && col_applies(d, p, q, false)) {
-            st = col_wgrad(ctx, d, p, q, reinterpret_cast<const bf16_t*>(x), reinterpret_cast<const bf16_t*>(dy), dw,
-                           accumulate);
         } else {
-            const int64_t M = d->k, N = d->c * d->r * d->s, K = d->n * p * q;
-            WgradALoader<T> la{static_cast<const T*>(dy), g, M, K};
-            WgradBLoader<T> lb{static_cast<const T*>(x), g, N, K};
-            WgradStore ep{dw, M, N, accumulate};
-            st = run<T>(ctx, la, lb, ep, M, N, K);
+            st = NOTT_ERR_ALLOC;
+            if (nott::conv_fast::rows_wgrad_applies(ctx, d, sizeof(T)))
+                st = nott::conv_fast::rows_wgrad<T>(ctx, d, p, q, static_cast<const T*>(x), static_cast<const T*>(dy),
+                                                    dw, accumulate);
+            // without it, or with no room for its copies: the paths that read x and dy where they lie
+            if (st == NOTT_ERR_ALLOC && sizeof(T) == 2 && col_applies(d, p, q, false))
+                st = col_wgrad(ctx, d, p, q, reinterpret_cast<const bf16_t*>(x), reinterpret_cast<const bf16_t*>(dy),
+                               dw, accumulate);
+            if (st == NOTT_ERR_ALLOC) {
+                const int64_t M = d->k, N = d->c * d->r * d->s, K = d->n * p * q;
+                WgradALoader<T> la{static_cast<const T*>(dy), g, M, K};
+                WgradBLoader<T> lb{static_cast<const T*>(x), g, N, K};
+                WgradStore ep{dw, M, N, accumulate};
+                st = run<T>(ctx, la, lb, ep, M, N, K);
+            }
         }
         if (st != NOTT_OK) return st;
     }
