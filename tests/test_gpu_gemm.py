@@ -324,6 +324,38 @@ def test_conv_channels_last_gemm(ops, oracle, case):
         assert torch.equal(again, dw + dw)
 
 
+def _context(ops, monkeypatch, **env):
+    """A context of its own, created under these environment variables."""
+    for key, value in env.items():
+        monkeypatch.setenv(key, value)
+    ctx = ops.Context(torch.cuda.current_device())
+    monkeypatch.setattr(ops, "_contexts", {torch.cuda.current_device(): ctx})
+    return ctx
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("case", [(64, 128, 28, 28, 256, 3, 3, 2, 1, 1), (64, 64, 56, 56, 128, 3, 3, 2, 1, 1),
+                                  (16, 256, 14, 14, 512, 3, 3, 2, 1, 1)], ids=lambda c: "n{}c{}h{}w{}k{}".format(*c))
+def test_conv_wgrad_precision(ops, monkeypatch, dt, case):
+    """Weight gradients from the channels-last copies are no further from 64 bits
+    than those of the paths that read x and dy where they lie (NOTT_CONV_TAP=0):
+    the ratio of the two errors of the same inputs, each a 2-norm over at least
+    73728 weights (a deviation of well under 1%), 5% allowed."""
+    n, c, h, w_, k, r, s, st, pad, dil = case
+    d = _desc(ops, case)
+    torch.manual_seed(sum(case))
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    x = torch.randn(n, c, h, w_, device="cuda").to(tdt)
+    dy = torch.randn(n, k, conv_out(h, r, st, pad, dil), conv_out(w_, s, st, pad, dil), device="cuda").to(tdt)
+    cols = torch.nn.functional.unfold(x.double(), (r, s), padding=pad, stride=st)
+    want = sum(dy[i].double().view(k, -1) @ cols[i].t().contiguous() for i in range(n)).view(k, c, r, s)
+    got = ops.conv2d_bwd_weight(x, dy, d)[0]
+    _context(ops, monkeypatch, NOTT_CONV_TAP="0")
+    plain = ops.conv2d_bwd_weight(x, dy, d)[0]
+    err, err_plain = ((t.double() - want).norm().item() for t in (got, plain))
+    assert err <= 1.05 * err_plain, (err / want.norm().item(), err_plain / want.norm().item())
+
+
 @pytest.mark.parametrize("name", ["conv3x3_s1p1_bias", "conv3x3_s2p1", "conv7x7_s2p3", "conv1x1_s2",
                                   "conv3x3_dil2_rect"])
 def test_conv_golden(ops, name):
