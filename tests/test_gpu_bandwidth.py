@@ -443,6 +443,23 @@ def test_layernorm(ops, oracle, dt, rows, d):
     check(host(dg2), 2 * dge, "f32", "ln dgamma accumulate")
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("d", [41, 2345, 10001, 16384])
+def test_layernorm_mean_precision(ops, dt, d):
+    """The mean is as near to 64 bits as a division of a pairwise sum leaves it:
+    exact for a row of ones (41 and 2345 are lengths whose fp32 reciprocal does
+    not give 1 again), and within half a unit of the last place (2^-24) in the
+    root mean square over rows of any values.  A sum of n parts added one after
+    another (16 waves) is off by up to sqrt(n/3) such units."""
+    gamma = torch.ones(d, device="cuda", dtype=getattr(torch, {"f32": "float32", "bf16": "bfloat16"}[dt]))
+    y, mean, _ = ops.layernorm_fwd(torch.ones(3, d, device="cuda", dtype=gamma.dtype), gamma, gamma)
+    assert (mean == 1).all() and (y == 1).all()
+    x = (torch.randn(512, d, device="cuda", generator=torch.Generator(device="cuda").manual_seed(d)) * 1.5 + 3).to(gamma.dtype)
+    _, mean, _ = ops.layernorm_fwd(x, gamma, gamma)
+    want = x.double().mean(1)
+    assert ((mean.double() - want) / want).pow(2).mean().sqrt().item() <= 2.0 ** -24
+
+
 def test_layernorm_full_size_invariants(ops):
     """C3a shape 16384 x 1024: per-row Σdx = 0 and Σdx·x̂ = 0 (exact in reals)."""
     g = torch.Generator(device="cuda").manual_seed(3)
