@@ -460,6 +460,22 @@ def test_layernorm_mean_precision(ops, dt, d):
     assert ((mean.double() - want) / want).pow(2).mean().sqrt().item() <= 2.0 ** -24
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("d", [72, 77, 100, 1100])
+def test_layernorm_large_mean(ops, oracle, dt, d):
+    """A row whose mean times rstd overflows while its columns are finite: the
+    lanes past its end take no part (1100 columns end inside the second wave)."""
+    x = np.full((2, d), 2.0 ** 110, np.float32)
+    mean = np.full(2, 2.0 ** 110, np.float32)
+    rstd = np.full(2, 2.0 ** 20, np.float32)   # -mean * rstd is past fp32's range; (x - mean) * rstd is 0
+    gamma, dy = np.ones(d, np.float32), host_input(rng(d).standard_normal((2, d)), dt)
+    dx, dg, db = ops.layernorm_bwd(dev(x, dt), dev(dy, dt), dev(mean), dev(rstd), dev(gamma, dt))
+    dxe, dge, dbe = oracle.layernorm_bwd(x, dy, mean, rstd, gamma)
+    check(host(dx), dxe, dt, "ln dx", atol=2.0 ** 20 * (2e-2 if dt == "bf16" else 1e-5))
+    check(host(dg), dge, "f32", "ln dgamma")
+    check(host(db), dbe, "f32", "ln dbeta")
+
+
 def test_layernorm_full_size_invariants(ops):
     """C3a shape 16384 x 1024: per-row Σdx = 0 and Σdx·x̂ = 0 (exact in reals)."""
     g = torch.Generator(device="cuda").manual_seed(3)

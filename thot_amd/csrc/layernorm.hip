@@ -50,7 +50,7 @@ struct Row {
     static constexpr int NG = DPL / G;
     static __device__ __forceinline__ int64_t col(int t, int e) { return ((int64_t)(e / G) * P + t) * G + e % G; }
     // Every lane issues all of its loads unconditionally (columns past d read
-    // column 0 and are zeroed by unpack), so a row's loads stay in flight
+    // column 0 and get unpack's `past`), so a row's loads stay in flight
     // together.
     template <typename T, bool NT>
     static __device__ __forceinline__ void load(const T* __restrict__ p, int64_t d, int t,
@@ -63,14 +63,14 @@ struct Row {
     }
     template <typename T>
     static __device__ __forceinline__ void unpack(const typename Group<T, G>::Raw (&raw)[NG], int64_t d, int t,
-                                                  float (&v)[DPL]) {
+                                                  float (&v)[DPL], float past = 0.f) {
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
             const int64_t c0 = ((int64_t)g * P + t) * G;
             float x[G];
             Group<T, G>::unpack(raw[g], x);
 #pragma unroll
-            for (int e = 0; e < G; ++e) v[G * g + e] = c0 < d ? x[e] : 0.f;
+            for (int e = 0; e < G; ++e) v[G * g + e] = c0 < d ? x[e] : past;
         }
     }
     template <typename T, bool NT>
@@ -224,9 +224,11 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_bwd_kernel(const T* __re
         if (WPR == 1 && r >= rows) break;
         const bool in = WPR == 1 || r < rows;
         float xv[DPL], gv[DPL];
-        R::template unpack<T>(rx, d, t, xv);
-        R::template unpack<T>(rd, d, t, gv);
         const float mu = nmu, rs = nrs;
+        // columns past d hold the mean: x̂ is 0 there (−μ·rstd may overflow, and
+        // times their zero dy it would be a NaN in the row's sums)
+        R::template unpack<T>(rx, d, t, xv, mu);
+        R::template unpack<T>(rd, d, t, gv);
         if (r0 + stride < rows) fetch(r + stride);
         float s[2] = {0.f, 0.f};
 #pragma unroll
