@@ -125,9 +125,15 @@ __device__ __forceinline__ void row_sum(float (&v)[K], float* red) {
 
 // s / d given inv = 1 / d: the product, corrected by what it leaves of s (the
 // product by itself is up to 1.13 times further from 64 bits in the mean and in
-// dx, and a division costs 11% of the forward at 30000 x 64).
+// dx, and a division costs 11% of the forward at 30000 x 64).  Aligned rows of up
+// to 1024 columns (SHORT: one wave, 16-byte groups) take the product alone and dy·γ
+// rounded; the rest would cost them 4% (30000 x 64 bf16: backward 13.5 against
+// 12.9 us).
+template <bool SHORT>
 __device__ __forceinline__ float over(float s, float d, float inv) {
-    const float q = s * inv, c = fmaf(fmaf(-q, d, s), inv, q);
+    const float q = s * inv;
+    if constexpr (SHORT) return q;
+    const float c = fmaf(fmaf(-q, d, s), inv, q);
     return c == c ? c : q;   // (an infinite sum)
 }
 
@@ -141,6 +147,7 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_fwd_kernel(const T* __re
                                                                    T* __restrict__ y, float* __restrict__ mean,
                                                                    float* __restrict__ rstd, int64_t rows, int64_t d) {
     constexpr int P = 64 * WPR;
+    constexpr bool SHORT = WPR == 1 && G > 1;
     typedef Row<DPL, G, P> R;
     __shared__ float red[2][GROUPS * WPR];
     const int t = threadIdx.x % P, grp = threadIdx.x / P;
@@ -159,7 +166,7 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_fwd_kernel(const T* __re
 #pragma unroll
         for (int e = 0; e < DPL; ++e) s[0] += v[e];
         row_sum<WPR, 1>(s, red[0]);
-        const float mu = over(s[0], fd, inv_d);
+        const float mu = over<SHORT>(s[0], fd, inv_d);
         s[0] = 0.f;
 #pragma unroll
         for (int e = 0; e < DPL; ++e) {
@@ -167,7 +174,7 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_fwd_kernel(const T* __re
             s[0] += u * u;
         }
         row_sum<WPR, 1>(s, red[1]);
-        const float rs = 1.f / sqrtf(over(s[0], fd, inv_d) + eps);
+        const float rs = 1.f / sqrtf(over<SHORT>(s[0], fd, inv_d) + eps);
 #pragma unroll
         for (int e = 0; e < DPL; ++e) v[e] = (v[e] - mu) * rs * gm[e] + bt[e];
         if (!in) continue;
@@ -183,7 +190,8 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_fwd_kernel(const T* __re
 // past 8192 columns): ordinary loads and stores, with the next row's loads in
 // flight while the current row is reduced (measured best at 16384x1024, where
 // it streams 5.8 TB/s fp32; wider rows keep the same bytes in flight per CU:
-// 4096x4096 bf16 24 us a call, 8192x8192 86 us).  A block per row whose dγ / dβ
+// 4096x4096 bf16 24 us a call, 8192x8192 86 us; past 8192 columns one row at a
+// time: 2048x16384 bf16 64 us, fp32 107).  A block per row whose dγ / dβ
 // partials were written for every row took 71 and 344 us, and 59 us for 5000x771
 // fp32 (19 now).
 template <typename T, int DPL, int G, int WPR, int GROUPS>
@@ -194,9 +202,14 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_bwd_kernel(const T* __re
                                                                    float* __restrict__ partial, int64_t rows,
                                                                    int64_t d) {
     constexpr int P = 64 * WPR, NT = P * GROUPS;
+    constexpr bool SHORT = WPR == 1 && G > 1;
     typedef Row<DPL, G, P> R;
     extern __shared__ float lds[];  // [GROUPS][2][d] (one group: unused)
     __shared__ float red[2][GROUPS * WPR * 2];
+    // 16 waves leave a lane 128 registers: enough for a row, not for the next one
+    // beside it (with it the kernel spilled 19 to 107 registers: 2000 x 10001 bf16
+    // 183 us against 39, 2048 x 16384 fp32 174 against 107)
+    constexpr bool AHEAD = WPR < 16;
     const int t = threadIdx.x % P, grp = threadIdx.x / P;
     float gm[DPL];
     R::template load_all<T, false>(gamma, d, t, gm);
@@ -210,26 +223,30 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_bwd_kernel(const T* __re
     typename Group<T, G>::Raw rx[R::NG], rd[R::NG];
     float nmu = 0.f, nrs = 0.f;
     auto fetch = [&](int64_t r) {
-        r = r < rows ? r : rows - 1;   // (a group past the end re-reads the last row)
-        R::template load<T, false>(x + r * d, d, t, rx);
-        R::template load<T, false>(dy + r * d, d, t, rd);
+        if (WPR > 1 && GROUPS > 1) r = r < rows ? r : rows - 1;   // (a group past the end re-reads the last row)
+        int at = t;
+        if constexpr (!AHEAD) asm volatile("" : "+v"(at));   // (its columns are formed here, not kept from row to row)
+        R::template load<T, false>(x + r * d, d, at, rx);
+        R::template load<T, false>(dy + r * d, d, at, rd);
         nmu = mean[r];
         nrs = rstd[r];
     };
     int buf = 0;
-    const int64_t first = (int64_t)blockIdx.x * GROUPS;
-    if (first < rows) fetch(first + grp);
-    for (int64_t r0 = first; r0 < rows; r0 += stride) {
-        const int64_t r = r0 + grp;
-        if (WPR == 1 && r >= rows) break;
+    // A wave that has rows to itself stops with its own last one; waves that share
+    // them go on with the block.
+    const int64_t own = WPR == 1 ? 0 : grp;   // rows of the block before the one that decides
+    const int64_t first = (int64_t)blockIdx.x * GROUPS + grp;
+    if (AHEAD && first - own < rows) fetch(first);
+    for (int64_t r = first; r - own < rows; r += stride) {
         const bool in = WPR == 1 || r < rows;
+        if (!AHEAD) fetch(r);
         float xv[DPL], gv[DPL];
         const float mu = nmu, rs = nrs;
         // columns past d hold the mean: x̂ is 0 there (−μ·rstd may overflow, and
         // times their zero dy it would be a NaN in the row's sums)
         R::template unpack<T>(rx, d, t, xv, mu);
         R::template unpack<T>(rd, d, t, gv);
-        if (r0 + stride < rows) fetch(r + stride);
+        if (AHEAD && r + stride - own < rows) fetch(r + stride);
         float s[2] = {0.f, 0.f};
 #pragma unroll
         for (int e = 0; e < DPL; ++e) {
@@ -243,25 +260,28 @@ __global__ __launch_bounds__(64 * WPR * GROUPS) void ln_bwd_kernel(const T* __re
             s[0] += g;
             s[1] += g * xh;
             xv[e] = xh;
+            if constexpr (SHORT) gv[e] = g;
         }
         row_sum<WPR, 2>(s, red[buf]);
         buf ^= 1;
-        const float sg = over(s[0], fd, inv_d), sgx = over(s[1], fd, inv_d);
+        const float sg = over<SHORT>(s[0], fd, inv_d), sgx = over<SHORT>(s[1], fd, inv_d);
 #pragma unroll
         for (int e = 0; e < DPL; ++e) {
-            // dy·γ unrounded (rounded as in the sums: 8% further from 64 bits in
-            // fp32), but for a single column, where it cancels against its own sum
-            float g = -sg;
-            if (WPR == 1 && G == 1 && e == 0 && d == 1) {
-                float rounded = gv[e] * gm[e];
+            float g;
+            if constexpr (SHORT) {
+                g = gv[e] - sg;
+            } else if (WPR == 1 && e == 0 && d == 1) {
+                float rounded = gv[e] * gm[e];   // a single column cancels against its own rounded sum
                 asm volatile("" : "+v"(rounded));
-                g += rounded;
+                g = rounded - sg;
             } else {
-                g = fmaf(gv[e], gm[e], g);
+                g = fmaf(gv[e], gm[e], -sg);     // dy·γ unrounded
             }
             xv[e] = rs * (g - xv[e] * sgx);
         }
-        if (in) R::template store<T>(dx + r * d, d, t, xv);
+        int at = t;
+        if constexpr (!AHEAD) asm volatile("" : "+v"(at));
+        if (in) R::template store<T>(dx + r * d, d, at, xv);
     }
     // This block's partial row: layout [which][16-column group][block][16], so
     // that the reduction reads each group's partials as one contiguous run.
