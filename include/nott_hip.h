@@ -300,7 +300,8 @@ int nott_layernorm_bwd_noalloc(nott_ctx ctx, nott_dtype dtype, int64_t rows, int
  * ignore_index -100, optional label smoothing, no class weights.
  * logits, dlogits [n, c] (dtype); labels int64 [n].  One pass computes
  * dlogits = grad_scale·(softmax − (1−ε)·onehot − ε/c)/n_valid and, if loss
- * is non-NULL, the mean loss (fp32 scalar). */
+ * is non-NULL, the mean loss (fp32 scalar; infinite where smoothing meets a
+ * logit of −inf).  dlogits may be logits. */
 int nott_softmax_xent_bwd(nott_ctx ctx, nott_dtype dtype, int64_t n, int64_t c,
                           const void* logits, const int64_t* labels,
                           double label_smoothing, double grad_scale,

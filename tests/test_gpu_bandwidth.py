@@ -547,13 +547,49 @@ def test_softmax_xent_any_row(ops, oracle, dt, n, c, eps, at):
     db = torch.full((n * c + 8,), 7.0, dtype=tdt, device="cuda")
     zv, dv = zb[at[0]:at[0] + n * c].view(n, c), db[at[1]:at[1] + n * c].view(n, c)
     zv.copy_(dev(z, dt))
-    if eps == 0.0:                             # (a smoothed loss of −inf is infinite)
+    if eps == 0.0:                             # (with smoothing it makes the loss infinite)
         zv[0, c // 2] = -math.inf
     _, loss = ops.softmax_xent_bwd(zv, torch.from_numpy(y).cuda(), label_smoothing=eps, out=dv)
     dle, losse = oracle.softmax_xent(z, y, eps)
     check(host(dv), dle, dt, "xent dlogits")
     check(loss.item(), losse, "f32", "xent loss", rtol=1e-5)
     assert (db[:at[1]] == 7).all() and (db[at[1] + n * c:] == 7).all()
+
+
+# One size for each kernel and register shape, in whole 16-byte groups and not.
+XENT_PATHS = [(64, 10), (300, 10), (300, 37), (300, 40), (100, 77), (100, 200), (40, 1000), (40, 1001), (20, 8192),
+              (20, 9001), (9, 16383), (9, 16385), (9, 20000), (7, 32768), (5, 32769), (5, 50257), (4, 106001),
+              (3, 128256), (3, 150001)]
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n,c", XENT_PATHS)
+def test_softmax_xent_minus_infinity_and_in_place(ops, oracle, dt, n, c):
+    """A logit of -inf has probability 0 and makes the smoothed loss (its sum of
+    -log p) infinite, at every length and alignment; dlogits may be logits."""
+    g = rng(n + c)
+    z = host_input(g.standard_normal((n, c)) * 2.0, dt)
+    y = torch.from_numpy(g.integers(0, c - 1, n).astype(np.int64)).cuda()
+    zi = z.copy()
+    zi[1, c - 1] = -math.inf
+    for eps in (0.0, 0.1):
+        dl, loss = ops.softmax_xent_bwd(dev(zi, dt), y, label_smoothing=eps)
+        dle, losse = oracle.softmax_xent(np.where(np.isinf(zi), -9984.0, zi).astype(np.float32), y.cpu().numpy(), eps)
+        check(host(dl), dle, dt, "dlogits with -inf")
+        if eps:
+            assert loss.item() == math.inf
+        else:
+            check(loss.item(), losse, "f32", "loss with -inf", rtol=1e-5)
+        buf = torch.zeros(n * c + 1, dtype=dl.dtype, device="cuda")
+        for at in (0, 1):                      # an element off the 16-byte boundary: the kernels for any row
+            plain = buf[at:at + n * c].view(n, c)
+            plain.copy_(dev(z, dt))
+            want, want_loss = ops.softmax_xent_bwd(plain, y, label_smoothing=eps)
+            got, got_loss = ops.softmax_xent_bwd(plain, y, label_smoothing=eps, out=plain)
+            assert torch.equal(got_loss, want_loss)
+            check(host(got), host(want), dt, "dlogits in place")
+            plain.copy_(dev(zi, dt))
+            assert (ops.softmax_xent_bwd(plain, y, label_smoothing=eps)[1].item() == math.inf) == (eps > 0)
 
 
 @pytest.mark.parametrize("dt", DTYPES)

@@ -8,7 +8,9 @@
 //   lse = max + log Σ exp(z − max)
 //   dz  = grad_scale · (exp(z − lse) − (1−ε)·[j == y] − ε/c) / n_valid
 //   loss_i = (1−ε)·(lse − z_y) + (ε/c)·(c·lse − Σ_j z_j)
-// Each row lives in registers of one workgroup: one HBM read, one write.
+// (a logit of −inf makes the smoothed loss infinite, as Σ_j z_j does.)
+// Each row lives in registers of one workgroup: one HBM read, one write; what a
+// row's stores follow is read before them, so dlogits may be logits itself.
 #include "common.hpp"
 
 #include <algorithm>
@@ -74,9 +76,9 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
 // (the label's term applied once, by the thread that holds it); the row sum
 // of the logits is formed only when label smoothing needs it.
 template <typename T, int NT, int EPT>
-__device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int64_t y, const T* __restrict__ z,
-                                              int64_t c, float smoothing, float grad_scale, int nv,
-                                              T* __restrict__ dz, float* __restrict__ row_loss, float* red) {
+__device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int64_t y, const T* z,
+                                              int64_t c, float smoothing, float grad_scale, int nv, T* dz,
+                                              float* __restrict__ row_loss, float* red) {
     constexpr int NWAVES = NT / 64;
     constexpr int G = Pack16<T>::N;
     constexpr int NG = EPT / G;
@@ -104,8 +106,13 @@ __device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int6
     float se = 0.f, sz = 0.f;
     if (smoothing != 0.f) {
 #pragma unroll
-        for (int e = 0; e < EPT; ++e) sz += (v[e] == -INFINITY) ? 0.f : v[e];
+        for (int g = 0; g < NG; ++g)
+            if ((g * NT + (int)threadIdx.x) * G < ci) {
+#pragma unroll
+                for (int e = 0; e < G; ++e) sz += v[g * G + e];
+            }
     }
+    const float zy = Io<T>::ld(z, y);   // before the stores: dlogits may be logits
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
         const float pe = __builtin_amdgcn_exp2f(fmaf(v[e], kLog2e, -mxl));
@@ -133,10 +140,7 @@ __device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int6
         }
         Pack16<T>::template st<true>(dz + j0, t);
     }
-    if (threadIdx.x == 0 && row_loss) {
-        const float zy = Io<T>::ld(z, y);
-        row_loss[row] = hit * (lse - zy) + off * ((float)c * lse - sz);
-    }
+    if (threadIdx.x == 0 && row_loss) row_loss[row] = hit * (lse - zy) + off * ((float)c * lse - sz);
 }
 
 // Vector path: 16-byte groups of G = 4 (fp32) or 8 (bf16) elements, strided
@@ -146,10 +150,9 @@ __device__ __forceinline__ void xent_row_body(float (&v)[EPT], int64_t row, int6
 // loads are issued before the current row is reduced and written, so a CU's
 // loads stay in flight through the block reductions and the stores.
 template <typename T, int NT, int EPT>
-__global__ __launch_bounds__(NT) void xent_rows_vec_kernel(const T* __restrict__ logits,
-                                                           const int64_t* __restrict__ labels, int64_t n, int64_t c,
-                                                           float smoothing, float grad_scale,
-                                                           const int* __restrict__ nvalid, T* __restrict__ dlogits,
+__global__ __launch_bounds__(NT) void xent_rows_vec_kernel(const T* logits, const int64_t* __restrict__ labels,
+                                                           int64_t n, int64_t c, float smoothing, float grad_scale,
+                                                           const int* __restrict__ nvalid, T* dlogits,
                                                            float* __restrict__ row_loss) {
     constexpr int G = Pack16<T>::N;
     constexpr int NG = EPT / G;
@@ -232,11 +235,10 @@ __device__ __forceinline__ typename Pack16<T>::Raw minus_inf() {
 // moves 4096 x 50257 fp32 at 5.1 TB/s (324 us), 8192 x 128256 bf16 at 5.4 TB/s
 // (780 us) and 2048 x 151936 fp32 at 5.2 TB/s (482 us); three passes of single
 // elements per row took 846, 3529 and 1247 us.
-// inf_counts: whether a logit of −inf enters the smoothed loss's Σ z_j.
 template <typename T, int NT, int EPT, bool REST>
 __global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
-    const T* __restrict__ logits, const int64_t* __restrict__ labels, int64_t c, float smoothing, float grad_scale,
-    const int* __restrict__ nvalid, T* __restrict__ dlogits, float* __restrict__ row_loss, int inf_counts) {
+    const T* logits, const int64_t* __restrict__ labels, int64_t c, float smoothing, float grad_scale,
+    const int* __restrict__ nvalid, T* dlogits, float* __restrict__ row_loss) {
     constexpr int G = Pack16<T>::N;
     constexpr int NG = EPT / G;
     constexpr int NWAVES = NT / 64;
@@ -296,7 +298,7 @@ __global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
 #pragma unroll
                 for (int e = 0; e < G; ++e) {
                     se += __builtin_amdgcn_exp2f(fmaf(t[u][e], kLog2e, -ml));
-                    if (k + u * NT < groups && (inf_counts || t[u][e] != -INFINITY)) sz += t[u][e];
+                    if (k + u * NT < groups) sz += t[u][e];
                 }
         }
     }
@@ -328,15 +330,14 @@ __global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
     if constexpr (REST) se = mx == -INFINITY ? se : se * __builtin_amdgcn_exp2f((mx - m) * kLog2e);
     se += ej >= 0 ? ep : 0.f;
     if (smoothing != 0.f) {
-        if (ej >= 0 && (inf_counts || ez != -INFINITY)) sz += ez;
+        if (ej >= 0) sz += ez;
 #pragma unroll
         for (int g = 0; g < NG; ++g)
             if (g * NT < rem) {
                 float t[G];
                 Pack16<T>::unpack(raw[g], t);
 #pragma unroll
-                for (int e = 0; e < G; ++e)
-                    if (inf_counts || t[e] != -INFINITY) sz += t[e];
+                for (int e = 0; e < G; ++e) sz += t[e];
                 asm volatile("" : "+v"(raw[g]));
             }
     }
@@ -420,8 +421,8 @@ __global__ void xent_nan_kernel(float* __restrict__ loss) { *loss = __builtin_na
 // One row of c <= 64 columns per wave, lane j holding column j: writes the
 // gradient and returns the row's loss (0 for an ignored row).
 template <typename T>
-__device__ __forceinline__ float xent_wave_row(const T* __restrict__ z, int64_t y, int64_t c, float smoothing,
-                                               float grad_scale, int nv, T* __restrict__ dz) {
+__device__ __forceinline__ float xent_wave_row(const T* z, int64_t y, int64_t c, float smoothing, float grad_scale,
+                                               int nv, T* dz) {
     constexpr float kLog2e = 1.4426950408889634f;
     const int lane = threadIdx.x & 63, ci = (int)c;
     const float v = lane < ci ? Io<T>::ld(z, lane) : -INFINITY;
@@ -431,7 +432,7 @@ __device__ __forceinline__ float xent_wave_row(const T* __restrict__ z, int64_t 
     }
     const float zy = Io<T>::ld(z, y);
     const float mx = wave_max(v);
-    const float sz = smoothing != 0.f ? wave_sum(v == -INFINITY ? 0.f : v) : 0.f;
+    const float sz = smoothing != 0.f ? wave_sum(lane < ci ? v : 0.f) : 0.f;
     const float pe = __builtin_amdgcn_exp2f(fmaf(v, kLog2e, -mx * kLog2e));
     const float se = wave_sum(pe);
     const float lse = mx + __logf(se);
@@ -453,10 +454,9 @@ __device__ __forceinline__ float xent_wave_row(const T* __restrict__ z, int64_t 
 // Rows of c <= 64 columns that are not whole 16-byte groups, when there are
 // too many for the single-workgroup kernel below: one row per wave.
 template <typename T>
-__global__ __launch_bounds__(256) void xent_wave_kernel(const T* __restrict__ logits,
-                                                        const int64_t* __restrict__ labels, int64_t n, int64_t c,
-                                                        float smoothing, float grad_scale,
-                                                        const int* __restrict__ nvalid, T* __restrict__ dlogits,
+__global__ __launch_bounds__(256) void xent_wave_kernel(const T* logits, const int64_t* __restrict__ labels, int64_t n,
+                                                        int64_t c, float smoothing, float grad_scale,
+                                                        const int* __restrict__ nvalid, T* dlogits,
                                                         float* __restrict__ row_loss) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= n) return;
@@ -476,9 +476,8 @@ __global__ __launch_bounds__(256) void xent_wave_kernel(const T* __restrict__ lo
 // against 17 us on the general path; the two meet near 250 rows.)
 constexpr int64_t kSmallRows = 256;
 template <typename T>
-__global__ __launch_bounds__(1024) void xent_small_kernel(const T* __restrict__ logits,
-                                                          const int64_t* __restrict__ labels, int64_t n, int64_t c,
-                                                          float smoothing, float grad_scale, T* __restrict__ dlogits,
+__global__ __launch_bounds__(1024) void xent_small_kernel(const T* logits, const int64_t* __restrict__ labels, int64_t n,
+                                                          int64_t c, float smoothing, float grad_scale, T* dlogits,
                                                           float* __restrict__ loss,
                                                           unsigned long long* __restrict__ err) {
     __shared__ float red[16];
@@ -539,9 +538,9 @@ void launch_vec(nott_ctx ctx, const RowArgs<T>& a) {
 }
 
 template <typename T, int NT, int EPT, bool REST>
-void launch_any(nott_ctx ctx, const RowArgs<T>& a, int inf_counts) {
+void launch_any(nott_ctx ctx, const RowArgs<T>& a) {
     hipLaunchKernelGGL((xent_any_kernel<T, NT, EPT, REST>), dim3((unsigned)a.n), dim3(NT), 0, ctx->stream, a.logits,
-                       a.labels, a.c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss, inf_counts);
+                       a.labels, a.c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
 }
 
 template <typename T>
@@ -564,13 +563,13 @@ void dispatch(nott_ctx ctx, const RowArgs<T>& a) {
                            a.logits, a.labels, a.n, c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
         return;
     }
-    if (c <= 64 * 16) return launch_any<T, 64, 16, false>(ctx, a, 0);
-    if (c <= 256 * 32) return launch_any<T, 256, 32, false>(ctx, a, 0);
-    if (c <= 512 * 32) return launch_any<T, 512, 32, false>(ctx, a, 0);
-    if (c <= 512 * 64) return launch_any<T, 512, 64, false>(ctx, a, 1);
-    if (c <= 512 * 104) return launch_any<T, 512, 104, false>(ctx, a, 1);
-    if (c <= 1024 * 104) return launch_any<T, 1024, 104, false>(ctx, a, 1);
-    return launch_any<T, 1024, 104, true>(ctx, a, 1);
+    if (c <= 64 * 16) return launch_any<T, 64, 16, false>(ctx, a);
+    if (c <= 256 * 32) return launch_any<T, 256, 32, false>(ctx, a);
+    if (c <= 512 * 32) return launch_any<T, 512, 32, false>(ctx, a);
+    if (c <= 512 * 64) return launch_any<T, 512, 64, false>(ctx, a);
+    if (c <= 512 * 104) return launch_any<T, 512, 104, false>(ctx, a);
+    if (c <= 1024 * 104) return launch_any<T, 1024, 104, false>(ctx, a);
+    return launch_any<T, 1024, 104, true>(ctx, a);
 }
 
 }  // namespace
