@@ -520,10 +520,11 @@ def test_softmax_xent(ops, oracle, dt, n, c, eps, ignore):
 
 
 # Rows that are not whole 16-byte groups, or longer than the vector path takes:
-# at the edges of what a thread holds (64 x 16, 256 x 32, 512 x 32, 512 x 64,
+# at the edges of what a thread holds (64 x 1, 2, 4, 8 and 16, 256 x 32, 512 x 32, 512 x 64,
 # 512 x 104 and 1024 x 104 elements), past the last (the rest is streamed), and
 # below two groups with too many rows for one workgroup.
-XENT_ANY = [(4100, 7, 0.0), (4100, 17, 0.1), (4097, 33, 0.0), (70, 65, 0.1), (50, 1023, 0.0), (40, 1025, 0.1),
+XENT_ANY = [(4100, 7, 0.0), (4100, 17, 0.1), (4097, 33, 0.0), (70, 65, 0.1), (71, 127, 0.0), (70, 129, 0.1),
+            (69, 255, 0.0), (69, 257, 0.1), (69, 511, 0.1), (70, 513, 0.0), (50, 1023, 0.0), (40, 1025, 0.1),
             (20, 8191, 0.0), (20, 8193, 0.1), (9, 16383, 0.1), (9, 16385, 0.1), (7, 32767, 0.0), (7, 32776, 0.1),
             (5, 53247, 0.1), (5, 53256, 0.0), (4, 106496, 0.1), (4, 106497, 0.0), (3, 128256, 0.1), (3, 250001, 0.1)]
 

@@ -234,7 +234,9 @@ __device__ __forceinline__ typename Pack16<T>::Raw minus_inf() {
 // (up to 53248 columns) or one 1024-thread row on a CU.  Bound by memory: it
 // moves 4096 x 50257 fp32 at 5.1 TB/s (324 us), 8192 x 128256 bf16 at 5.4 TB/s
 // (780 us) and 2048 x 151936 fp32 at 5.2 TB/s (482 us); three passes of single
-// elements per row took 846, 3529 and 1247 us.
+// elements per row took 846, 3529 and 1247 us.  Short rows share the lines at their
+// ends: up to 1024 columns loads, and fp32 stores, go through the caches (16000 x
+// 1001 fp32 31.7 us, 33.8 past them).
 template <typename T, int NT, int EPT, bool REST>
 __global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
     const T* logits, const int64_t* __restrict__ labels, int64_t c, float smoothing, float grad_scale,
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
     if (groups > 0) {
 #pragma unroll
         for (int g = 0; g < NG; ++g)
-            raw[g] = Pack16<T>::template raw<true>(zb + (unsigned)(tid + min(g * NT, rem - 1)) * G);
+            raw[g] = Pack16<T>::template raw<(EPT > 16)>(zb + (unsigned)(tid + min(g * NT, rem - 1)) * G);
     }
     float m = mx;
 #pragma unroll
@@ -371,7 +373,7 @@ __global__ __launch_bounds__(NT, EPT > 64 ? 4 : 1) void xent_any_kernel(
     };
     auto put = [&](T* p, const float (&t)[G]) {
         if (vec_st) {
-            Pack16<T>::template st<true>(p, t);
+            Pack16<T>::template st<(EPT > 16 || sizeof(T) == 2)>(p, t);
         } else {
 #pragma unroll
             for (int e = 0; e < G; ++e) Io<T>::st(p, e, t[e]);
@@ -418,42 +420,61 @@ __global__ __launch_bounds__(1024) void xent_loss_kernel(const float* __restrict
 
 __global__ void xent_nan_kernel(float* __restrict__ loss) { *loss = __builtin_nanf(""); }
 
-// One row of c <= 64 columns per wave, lane j holding column j: writes the
-// gradient and returns the row's loss (0 for an ignored row).
-template <typename T>
+// One row of c <= 64·EPL columns per wave, lane j holding columns j, j + 64, ...:
+// writes the gradient and returns the row's loss (0 for an ignored row).
+template <typename T, int EPL>
 __device__ __forceinline__ float xent_wave_row(const T* z, int64_t y, int64_t c, float smoothing, float grad_scale,
                                                int nv, T* dz) {
     constexpr float kLog2e = 1.4426950408889634f;
     const int lane = threadIdx.x & 63, ci = (int)c;
-    const float v = lane < ci ? Io<T>::ld(z, lane) : -INFINITY;
+    float v[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) v[e] = e * 64 + lane < ci ? Io<T>::ld(z, e * 64 + lane) : -INFINITY;
     if (!(y >= 0 && y < c)) {
-        if (lane < ci) Io<T>::st(dz, lane, 0.f);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e)
+            if (e * 64 + lane < ci) Io<T>::st(dz, e * 64 + lane, 0.f);
         return 0.f;
     }
     const float zy = Io<T>::ld(z, y);
-    const float mx = wave_max(v);
-    const float sz = smoothing != 0.f ? wave_sum(lane < ci ? v : 0.f) : 0.f;
-    const float pe = __builtin_amdgcn_exp2f(fmaf(v, kLog2e, -mx * kLog2e));
-    const float se = wave_sum(pe);
+    float mx = v[0], sz = 0.f, se = 0.f;
+#pragma unroll
+    for (int e = 1; e < EPL; ++e) mx = fmaxf(mx, v[e]);
+    mx = wave_max(mx);
+    if (smoothing != 0.f) {
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) sz += e * 64 + lane < ci ? v[e] : 0.f;
+        sz = wave_sum(sz);
+    }
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+        v[e] = __builtin_amdgcn_exp2f(fmaf(v[e], kLog2e, -mx * kLog2e));
+        se += v[e];
+    }
+    se = wave_sum(se);
     const float lse = mx + __logf(se);
     const float scale = grad_scale / (float)nv;
     const float off = smoothing / (float)c;
     const float hit = 1.f - smoothing;
-    if (lane < ci) {
-        float g = fmaf(pe, scale / se, -scale * off);
-        if (lane == (int)y) {
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+        const int j = e * 64 + lane;
+        if (j >= ci) continue;
+        float g = fmaf(v[e], scale / se, -scale * off);
+        if (j == (int)y) {
             // not contracted, whatever a caller's loop hoists: both kernels give the same bits
 #pragma clang fp contract(off)
             g = g - scale * hit;
         }
-        Io<T>::st(dz, lane, g);
+        Io<T>::st(dz, j, g);
     }
     return hit * (lse - zy) + off * ((float)c * lse - sz);
 }
 
-// Rows of c <= 64 columns that are not whole 16-byte groups, when there are
-// too many for the single-workgroup kernel below: one row per wave.
-template <typename T>
+// Rows of c <= 64·EPL columns that are not whole 16-byte groups (of up to 64
+// columns when there are too many for the single-workgroup kernel below): one
+// row per wave.
+template <typename T, int EPL>
 __global__ __launch_bounds__(256) void xent_wave_kernel(const T* logits, const int64_t* __restrict__ labels, int64_t n,
                                                         int64_t c, float smoothing, float grad_scale,
                                                         const int* __restrict__ nvalid, T* dlogits,
@@ -461,7 +482,7 @@ __global__ __launch_bounds__(256) void xent_wave_kernel(const T* logits, const i
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= n) return;
     const float l =
-        xent_wave_row(logits + row * c, labels[row], c, smoothing, grad_scale, *nvalid, dlogits + row * c);
+        xent_wave_row<T, EPL>(logits + row * c, labels[row], c, smoothing, grad_scale, *nvalid, dlogits + row * c);
     if ((threadIdx.x & 63) == 0 && row_loss) row_loss[row] = l;
 }
 
@@ -498,7 +519,8 @@ __global__ __launch_bounds__(1024) void xent_small_kernel(const T* logits, const
     const int nv = nvs;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     for (int64_t row = wid; row < n; row += 16) {
-        const float l = xent_wave_row(logits + row * c, labels[row], c, smoothing, grad_scale, nv, dlogits + row * c);
+        const float l =
+            xent_wave_row<T, 1>(logits + row * c, labels[row], c, smoothing, grad_scale, nv, dlogits + row * c);
         if (lane == 0) rl[row] = l;
     }
     if (!loss) return;
@@ -537,6 +559,12 @@ void launch_vec(nott_ctx ctx, const RowArgs<T>& a) {
                        a.n, a.c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
 }
 
+template <typename T, int EPL>
+void launch_wave(nott_ctx ctx, const RowArgs<T>& a) {
+    hipLaunchKernelGGL((xent_wave_kernel<T, EPL>), dim3((unsigned)nott::ceil_div(a.n, 4)), dim3(256), 0, ctx->stream,
+                       a.logits, a.labels, a.n, a.c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
+}
+
 template <typename T, int NT, int EPT, bool REST>
 void launch_any(nott_ctx ctx, const RowArgs<T>& a) {
     hipLaunchKernelGGL((xent_any_kernel<T, NT, EPT, REST>), dim3((unsigned)a.n), dim3(NT), 0, ctx->stream, a.logits,
@@ -548,8 +576,11 @@ void dispatch(nott_ctx ctx, const RowArgs<T>& a) {
     constexpr int G = Pack16<T>::N;
     // Whole aligned groups of up to 32768 columns: the persistent kernel, whose
     // next row is in flight during the reductions (5.7 TB/s at 16384 x 32000
-    // fp32).  Everything else: the kernel for any row, in the smallest shape
-    // that holds it (the single-column rows of up to 64 one wave each).
+    // fp32).  Everything else: up to 512 columns one wave a row, single elements
+    // (16000 x 77 15.7 us, x 255 18.2 to 19.9, x 511 23.1 to 24.8; one 64-thread
+    // workgroup of the kernel for any row 21.3, 22, 22.9 to 24.5 and 0.8 us more
+    // at 100 rows); past that the kernel for any row, in the smallest shape that
+    // holds it.
     const int64_t c = a.c;
     const bool vec = (c % G == 0) && ((uintptr_t)a.logits % 16 == 0) && ((uintptr_t)a.dl % 16 == 0);
     if (vec && c <= 64 * 16) return launch_vec<T, 64, 16>(ctx, a);
@@ -558,11 +589,10 @@ void dispatch(nott_ctx ctx, const RowArgs<T>& a) {
     // two rows (plus the two prefetched ones) are in flight per CU.
     if (vec && sizeof(T) == 2 && c <= 512 * 64) return launch_vec<T, 512, 64>(ctx, a);
     if (vec && c <= 1024 * 32) return launch_vec<T, 1024, 32>(ctx, a);
-    if (c <= 64) {
-        hipLaunchKernelGGL(xent_wave_kernel<T>, dim3((unsigned)nott::ceil_div(a.n, 4)), dim3(256), 0, ctx->stream,
-                           a.logits, a.labels, a.n, c, a.eps, a.scale, a.nvalid, a.dl, a.row_loss);
-        return;
-    }
+    if (c <= 64) return launch_wave<T, 1>(ctx, a);
+    if (c <= 128) return launch_wave<T, 2>(ctx, a);
+    if (c <= 256) return launch_wave<T, 4>(ctx, a);
+    if (c <= 512) return launch_wave<T, 8>(ctx, a);
     if (c <= 64 * 16) return launch_any<T, 64, 16, false>(ctx, a);
     if (c <= 256 * 32) return launch_any<T, 256, 32, false>(ctx, a);
     if (c <= 512 * 32) return launch_any<T, 512, 32, false>(ctx, a);
