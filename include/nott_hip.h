@@ -55,8 +55,10 @@ typedef struct nott_ctx_s* nott_ctx;
  * word.  When a call needs more workspace, a new arena (at least twice the
  * size) is allocated and the old one is kept, not freed, until nott_destroy:
  * a HIP graph captured earlier keeps its workspace pointer valid, and no
- * stream is synchronised for growth.  The workspace is shared by every call
- * on the context, so calls on different streams that overlap race on it.
+ * stream is synchronised for growth.  While the stream is captured the arena
+ * cannot grow (run the same calls once before): calls that can do with less
+ * then take a slower path, the others return NOTT_ERR_ALLOC.  The workspace
+ * is shared by every call on the context, so calls on different streams that overlap race on it.
  * Replaces nothing in the reference (libtorch keeps this state in its
  * caching allocator and per-device stream pool). */
 int nott_create(int device, nott_ctx* out);
@@ -81,7 +83,11 @@ int nott_workspace_bytes(nott_ctx ctx, int64_t* bytes);
  * (layer/details/conv.hpp:140-191, module created at :177; options :39-49).
  * Layout NCHW is the reference default; NHWC is its ChannelsLast mode
  * (core.hpp:2546-2561, conv.hpp:178-182).  groups must be 1, padding_mode
- * "zeros".  Output size p = (h + 2*pad_h - dil_h*(r-1) - 1)/stride_h + 1. */
+ * "zeros".  Output size p = (h + 2*pad_h - dil_h*(r-1) - 1)/stride_h + 1.
+ * Workspace: NCHW layers other than 3x3 stride 1 (strided, 1x1, 5x5, ...)
+ * hold a zero-padded channels-last copy of what they stream in the arena: bf16
+ * forward x, data gradient dy; weight gradient (both types) x and dy.  Where
+ * the arena cannot hold it they read the tensors where they lie, slower. */
 typedef struct nott_conv2d_desc {
     int64_t n, c, h, w;        /* input  x  [n, c, h, w] (logical)          */
     int64_t k;                 /* output channels; weight [k, c, r, s]      */

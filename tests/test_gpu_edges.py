@@ -121,3 +121,59 @@ def test_empty_elementwise(dt):
     e = torch.empty(0, dtype=dt, device="cuda")
     assert ops.relu_bwd(e, e).shape == (0,)
     assert ops.add(e, e).shape == (0,)
+
+
+# Calls on a context whose workspace cannot grow (its stream is being captured, so
+# an allocation would end the capture): the arena is what one small call left, 1
+# MiB.  Each has a path that does with less: a convolution without its
+# channels-last copies, a product without split partials, the single-workgroup
+# cross-entropy.
+def _conv(n, c, h, k):
+    d = ops.conv_desc((n, c, h, h), (k, c, 3, 3), stride=(2, 2), padding=(1, 1))
+    xs, ys = ops._conv_shapes(d)
+    return d, torch.randn(xs, device="cuda").bfloat16(), torch.randn((k, c, 3, 3), device="cuda").bfloat16(), \
+        torch.randn(ys, device="cuda").bfloat16()
+
+
+def _small_workspace_calls():
+    torch.manual_seed(4)
+    d, x, w, dy = _conv(8, 32, 64, 32)
+    d2, x2, _, dy2 = _conv(16, 24, 32, 24)
+    a, b, g = (torch.randn(s, device="cuda").bfloat16() for s in ((2040, 1024), (136, 1024), (2040, 136)))
+    z, y = torch.randn((4096, 10), device="cuda"), torch.randint(0, 10, (4096,), device="cuda")
+    return {"conv forward": lambda: ops.conv2d_fwd(x, w, None, d),
+            "conv data gradient": lambda: ops.conv2d_bwd_data(dy, w, d),
+            "conv weight gradient": lambda: ops.conv2d_bwd_weight(x2, dy2, d2)[0],
+            "linear": lambda: ops.linear_fwd(a, b),
+            "linear weight gradient": lambda: ops.linear_bwd(g, a, b, need_dx=False)[1],
+            "cross-entropy": lambda: ops.softmax_xent_bwd(z, y)[0]}
+
+
+@pytest.mark.parametrize("what", sorted(["conv forward", "conv data gradient", "conv weight gradient", "linear",
+                                         "linear weight gradient", "cross-entropy"]))
+def test_without_room_in_the_workspace(monkeypatch, what):
+    call = _small_workspace_calls()[what]
+    want = call().float()
+    ctx = ops.Context(torch.cuda.current_device())
+    monkeypatch.setattr(ops, "_contexts", {torch.cuda.current_device(): ctx})
+    if what != "cross-entropy":                # (that one needs none at all)
+        one = torch.ones((2, 64), device="cuda")
+        ops.layernorm_bwd(one, one, one[:, 0].contiguous(), one[:, 0].contiguous(), one[0].contiguous())
+    torch.cuda.synchronize()
+    held = ctx.workspace_bytes()
+    assert held <= 1 << 20
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = call()
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        # bf16 results of two orders of summation: a unit of the last place (2^-8) of the
+        # result, and fp32 sums of at most 8192 terms of order 1
+        torch.testing.assert_close(got.float(), want, rtol=2.0 ** -7, atol=1e-3 * want.abs().max().item())
+    assert ctx.workspace_bytes() == held
+    assert ctx.lib.nott_last_error(ctx.handle) == b""
+    # the same call where the arena may grow
+    again = call().float()
+    torch.testing.assert_close(again, want, rtol=0, atol=0)

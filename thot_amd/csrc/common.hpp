@@ -20,6 +20,8 @@ struct nott_ctx_s {
     size_t ws_bytes = 0;
     std::vector<void*> retired;    // earlier, smaller workspaces: kept until nott_destroy
     size_t retired_bytes = 0;      // their total size
+    size_t refused_bytes = 0;      // the last optional workspace that could not be allocated,
+    int refused_calls = 0;         // and how many more calls do not ask for as much again
     void* ln_scratch = nullptr;    // this device's static LayerNorm scratch (nott_layernorm_bwd_noalloc)
     unsigned long long* err_word = nullptr;  // device counter of data errors
     int num_cu = 256;
@@ -52,6 +54,11 @@ int hip_fail(nott_ctx ctx, hipError_t e, const char* what);
 // stream, and HIP graphs captured with the old pointer, keep valid memory.
 // Retired arenas are freed by nott_destroy.
 void* workspace(nott_ctx ctx, size_t bytes);
+// The same for a caller that has a way without it: nullptr, with no error set,
+// also while the context's stream is captured and the arena would have to grow
+// (an allocation would end the capture), and for some calls after a failed
+// allocation of this size or less.
+void* optional_workspace(nott_ctx ctx, size_t bytes);
 // Looks up this device's static LayerNorm scratch (layernorm.hip).
 int layernorm_scratch_setup(nott_ctx ctx);
 // Checks the last launch and records an error message.

@@ -40,6 +40,29 @@ void* workspace(nott_ctx ctx, size_t bytes) {
     return ctx->ws;
 }
 
+void* optional_workspace(nott_ctx ctx, size_t bytes) {
+    constexpr int kCallsBetweenTries = 64;   // a failing hipMalloc may go through the driver, and memory may come free
+    if (bytes <= ctx->ws_bytes && ctx->ws) return ctx->ws;
+    if (ctx->stream) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (status != hipStreamCaptureStatusNone) return nullptr;
+    }
+    if (ctx->refused_calls > 0 && bytes >= ctx->refused_bytes) {
+        --ctx->refused_calls;
+        return nullptr;
+    }
+    const std::string before = ctx->last_error;
+    void* ws = workspace(ctx, bytes);
+    if (!ws) ctx->last_error = before;
+    ctx->refused_bytes = ws ? 0 : bytes;
+    ctx->refused_calls = ws ? 0 : kCallsBetweenTries;
+    return ws;
+}
+
 int launch_status(nott_ctx ctx, const char* kernel) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(ctx, e, kernel);

@@ -504,7 +504,7 @@ int col_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, con
     Carve cv;
     const int64_t o_dyt = cv.take(2 * d->k * NPQ), o_col = cv.take(2 * CRSp * NPQ);
     const int64_t o_part = cv.take(4 * (int64_t)fast::partial_floats(ctx, d->k, CRSp, NPQ));
-    char* ws = static_cast<char*>(nott::workspace(ctx, (size_t)cv.off));
+    char* ws = static_cast<char*>(nott::optional_workspace(ctx, (size_t)cv.off));
     if (!ws) return NOTT_ERR_ALLOC;
     bf16_t* dyt = reinterpret_cast<bf16_t*>(ws + o_dyt);
     bf16_t* col = reinterpret_cast<bf16_t*>(ws + o_col);

@@ -675,7 +675,7 @@ int rows_fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, cons
     const Gather g(d, p, q);
     const int64_t taps = d->r * d->s;
     const int64_t xb = align256(2 * d->n * g.hp * g.wp * d->c);
-    char* ws = static_cast<char*>(workspace(ctx, (size_t)(xb + 2 * d->k * d->c * taps)));
+    char* ws = static_cast<char*>(optional_workspace(ctx, (size_t)(xb + 2 * d->k * d->c * taps)));
     if (!ws) return NOTT_ERR_ALLOC;
     PrepParams<bf16_t> pp{};
     pp.part[0] = part_of(x, reinterpret_cast<bf16_t*>(ws), d->n, d->c, d->h, d->w, g.hp, g.wp, d->pad_h, d->pad_w,
@@ -706,7 +706,7 @@ int rows_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
     axis_padding(d->h, p, d->pad_h, d->r, d->stride_h, d->dil_h, pt, hp);
     axis_padding(d->w, q, d->pad_w, d->s, d->stride_w, d->dil_w, pl, wp);
     const int64_t xb = align256(2 * d->n * hp * wp * d->k);
-    char* ws = static_cast<char*>(workspace(ctx, (size_t)(xb + 2 * d->k * d->c * taps)));
+    char* ws = static_cast<char*>(optional_workspace(ctx, (size_t)(xb + 2 * d->k * d->c * taps)));
     if (!ws) return NOTT_ERR_ALLOC;
     PrepParams<bf16_t> pp{};
     pp.part[0] = part_of(dy, reinterpret_cast<bf16_t*>(ws), d->n, d->k, p, q, hp, wp, pt, pl);
@@ -779,7 +779,7 @@ int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
     }
     const int64_t splits = ceil_div(nkb, stages);
     const int64_t xb = align256((int64_t)sizeof(T) * d->n * g.hp * g.wp * d->c), yb = align256((int64_t)sizeof(T) * K * M);
-    char* ws = static_cast<char*>(workspace(ctx, (size_t)(xb + yb + 4 * splits * M * N)));
+    char* ws = static_cast<char*>(optional_workspace(ctx, (size_t)(xb + yb + 4 * splits * M * N)));
     if (!ws) return NOTT_ERR_ALLOC;
     PrepParams<T> pp{};
     pp.part[0] = part_of(x, reinterpret_cast<T*>(ws), d->n, d->c, d->h, d->w, g.hp, g.wp, d->pad_h, d->pad_w,

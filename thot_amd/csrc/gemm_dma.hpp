@@ -573,11 +573,11 @@ int run(nott_ctx ctx, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb
     if (!applies<AT, BT>(A, lda, B, ldb, M, N, K)) return NOTT_ERR_UNSUPPORTED;
     // The split reduce that also sums rows works on 4-column groups.
     if (ROWSUM && N % 4 != 0) splits = 1;
-    const Plan p = plan(ctx, M, N, K, AT && BT, splits);
-    if (p.splits == 1) return launch_shape<AT, BT, ROWSUM>(ctx, p.shape, A, lda, B, ldb, ep, M, N, K, 1, p.kps);
+    Plan p = plan(ctx, M, N, K, AT && BT, splits);
     const size_t body = (size_t)(p.splits * M * N), rows = ROWSUM ? (size_t)(p.splits * M) : 0;
-    float* ws = static_cast<float*>(workspace(ctx, sizeof(float) * (body + rows)));
-    if (!ws) return NOTT_ERR_ALLOC;
+    float* ws = p.splits > 1 ? static_cast<float*>(optional_workspace(ctx, sizeof(float) * (body + rows))) : nullptr;
+    if (p.splits > 1 && !ws) p = plan(ctx, M, N, K, AT && BT, 1);   // no room for the partials
+    if (p.splits == 1) return launch_shape<AT, BT, ROWSUM>(ctx, p.shape, A, lda, B, ldb, ep, M, N, K, 1, p.kps);
     const int st = launch_shape<AT, BT, ROWSUM>(ctx, p.shape, A, lda, B, ldb, PartialRowStore{ws, ws + body, M, N}, M,
                                                 N, K, p.splits, p.kps);
     if (st != NOTT_OK) return st;

@@ -488,21 +488,23 @@ __global__ __launch_bounds__(256) void xent_wave_kernel(const T* logits, const i
 
 // Small problems (c <= 64 classes, n <= kSmallRows rows; a classifier head at
 // a small batch): the label count, every row and the mean loss in one
-// 1024-thread workgroup, where the general path takes three launches.  A wave
+// 1024-thread workgroup, where the general path takes three launches and a
+// workspace (without one, as under capture on a new context, up to
+// kMostSmallRows rows go this way).  A wave
 // owns rows wid, wid + 16, ...; the arithmetic and the summation orders are
 // those of xent_count_kernel, xent_wave_kernel and xent_loss_kernel, so where
 // the general path takes that kernel (c not a multiple of the 16-byte group)
 // both give the same bits; its vector path sums each thread's group first.
 // (One row per wave at a time costs 40 ns a row, 167 us at 4096 x 10 fp32
 // against 17 us on the general path; the two meet near 250 rows.)
-constexpr int64_t kSmallRows = 256;
+constexpr int64_t kSmallRows = 256, kMostSmallRows = 4096;
 template <typename T>
 __global__ __launch_bounds__(1024) void xent_small_kernel(const T* logits, const int64_t* __restrict__ labels, int64_t n,
                                                           int64_t c, float smoothing, float grad_scale, T* dlogits,
                                                           float* __restrict__ loss,
                                                           unsigned long long* __restrict__ err) {
     __shared__ float red[16];
-    __shared__ float rl[kSmallRows];
+    __shared__ float rl[kMostSmallRows];
     __shared__ int nvs;
     float cnt = 0.f;
     unsigned bad = 0;
@@ -619,7 +621,9 @@ extern "C" int nott_softmax_xent_bwd(nott_ctx ctx, nott_dtype dtype, int64_t n, 
         return nott::launch_status(ctx, "softmax_xent");
     }
     const float eps = (float)label_smoothing, scale = (float)grad_scale;
-    if (c <= 64 && n <= kSmallRows) {
+    // workspace: [nvalid int][pad to 256 B][row_loss n floats]
+    const size_t need = 256 + sizeof(float) * (size_t)n;
+    if (c <= 64 && (n <= kSmallRows || (n <= kMostSmallRows && !nott::optional_workspace(ctx, need)))) {
         if (dtype == NOTT_F32)
             hipLaunchKernelGGL(xent_small_kernel<float>, dim3(1), dim3(1024), 0, ctx->stream,
                                static_cast<const float*>(logits), labels, n, c, eps, scale,
@@ -630,8 +634,7 @@ extern "C" int nott_softmax_xent_bwd(nott_ctx ctx, nott_dtype dtype, int64_t n, 
                                static_cast<bf16_t*>(dlogits), loss, ctx->err_word);
         return nott::launch_status(ctx, "softmax_xent");
     }
-    // workspace: [nvalid int][pad to 256 B][row_loss n floats]
-    char* ws = static_cast<char*>(nott::workspace(ctx, 256 + sizeof(float) * (size_t)n));
+    char* ws = static_cast<char*>(nott::workspace(ctx, need));
     if (!ws) return NOTT_ERR_ALLOC;
     int* nvalid = reinterpret_cast<int*>(ws);
     float* row_loss = loss ? reinterpret_cast<float*>(ws + 256) : nullptr;
