@@ -20,6 +20,7 @@ HIPCC = "/opt/rocm/bin/hipcc"
 # source: (pattern of the kernels' names, spilled registers allowed)
 LIMITS = {
     "layernorm.hip": [(r"ln_(fwd|bwd)_kernel", 0)],
+    "attention.hip": [(r"attn_(fwd32|dq32|dkdv32)_kernel", 2)],
 }
 
 
