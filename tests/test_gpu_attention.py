@@ -66,6 +66,19 @@ CASES = [
     (1, 1, 260, 260, 104, False),
     (1, 2, 300, 300, 128, True),
     (1, 1, 1, 1, 128, True),
+    # head sizes past 96 on both sides of where the backward leaves the 16x16
+    # kernels: 64 rows, 96 by 96, a causal 128, 80 keys, 320 queries; then a grid
+    # of more 64-row blocks than CUs
+    (2, 2, 64, 64, 128, True),
+    (1, 2, 65, 64, 128, False),
+    (1, 2, 96, 96, 112, False),
+    (1, 2, 96, 97, 112, False),
+    (1, 2, 128, 128, 104, True),
+    (1, 2, 129, 129, 104, True),
+    (1, 1, 320, 80, 128, False),
+    (1, 1, 321, 80, 128, False),
+    (1, 1, 320, 81, 120, False),
+    (9, 29, 65, 65, 128, False),
 ]
 CASES_F32 = [c for c in CASES if c[4] <= 64]   # (fp32 takes head sizes up to 64)
 

@@ -970,6 +970,22 @@ int fwd_nd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const voi
 // score of ±inf survives.
 bool applies(const AttnParams& p, int elem) { return elem == 2 && p.vec && p.scale != 0.f; }
 
+// Whether the backward takes them too.  Head dims past 96 run one wave per SIMD
+// and 128 rows per workgroup, so short sequences stay on the 16×16 kernels: those
+// of one 64-row block (512 heads of 64 x 128, causal, 37.6 against 46.7 us; 32
+// heads 19.5 against 21.1), and while a 64-row grid has fewer workgroups than
+// CUs, up to 80 keys (8 x 192 queries, 64 keys 27.0 against 27.7; 32 x 300, 77 keys
+// 39.6 against 42.2), 96 by 96 (27.2 against 28.0) or a causal 128 (27.8 against
+// 30.4).  Past those lines these are the faster: 8 x 192 causal 35.1 against 35.6,
+// 8 x 320, 96 keys 38.0 against 38.8, 256 x 96 causal 20% and 256 x 96 full 39%.
+bool bwd_applies(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, int elem) {
+    if (!applies(p, elem)) return false;
+    if (d->dh <= 96) return true;
+    if (d->t <= 64 && d->s <= 64) return false;
+    if (d->b * d->h * ceil_div(d->t, 64) > ctx->num_cu || d->t > 320) return true;
+    return !(d->s <= 80 || (d->t <= 96 && d->s <= 96) || (p.causal && d->t <= 128));
+}
+
 int fwd(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const void* q, const void* k, const void* v, void* o,
         float* lse) {
     // A 2-deep ring leaves room for four workgroups per CU at 64 columns (a 3-deep
@@ -1634,7 +1650,8 @@ extern "C" int nott_attention_bwd(nott_ctx ctx, const nott_attn_desc* d, nott_dt
     NOTT_REQUIRE(ctx, q && k && v && o && dO && lse && dq && dk && dv, "nott_attention_bwd: null buffer");
     if (!(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(dO) && aligned16(o))) p.vec = 0;
     nott::DeviceScope scope(ctx->device);
-    if (fa::applies(p, (int)nott::dtype_size(dtype))) return fa::bwd(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
+    if (fa::bwd_applies(ctx, d, p, (int)nott::dtype_size(dtype)))
+        return fa::bwd(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
     return dtype == NOTT_F32 ? bwd<float>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv)
                              : bwd<bf16_t>(ctx, d, p, q, k, v, o, dO, lse, dq, dk, dv);
 }
