@@ -271,6 +271,7 @@ def test_conv_nhwc(ops, oracle, dt, case):
 # taps that no pixel takes), classes without taps (1×1 stride 2), strides above 2
 # (the data gradient stays on the general path), different strides per axis,
 # 25 taps, tiles on both sides of 64 and 128 rows and columns, rows over 64 wide.
+# (The weight gradients over 32 pixels or fewer stay on the general path.)
 CONV_ROWS = [
     (1, 8, 3, 3, 8, (3, 3), (1, 1), (0, 0), (1, 1)),
     (2, 24, 9, 7, 40, (3, 3), (2, 2), (1, 1), (1, 1)),
@@ -322,6 +323,59 @@ def test_conv_channels_last_gemm(ops, oracle, case):
         again = dw.clone()
         ops.conv2d_bwd_weight(X, DY, d, dw=again, accumulate=True)
         assert torch.equal(again, dw + dw)
+
+
+# n, c, h, w, k, r, s, stride, padding, dilation on both sides of the lines between the
+# channels-last copies and the paths that read the tensors where they lie: forward
+# (planes of whole 1024s of pixels, one channel chunk, an input past the cache, long
+# chains on few tiles), 1×1 and strided data gradients, more than 9 taps, and weight
+# gradients over few pixels (32 of few weights, 73 and 80 of 1.2 million, whole 64s).
+CONV_LINES = [
+    (64, 32, 64, 64, 40, 3, 3, 2, 1, 1), (63, 32, 64, 64, 40, 3, 3, 2, 1, 1),
+    (57, 24, 48, 48, 24, 3, 3, 2, 1, 1), (56, 24, 48, 48, 24, 3, 3, 2, 1, 1),
+    (64, 96, 96, 96, 8, 3, 3, 2, 1, 1), (62, 96, 96, 96, 8, 3, 3, 2, 1, 1),
+    (1, 256, 16, 16, 64, 3, 3, 2, 1, 1), (16, 256, 32, 32, 64, 3, 3, 2, 1, 1),
+    (15, 64, 56, 56, 96, 1, 1, 1, 0, 1), (14, 64, 56, 56, 96, 1, 1, 1, 0, 1),
+    (16, 128, 56, 56, 160, 1, 1, 1, 0, 1), (16, 128, 56, 56, 32, 1, 1, 1, 0, 1),
+    (4, 32, 7, 7, 512, 3, 3, 2, 1, 1), (40, 32, 28, 28, 256, 3, 3, 2, 1, 1),
+    (1, 16, 16, 16, 512, 5, 5, 1, 2, 1), (1, 16, 16, 16, 256, 5, 5, 1, 2, 1),
+    (2, 24, 8, 8, 32, 3, 3, 2, 1, 1), (2, 24, 9, 8, 32, 3, 3, 2, 1, 1),
+    (8, 256, 6, 6, 512, 3, 3, 2, 1, 1), (5, 256, 8, 8, 512, 3, 3, 2, 1, 1),
+    (8, 256, 16, 16, 512, 3, 3, 2, 1, 1), (9, 256, 16, 16, 512, 3, 3, 2, 1, 1),
+]
+
+
+@pytest.mark.parametrize("case", CONV_LINES, ids=lambda c: "n{}c{}h{}w{}k{}r{}".format(*c[:6]))
+def test_conv_both_sides_of_the_lines(ops, case):
+    """Against float64, with the bounds of test_conv_channels_last_gemm."""
+    n, c, h, w_, k, r, s, st, pad, dil = case
+    d = _desc(ops, case)
+    torch.manual_seed(sum(case))
+    x = torch.randn(n, c, h, w_, device="cuda").bfloat16()
+    w = torch.randn(k, c, r, s, device="cuda").bfloat16()
+    dy = torch.randn(n, k, conv_out(h, r, st, pad, dil), conv_out(w_, s, st, pad, dil), device="cuda").bfloat16()
+    b = torch.randn(k, device="cuda")
+
+    def near(got, want, mag, terms, rel, what):
+        over = (got.double() - want.view_as(got)).abs() - (terms * 2.0 ** -23 * mag.view_as(got) + rel * want.view_as(got).abs())
+        assert over.max().item() <= 0, f"{what}: over the bound by {over.max().item():.3g}"
+
+    def sums(f):
+        wd, yd, geo = f(w.double()).view(k, -1), f(dy.double()).view(n, k, -1), dict(padding=pad, stride=st, dilation=dil)
+        y, dx, dw = [], [], 0
+        for i in range(n):
+            cols = torch.nn.functional.unfold(f(x[i:i + 1].double()), (r, s), **geo)[0]
+            y.append(wd @ cols + f(b.double())[:, None])
+            dx.append(torch.nn.functional.fold((wd.t().contiguous() @ yd[i])[None], (h, w_), (r, s), **geo)[0])
+            dw = dw + yd[i] @ cols.t().contiguous()
+        return torch.stack(y), torch.stack(dx), dw
+
+    (y, dx, dw), (ym, dxm, dwm) = sums(lambda t: t), sums(torch.abs)
+    pixels = dy.numel() // k
+    near(ops.conv2d_fwd(x, w, b, d), y, ym, c * r * s + 1, 2.0 ** -8, "y")
+    near(ops.conv2d_bwd_data(dy, w, d), dx, dxm, k * r * s, 2.0 ** -8, "dx")
+    near(ops.conv2d_bwd_weight(x, dy, d)[0], dw, dwm, pixels, 0.0, "dw")
+    near(ops.conv2d_bwd_weight(x.float(), dy.float(), d)[0], dw, dwm, pixels, 0.0, "dw f32")
 
 
 def _context(ops, monkeypatch, **env):

@@ -750,7 +750,7 @@ int fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const voi
         return nott::conv_fast::stem_fwd<T>(ctx, d, static_cast<const T*>(x), static_cast<const T*>(w), b,
                                             static_cast<T*>(y), relu);
     if constexpr (sizeof(T) == 2) {
-        if (nott::conv_fast::rows_fwd_applies(ctx, d)) {
+        if (nott::conv_fast::rows_fwd_applies(ctx, d, p, q, col_applies(d, p, q, false))) {
             const int st = nott::conv_fast::rows_fwd(ctx, d, p, q, static_cast<const T*>(x), static_cast<const T*>(w),
                                                      b, static_cast<T*>(y), relu);
             if (st != NOTT_ERR_ALLOC) return st;   // no room for the channels-last copy: the paths below
@@ -808,7 +808,7 @@ int wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const v
             db = nullptr;
         } else {
             st = NOTT_ERR_ALLOC;
-            if (nott::conv_fast::rows_wgrad_applies(ctx, d, sizeof(T)))
+            if (nott::conv_fast::rows_wgrad_applies(ctx, d, p, q, sizeof(T), sizeof(T) == 2 && col_applies(d, p, q, false)))
                 st = nott::conv_fast::rows_wgrad<T>(ctx, d, p, q, static_cast<const T*>(x), static_cast<const T*>(dy),
                                                     dw, accumulate);
             // without it, or with no room for its copies: the paths that read x and dy where they lie

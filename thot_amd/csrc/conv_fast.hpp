@@ -36,9 +36,10 @@ int tap_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, const T* dy, const T* w, 
 
 // Implicit GEMMs over a channels-last copy (the weight gradient in both types, the rest bf16), for the shapes without a kernel
 // of their own (conv_gemm.hip; NOTT_CONV_TAP=0 switches them off as well).
-bool rows_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d);
+// Each answers whether they take the shape and are not slower there than the path below; `col`: that is the column path.
+bool rows_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, bool col);
 bool rows_dgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q);
-bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, size_t elem);
+bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, size_t elem, bool col);
 int rows_fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* x, const bf16_t* w,
              const float* b, bf16_t* y, int relu);
 int rows_dgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* dy, const bf16_t* w,

@@ -16,8 +16,8 @@
 //             split over the pixels, partials summed in order
 // 128×128 (or 128×64) tiles of 32×32×16 MFMAs, a 3-deep ring of 64-deep stages.
 //
-// With the copies, µs of forward / data / weight gradient, against the tap and
-// im2col paths (which stay for other channel counts):
+// With the copies, µs of forward / data / weight gradient, against the tap and im2col
+// paths (which take other channel counts, and where the rules below say so):
 //   [64, 128, 28, 28] → 256, 3×3 stride 2    29 / 38 / 38    was  56 / 60 / 54
 //   [64, 64, 56, 56] → 128, 3×3 stride 2     38 / 41 / 50    was  53 / 59 / 69
 //   [64, 512, 14, 14] → 512, 1×1             35 / 35 / 34    was  51 / 73 / 46
@@ -577,12 +577,11 @@ template <int BN, int P> int launch_rows_as(nott_ctx ctx, RowParams& p) {
     hipLaunchKernelGGL(fn, dim3((unsigned)tiles), dim3(64 * NW), (size_t)p.ring + 8 * kMaxTaps, ctx->stream, p);
     return launch_status(ctx, "conv_gemm");
 }
+bool narrow_tiles(nott_ctx ctx, int64_t wide, int64_t N);
 int launch_rows(nott_ctx ctx, RowParams& p, int products) {
     int64_t wide = 0;
     for (int i = 0; i < p.ncls; ++i) wide += ceil_div(p.cls[i].M, BM) * ceil_div(p.N, 128);
-    // 128 × 64 tiles also where the wide ones would not give every CU one: [64, 256,
-    // 14, 14] → 512, stride 2, 34 µs forward and 42 data gradient against 36 and 46.
-    const bool n64 = p.N <= 64 || wide < ctx->num_cu;
+    const bool n64 = narrow_tiles(ctx, wide, p.N);
     if (products == 2) return n64 ? launch_rows_as<64, 2>(ctx, p) : launch_rows_as<128, 2>(ctx, p);
     return n64 ? launch_rows_as<64, 1>(ctx, p) : launch_rows_as<128, 1>(ctx, p);
 }
@@ -646,13 +645,52 @@ bool shape_ok(nott_ctx ctx, const nott_conv2d_desc* d, int64_t chunk = 8) {
 }
 bool fits(int64_t elems) { return elems < (int64_t(1) << 31); }
 
+// Tiles of M rows and N columns of a product over `classes` row classes of about M
+// rows each: 128 × 64 ones also where the wide ones would not give every CU one ([64,
+// 256, 14, 14] → 512, stride 2, 34 µs forward and 42 data gradient against 36 and 46).
+bool narrow_tiles(nott_ctx ctx, int64_t wide, int64_t N) { return N <= 64 || wide < ctx->num_cu; }
+int64_t row_tiles(nott_ctx ctx, int64_t M, int64_t N, int64_t classes) {
+    const int64_t wide = ceil_div(M, BM) * ceil_div(N, 128);
+    return narrow_tiles(ctx, wide * classes, N) ? ceil_div(M, BM) * ceil_div(N, 64) : wide;
+}
+
 }  // namespace
 
-bool rows_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d) {
-    return shape_ok(ctx, d) && fits(d->n * (d->h + 2 * d->pad_h) * (d->w + 2 * d->pad_w) * d->c);
+// A product of `stages` 64-deep stages on few tiles is one long chain, about 7 +
+// 0.5·stages µs; the column path splits it, after an im2col of 17 µs and 1 µs a MB:
+// [6, 512, 28, 32] → 32, 3×3 stride 2, 72 stages on 11 tiles, 45 µs against 30, [1,
+// 256, 16, 16] → 64 24 against 19; but [8, 256, 28, 28] → 64, 5×5, 59 against 73.
+// Up to 64 output channels the tap kernel (which reads x once where it lies) keeps
+// three cases: many pixels in output planes of whole 1024s, whose channels' stores
+// fall on the same memory channels ([64, 64, 64, 64] → 64, stride 2, 35 µs against
+// 30, [64, 256, 64, 64] 97 against 70; half the images 23 against 26), and one
+// channel chunk on 256 to 384 tiles ([64, 32, 48, 48] 21 against 17, [32, 32, 64, 64]
+// 19 against 16; 10 against 15 at half, 32 against 35 at twice the images); and an
+// input of up to 128 channels that with its copy outgrows the 256 MB of cache ([64,
+// 96, 96, 96] 119 against 99; [64, 64, 112, 112] still 91 against 97).
+bool rows_fwd_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, bool col) {
+    if (!shape_ok(ctx, d) || !fits(d->n * (d->h + 2 * d->pad_h) * (d->w + 2 * d->pad_w) * d->c)) return false;
+    const int64_t M = d->n * p * q, K = d->r * d->s * d->c, stages = ceil_div(K, BK);
+    if (col && row_tiles(ctx, M, d->k, 1) <= 64 && (double)stages > 20 + 4e-6 * (double)(K * M)) return false;
+    const bool same_channels = p * q % 1024 == 0 && M >= 65536, one_chunk = d->c <= 32 && M >= 32768 && M < 49152;
+    const bool past_cache = d->c <= 128 && d->n * d->h * d->w * d->c >= 55000000;
+    return !(d->k <= 64 && (same_channels || one_chunk || past_cache) && tap_fwd_applies(ctx, d, 2));
 }
-bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, size_t elem) {
-    return shape_ok(ctx, d, 16 / (int64_t)elem) && fits(d->n * (d->h + 2 * d->pad_h) * (d->w + 2 * d->pad_w) * d->c);
+// The other paths go through no copies and no partials, whose turn and sum cost
+// about 10 µs a million weights: with few pixels a large gradient is better there.
+// [2, 512, 8, 8] → 512, 3×3 stride 2 (32 pixels) 32 µs against 12 in bf16, 33 against
+// 14 in fp32; with 32 pixels or fewer every one ([1, 32, 8, 8] → 32 12.0 against 7.6
+// fp32, 10.2 against 8.7 bf16).  The lines are where they meet: the column path
+// (whole 64s of pixels) 64 pixels, from 100 thousand weights 128 or the weights over
+// 2300 ([8, 512, 16, 16], 512 pixels, 39 against 33); else 64 pixels from 500
+// thousand weights ([1, 256, 16, 16] fp32 19.7 against 18.4) or the weights over 16000
+// ([1, 512, 14, 14], 5×5, 196 pixels, bf16 74 against 46; 3×3 equal).
+bool rows_wgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, size_t elem, bool col) {
+    if (!shape_ok(ctx, d, 16 / (int64_t)elem) || !fits(d->n * (d->h + 2 * d->pad_h) * (d->w + 2 * d->pad_w) * d->c))
+        return false;
+    const int64_t K = d->n * p * q, MN = d->k * d->c * d->r * d->s;
+    if (col) return K > (MN < 100000 ? 64 : std::max<int64_t>(128, std::min<int64_t>(512, MN / 2300)));
+    return K > std::max<int64_t>(MN < 500000 ? 32 : 64, std::min<int64_t>(256, MN / 16000));
 }
 bool rows_dgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q) {
     if (!shape_ok(ctx, d) || d->stride_h > 2 || d->stride_w > 2) return false;
@@ -661,13 +699,37 @@ bool rows_dgrad_applies(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int6
     // channels 24 µs against 28 with the copy, k = 256 → c = 64 51 against 63; 28×28,
     // k = 512 → c = 128 40 against 42; but k = 64 → c = 256 at 56×56 66 against 41,
     // and planes that are not whole 16 bytes (512 → 512 at 14×14) 73 against 35.
+    // k in odd 32s from 45000 pixels: up to 64 columns (16 images of 64×64, k = 96 →
+    // c = 64 13 against 20; of 28×28 10 against 9), up to 128 where the planes are whole
+    // 1024s of pixels, or k is at least 128 or, below 100000 pixels, 96 (16 images of
+    // 56×56, k = 160 → c = 128 24 against 28; 64 images, k = 32 31 against 34).
     if (d->r == 1 && d->s == 1 && d->stride_h == 1 && d->stride_w == 1 && d->pad_h == 0 && d->pad_w == 0 &&
-        d->c <= 128 && d->k % 64 == 0 && p * q % 8 == 0)
-        return false;
+        d->c <= 128 && p * q % 8 == 0) {
+        if (d->k % 64 == 0) return false;
+        if (d->k % 32 == 0 && d->n * p * q >= 45000 &&
+            (d->c <= 64 || p * q % 1024 == 0 || d->k >= 128 || (d->k >= 96 && d->n * p * q < 100000)) &&
+            tap_dgrad_applies(ctx, d, 2))
+            return false;
+    }
     int64_t lo, hp, wp;
     axis_padding(d->h, p, d->pad_h, d->r, d->stride_h, d->dil_h, lo, hp);
     axis_padding(d->w, q, d->pad_w, d->s, d->stride_w, d->dil_w, lo, wp);
-    return fits(d->n * hp * wp * d->k);
+    if (!fits(d->n * hp * wp * d->k)) return false;
+    // A long chain on few tiles, as in the forward: the tap kernel splits it ([4, 32,
+    // 7, 7], k = 512, 3×3 stride 2, 48 stages on 2 tiles, 33 µs against 17; 24 stages on
+    // 8 tiles 24 against 17, on 56 24 against 31), the other paths past 9 taps are
+    // slower until about 100 stages (200 on 32 tiles 107 against 70, 100 on 15 equal).
+    int64_t stages = 0, tiles = 0;
+    for (int64_t a = 0; a < d->stride_h && a < d->h; ++a) {
+        int64_t pos[kMaxTaps], sh[kMaxTaps], deep = 0;
+        const int nr = axis_taps(a, d->pad_h, d->r, d->stride_h, d->dil_h, pos, sh);
+        for (int64_t b = 0; b < d->stride_w && b < d->w; ++b)
+            deep += ceil_div(nr * axis_taps(b, d->pad_w, d->s, d->stride_w, d->dil_w, pos, sh) * d->k, BK);
+        stages = std::max(stages, deep);
+        tiles += row_tiles(ctx, d->n * ceil_div(d->h - a, d->stride_h) * ceil_div(d->w, d->stride_w), d->c, d->stride_h);
+    }
+    if (d->r * d->s > 9) return stages <= 100 || tiles > 64;
+    return stages < 12 || 20 * stages <= 120 + 11 * tiles || !tap_dgrad_applies(ctx, d, 2);
 }
 
 int rows_fwd(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, const bf16_t* x, const bf16_t* w,
