@@ -36,7 +36,10 @@ LIN = [(1, 1, 1), (7, 5, 3), (64, 3136, 128), (64, 128, 10), (64, 512, 1000), (1
        (384, 192, 256), (136, 64, 64), (4096, 64, 64), (1024, 320, 192),
        # 64x64-tile grids (run_small): forward split over 16 stages with a
        # partial last stage; dW split over 2000 rows, ragged tiles
-       (33, 1000, 17), (2000, 40, 24)]
+       (33, 1000, 17), (2000, 40, 24),
+       # a bf16 backward of which one gradient could run register-staged: both
+       # on the generic engine (the bias gradient from its column of ones)
+       (23, 64, 192), (448, 64, 104)]
 
 
 @pytest.mark.parametrize("dt", DTYPES)
