@@ -60,18 +60,24 @@ def test_linear(ops, oracle, dt, m, kin, nout):
     check(host(db), rdb, "f32" if dt == "f32" else dt, "linear db")
 
 
-# bf16 shapes chosen for the direct-to-LDS GEMM's tile plans, each with
-# partial tiles: (4104, 192, 2056) forward on 256x128 tiles; (2048, 1288,
-# 1544) dW on 256x256 tiles split over K with the fused bias gradient;
-# (1024, 200, 320) dX on unsplit 128x128 and dW split 4 ways; (256, 384, 256)
-# dW unsplit over three tile columns (the bias gradient is summed once);
-# (4100, 2048, 4104) forward on unsplit 256x256 tiles (17 x 17, K = 2048).
+# bf16 shapes chosen for the direct-to-LDS GEMM's tile plans, most with partial
+# tiles: (4104, 192, 2056) forward on 256x256 tiles, dX on 128x128 in 3 splits;
+# (2048, 1288, 1544) and (1024, 200, 320) dW on two 128x128 workgroups per CU in 2
+# and 4 splits with the fused bias gradient; (256, 384, 256) dW unsplit over three
+# tile columns (the bias gradient is summed once); (4100, 2048, 4104) forward on
+# 256x128, dX and dW on unsplit 256x256.
 DMA_LIN = [(4104, 192, 2056), (2048, 1288, 1544), (1024, 200, 320), (256, 384, 256), (4100, 2048, 4104)]
 # k extents that end inside a 64-deep stage (their last stage is zero-filled):
-# odd token counts in dW, whole 8s in the forward and dX; a single partial
-# stage, one step past a stage, 8 short of one; 256x128 (8200 rows), 128x128
-# with two workgroups per CU (1576 -> 3072) and split dW (4001 tokens).
-DMA_LIN += [(129, 136, 128), (1576, 768, 3072), (8200, 328, 264), (4001, 152, 200), (257, 2040, 136)]
+# odd token counts in dW, whole 8s in the forward and dX; a single partial stage
+# and one step past a stage (129 rows and 136 columns), 8 short of one (2040); each
+# tile shape, unsplit and split: 256x128 forward in 3 splits (2640), dW in 2 (2757
+# tokens), 256x256 dX (160), dW in 3 (4173), 128x128 dW in 19 (8200 -> 264).
+DMA_LIN += [(129, 136, 128), (1576, 768, 3072), (8200, 328, 264), (4001, 152, 200), (257, 2040, 136),
+            (1202, 2640, 1568), (2757, 1984, 2008), (2843, 2832, 160), (4173, 2440, 1568)]
+# dW over more than 16 splits, with row sums (16390 rows) and, of few weights, on
+# the generic engine's column of ones; operands of 5 to 22 MB on whole 8s of tiles
+# (each XCD its tiles of all splits) and on 36 tiles.
+DMA_LIN += [(16390, 256, 264), (16384, 1024, 128), (8200, 128, 136), (2056, 1024, 1024), (4096, 768, 768)]
 
 
 def _edge(idx, n):

@@ -390,7 +390,7 @@ template <typename T> __global__ __launch_bounds__(64 * NW) void conv_wgrad_rows
     char NOTT_LDS* smem = (char NOTT_LDS*)smem_raw;
     int32_t NOTT_LDS* lpix = (int32_t NOTT_LDS*)(smem + S * STAGE);
     int pm, pn, z;
-    gemm::dma::tile_of((int)blockIdx.x, (p.M + BM - 1) / BM, (p.N + BN - 1) / BN, p.splits, 4, pm, pn, z);
+    gemm::dma::tile_of((int)blockIdx.x, (p.M + BM - 1) / BM, (p.N + BN - 1) / BN, p.splits, 4, 0, pm, pn, z);
     const int32_t m0 = pm * BM, n0 = pn * BN, kb = z * p.kps, ke = min(p.K, kb + p.kps);
     const int nk = (ke - kb + BK - 1) / BK;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;

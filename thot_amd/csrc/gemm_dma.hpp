@@ -159,12 +159,18 @@ __device__ __forceinline__ void read_all(Frag<TR> (&d)[F], const FragAddr<TR, R,
 // XCD (every eighth) take one contiguous run of the order split-major, then
 // grouped `gm` tile-rows at a time, so that an XCD's L2 serves few k ranges and
 // a compact block of tiles of each.  (With the splits outermost over all XCDs,
-// every XCD read a part of every k range: 3072x1024, K = 8192 in 4 splits.)
-__device__ __forceinline__ void tile_of(int id, int tm, int tn, int splits, int gm, int& pm, int& pn, int& z) {
-    const int nt = tm * tn, all = nt * splits;
-    if ((all & 7) == 0) id = (id & 7) * (all >> 3) + (id >> 3);
-    z = id / nt;
-    id -= z * nt;
+// every XCD read a part of every k range: 3072x1024, K = 8192 in 4 splits.)  Any
+// count is shared out so: 252 workgroups in order, 18 tiles of 768x768, K = 32768 in
+// 14 splits, took 81 us, 52 this way.
+// Where the operands are small (by_tile) an XCD takes the same tiles of all splits:
+// 2048x1024, K = 1024 in 4 splits 19.0 us against 20.1, 512x768, K = 3072 in 8 16
+// against 18; with 61 MB of operands, 512x256, K = 40000 in 32, 33 against 24.
+__device__ __forceinline__ void tile_of(int id, int tm, int tn, int splits, int gm, int by_tile, int& pm, int& pn,
+                                        int& z) {
+    const int nt = tm * tn, all = by_tile ? nt : nt * splits;
+    if (by_tile) z = id / nt, id -= z * nt;
+    id = (id & 7) * (all >> 3) + min(id & 7, all & 7) + (id >> 3);   // the first all % 8 XCDs have one more
+    if (!by_tile) z = id / nt, id -= z * nt;
     const int per_group = gm * tn;
     const int g = id / per_group;
     const int first = g * gm;
@@ -285,18 +291,20 @@ __device__ __forceinline__ void store_tile(const EP& ep, const f32x16 (&acc)[FM]
     }
 }
 
-// grid: tiles (tm·tn) times k splits of kps (a multiple of BK) each.
+// grid: tiles (tm·tn) times k splits of kps (a multiple of BK) each.  TAIL: K is
+// not a multiple of 64 (a test at every fill, and the other fill's addresses, cost 2
+// to 5%: 1080x1000, K = 2368 21.3 us against 20.3 without).
 // ROWSUM: also Σ_k A(m, k) for every row m of the tile (the bias gradient
 // when A is the output gradient of a Linear), summed in fp32 from the A
 // fragments already in registers: only the tiles of tile column 0 sum, and
 // there fragment f's sum is kept by wave column f % WN, so each row is
 // summed once; the two k-halves of a row are held by lanes l and l+32 and
 // combined at the end; the epilogue receives it via ep.rowsum(m, v).
-template <bool AT, bool BT, int BM, int BN, int WM, int WN, int S, bool ROWSUM, class EP>
+template <bool AT, bool BT, int BM, int BN, int WM, int WN, int S, bool ROWSUM, bool TAIL, class EP>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const bf16_t* __restrict__ A, int64_t lda,
                                                              const bf16_t* __restrict__ B, int64_t ldb, EP ep0,
                                                              int64_t M, int64_t N, int64_t K, int64_t kps, int splits,
-                                                             int gm) {
+                                                             int gm, int by_tile) {
     constexpr int NW = WM * WN;
     constexpr int TM = BM / WM, TN = BN / WN;
     constexpr int FM = TM / 32, FN = TN / 32;
@@ -312,7 +320,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const bf16_t* __rest
 
     const int tm = (int)((M + BM - 1) / BM), tn = (int)((N + BN - 1) / BN);
     int pm, pn, z;
-    tile_of((int)blockIdx.x, tm, tn, splits, gm, pm, pn, z);
+    tile_of((int)blockIdx.x, tm, tn, splits, gm, by_tile, pm, pn, z);
     const EP ep = at_split(ep0, z);
     const int64_t m0 = (int64_t)pm * BM, n0 = (int64_t)pn * BN;
     const int64_t kb = (int64_t)z * kps;
@@ -334,7 +342,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const bf16_t* __rest
     auto issue = [&](int t, int slot, int from, int to) {
         char NOTT_LDS* st = smem + slot * STAGE;
         const int64_t k0 = kb + (int64_t)t * BK;
-        if (k0 + BK <= K) {
+        if (!TAIL || k0 + BK <= K) {
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) {
                 if (i < from || i >= to) continue;
@@ -472,41 +480,48 @@ struct Plan {
 // Picks the tile shape and the split-K count with the least estimated time:
 //   rounds of workgroups × (64-deep stages × stage + tile),
 //   stage: idle + load · (how much of the chip's slots is filled), the load
-//   larger where both operands are row-contiguous (both_tr, weight gradients);
+//   another where both operands are row-contiguous (both_tr, weight gradients),
+//   and more with the row sums (rowsum);
 //   tile: the first fill and the output; for a split also the second launch
-//   and the partials' write and read.
-// The constants (us) are a fit to each shape and split forced on 33 products
-// of 512..8192 rows and columns and K = 512..8192 with inputs changing from
-// call to call; the pick is 1.5% off the best of them in the mean (at most 5%).
-// A rule that split whenever there are fewer tiles than CUs took 32 us for
-// 2048x1024x1024 (14.8 now), 18.7 for 1536x768x768 (12.0), 33 for the weight
-// gradient of 1576x768->3072 (28).
-inline Plan plan(nott_ctx ctx, int64_t M, int64_t N, int64_t K, bool both_tr, int64_t splits) {
+//   with a chain over the partials, the partials' write and read, and uneven
+//   splits, of which the 8 XCDs share some (tile_of).
+// The constants (us) are a fit to each shape and split forced on 118 products of
+// 128..65536 rows, 128..8192 columns and K = 64..65536, forward and both gradients,
+// with inputs changing from call to call; the pick is 0.7% off the best of them in
+// the mean (at most 12%).  A pick of at most 16 splits with constants from fewer
+// products was 2.9% off (34%): weight gradients of 16384 tokens, 256 → 256, 20 us
+// against 16, 128 → 1024 23 against 18, of 65536 tokens, 128 → 128, 56 against 20.
+inline Plan plan(nott_ctx ctx, int64_t M, int64_t N, int64_t K, bool both_tr, bool rowsum, int64_t splits) {
     struct Cost {
         Shape shape;
         int bm, bn, per_cu;
-        float idle, load, load_tr, tile;
+        float idle, load, load_tr, rows, tile;
     };
     static constexpr Cost kCosts[] = {
-        {Shape::T256x256, 256, 256, 1, 1.52f, 0.24f, 0.53f, 4.8f},
-        {Shape::T256x128, 256, 128, 1, 0.71f, 0.26f, 0.38f, 4.5f},
-        {Shape::T128x128, 128, 128, 1, 0.63f, 0.09f, 0.53f, 3.2f},
-        {Shape::T128x128x2, 128, 128, 2, 0.61f, 0.45f, 0.49f, 4.6f},
+        {Shape::T256x256, 256, 256, 1, 1.31f, 0.08f, 0.015f, 0.14f, 6.6f},
+        {Shape::T256x128, 256, 128, 1, 0.73f, 0.06f, 0.005f, 0.15f, 4.8f},
+        {Shape::T128x128, 128, 128, 1, 0.50f, 0.14f, 0.03f, 0.51f, 3.0f},
+        {Shape::T128x128x2, 128, 128, 2, 0.70f, 0.50f, 0.27f, 0.00f, 3.0f},
     };
-    constexpr float kSplitUs = 4.2f, kPartialBytesPerUs = 7.85e6f;
+    constexpr float kSplitUs = 1.8f, kUnevenUs = 1.4f, kPartialUs = 0.04f, kPartialRowsUs = 0.21f;
+    constexpr float kPartialBytesPerUs = 5.9e6f;
     const int64_t nkb = ceil_div(K, BK);
     Plan best{Shape::T128x128, 1, K};
     float best_us = 0.f;
     for (const Cost& c : kCosts) {
         const int64_t tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn), slots = (int64_t)ctx->num_cu * c.per_cu;
-        const float load = both_tr ? c.load_tr : c.load;
-        for (int64_t s = 1; s <= 16; ++s) {
+        const float idle = c.idle + (rowsum ? c.rows : 0.f), load = both_tr ? c.load_tr : c.load;
+        // past 16 in steps of a quarter of the power of two below: the best lie in a flat valley
+        for (int64_t s = 1, step = 1; s <= 256; s += step) {
+            if (s >= 16 && (s & (s - 1)) == 0) step = s / 4;
             const int64_t want = splits > 0 ? std::min(splits, std::min<int64_t>(nkb, 65535)) : s;
             if (want > 1 && splits <= 0 && nkb / want < 4) break;
             const int64_t stages = ceil_div(nkb, want), n = ceil_div(nkb, stages);
             const float fill = std::min(1.f, (float)(tiles * n) / (float)slots);
-            float us = (float)ceil_div(tiles * n, slots) * ((float)stages * (c.idle + load * fill) + c.tile);
-            if (n > 1) us += kSplitUs + 8.f * (float)(n * M * N) / kPartialBytesPerUs;
+            float us = (float)ceil_div(tiles * n, slots) * ((float)stages * (idle + load * fill) + c.tile);
+            if (n > 1)
+                us += kSplitUs + (n % 8 && n != 2 && n != 4 ? kUnevenUs : 0.f) + (float)n * (rowsum ? kPartialRowsUs : kPartialUs) +
+                      8.f * (float)(n * M * N) / kPartialBytesPerUs;
             if (best_us == 0.f || us < best_us) {
                 best_us = us;
                 best = Plan{c.shape, n, n > 1 ? stages * BK : K};
@@ -530,10 +545,10 @@ inline bool applies(const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, 
     return ceil_div(M, 128) * ceil_div(N, 128) < (int64_t)1 << 26;   // tiles times splits in an int
 }
 
-template <class Cfg, bool ROWSUM, class EP>
-int launch(nott_ctx ctx, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, const EP& ep, int64_t M,
+template <class Cfg, bool ROWSUM, bool TAIL, class EP>
+int launch_as(nott_ctx ctx, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, const EP& ep, int64_t M,
            int64_t N, int64_t K, int64_t splits, int64_t kps) {
-    auto fn = gemm_kernel<Cfg::kAT, Cfg::kBT, Cfg::kBM, Cfg::kBN, Cfg::kWM, Cfg::kWN, Cfg::kS, ROWSUM, EP>;
+    auto fn = gemm_kernel<Cfg::kAT, Cfg::kBT, Cfg::kBM, Cfg::kBN, Cfg::kWM, Cfg::kWN, Cfg::kS, ROWSUM, TAIL, EP>;
     static bool attr = false;   // one setting per kernel instantiation
     if (!attr) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -542,9 +557,18 @@ int launch(nott_ctx ctx, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t 
         attr = true;
     }
     const int64_t tiles = ceil_div(M, Cfg::kBM) * ceil_div(N, Cfg::kBN);
+    const int64_t bytes = 2 * (M + N) * K;
+    const int by_tile = splits > 1 && tiles % 8 == 0 && bytes >= 5000000 && bytes < 22000000;
     hipLaunchKernelGGL(fn, dim3((unsigned)(tiles * splits)), dim3(Cfg::kThreads), Cfg::kLds, ctx->stream, A, lda, B,
-                       ldb, ep, M, N, K, kps, (int)splits, 4);
+                       ldb, ep, M, N, K, kps, (int)splits, 4, by_tile);
     return launch_status(ctx, "gemm_dma");
+}
+
+template <class Cfg, bool ROWSUM, class EP>
+int launch(nott_ctx ctx, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, const EP& ep, int64_t M,
+           int64_t N, int64_t K, int64_t splits, int64_t kps) {
+    return K % BK ? launch_as<Cfg, ROWSUM, true>(ctx, A, lda, B, ldb, ep, M, N, K, splits, kps)
+                  : launch_as<Cfg, ROWSUM, false>(ctx, A, lda, B, ldb, ep, M, N, K, splits, kps);
 }
 
 template <bool AT, bool BT, bool ROWSUM, class EP>
@@ -573,10 +597,10 @@ int run(nott_ctx ctx, const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb
     if (!applies<AT, BT>(A, lda, B, ldb, M, N, K)) return NOTT_ERR_UNSUPPORTED;
     // The split reduce that also sums rows works on 4-column groups.
     if (ROWSUM && N % 4 != 0) splits = 1;
-    Plan p = plan(ctx, M, N, K, AT && BT, splits);
+    Plan p = plan(ctx, M, N, K, AT && BT, ROWSUM, splits);
     const size_t body = (size_t)(p.splits * M * N), rows = ROWSUM ? (size_t)(p.splits * M) : 0;
     float* ws = p.splits > 1 ? static_cast<float*>(optional_workspace(ctx, sizeof(float) * (body + rows))) : nullptr;
-    if (p.splits > 1 && !ws) p = plan(ctx, M, N, K, AT && BT, 1);   // no room for the partials
+    if (p.splits > 1 && !ws) p = plan(ctx, M, N, K, AT && BT, ROWSUM, 1);   // no room for the partials
     if (p.splits == 1) return launch_shape<AT, BT, ROWSUM>(ctx, p.shape, A, lda, B, ldb, ep, M, N, K, 1, p.kps);
     const int st = launch_shape<AT, BT, ROWSUM>(ctx, p.shape, A, lda, B, ldb, PartialRowStore{ws, ws + body, M, N}, M,
                                                 N, K, p.splits, p.kps);

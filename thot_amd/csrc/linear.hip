@@ -233,6 +233,11 @@ int bwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* dy, cons
         // rows or outputs the generic engine, on 64×64 tiles and with db in its ones
         // column, is faster ([3776, 64] → 1000 30 µs against 47 with the staged dw and its
         // separate column sums; [23, 64] → 832 17 against 19 with the staged dx).
+        // A small dw with db goes there as well: the row sums cost the direct-to-LDS
+        // engine 0.5 us a stage ([2100, 128] → 128 15.4 us against 10.5, [8200, 256] → 192
+        // 20.4 against 17.7; with more rows or weights its wide tiles win, [16390, 256] →
+        // 128 24.9 against 30, [1578, 312] → 864 17 against 20).
+        const bool ones = dw && db && nout * kin <= 50000 && m * nout * kin <= 420000000;
         const bool staged = (!dx || (nout % fast::BK == 0 && kin % 8 == 0)) &&
                             (!dw || (m % fast::BK == 0 && nout % 8 == 0 && kin % 8 == 0));
         if (dx) {
@@ -243,7 +248,7 @@ int bwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* dy, cons
                 dx = nullptr;
             }
         }
-        if (dw && db) {
+        if (dw && db && !ones) {
             // db = Σ_rows dy summed from the dw GEMM's dy fragments.
             DwRowsumStore ep{dw, db, nout, kin, accumulate};
             const int st = dma::run<true, true, true>(ctx, dyp, nout, static_cast<const T*>(x), kin, ep, nout, kin, m);
@@ -253,7 +258,7 @@ int bwd(nott_ctx ctx, int64_t m, int64_t kin, int64_t nout, const void* dy, cons
                 db = nullptr;
             }
         }
-        if (dw) {
+        if (dw && !ones) {
             DwDbStore ep{dw, nullptr, nout, kin, accumulate};
             const int st = bf16_gemm<true, true>(ctx, dyp, nout, static_cast<const T*>(x), kin, ep, nout, kin, m, staged);
             if (st != NOTT_ERR_UNSUPPORTED) {
