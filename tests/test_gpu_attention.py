@@ -79,6 +79,12 @@ CASES = [
     (1, 1, 321, 80, 128, False),
     (1, 1, 320, 81, 120, False),
     (9, 29, 65, 65, 128, False),
+    # head sizes that are not whole 8s: bf16 on the 16x16 kernels as fp32 is, over
+    # several 64-row blocks, ragged, causal and full
+    (1, 2, 150, 150, 20, True),
+    (2, 1, 130, 200, 44, False),
+    (1, 2, 190, 190, 100, True),
+    (1, 1, 257, 70, 100, False),
 ]
 CASES_F32 = [c for c in CASES if c[4] <= 64]   # (fp32 takes head sizes up to 64)
 
@@ -126,6 +132,45 @@ def test_attention_bf16_growing_scores(ops, oracle, case, scale):
     torch.cuda.synchronize()
     check(host(o), ro, "bf16", "o")
     check(host(lse), rlse, "bf16", "lse")
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0])
+@pytest.mark.parametrize("case", [(1, 2, 200, 330, 64, False), (1, 1, 300, 300, 128, True), (1, 1, 150, 150, 32, True)])
+def test_attention_bwd_bf16_scale(ops, oracle, case, scale):
+    """The backward at a negative scale and at none (every score equal: the 16x16 kernels)."""
+    b, h, t, s, dh, causal = case
+    print(f"attention bf16 bwd {case} scale {scale}", flush=True)
+    g = rng(t + s + dh)
+    q, k, v, dO = (host_input(g.standard_normal((b, h, n, dh)), "bf16") for n in (t, s, s, t))
+    d = ops.attn_desc(b, h, t, s, dh, causal, scale=scale)
+    ro, _ = oracle.attention_fwd(d, q, k, v)
+    lse = ops.attention_fwd(dev(q, "bf16"), dev(k, "bf16"), dev(v, "bf16"), d)[1]
+    o = host_input(ro, "bf16")
+    got = ops.attention_bwd(*(dev(a, "bf16") for a in (q, k, v, o, dO)), lse, d)
+    for name, a, w in zip(("dq", "dk", "dv"), got, oracle.attention_bwd(d, q, k, v, o, dO)):
+        check(host(a), w, "bf16", name)
+
+
+@pytest.mark.parametrize("case", [(1, 2, 150, 150, 64, True), (2, 1, 70, 130, 128, False)])
+def test_attention_bf16_off_alignment(ops, oracle, case):
+    """Operands one element past a 16-byte boundary."""
+    b, h, t, s, dh, causal = case
+    print(f"attention bf16 shifted {case}", flush=True)
+    g = rng(t + s + dh)
+    q, k, v, dO = (host_input(g.standard_normal((b, h, n, dh)), "bf16") for n in (t, s, s, t))
+
+    def shifted(a):
+        return torch.empty(a.size + 1, dtype=torch.bfloat16, device="cuda")[1:].view(a.shape).copy_(dev(a, "bf16"))
+
+    d = ops.attn_desc(b, h, t, s, dh, causal)
+    o, lse = ops.attention_fwd(shifted(q), shifted(k), shifted(v), d)
+    ro, rlse = oracle.attention_fwd(d, q, k, v)
+    check(host(o), ro, "bf16", "o")
+    check(host(lse), rlse, "bf16", "lse")
+    o_in = host_input(ro, "bf16")
+    got = ops.attention_bwd(*(shifted(a) for a in (q, k, v, o_in, dO)), lse, d)
+    for name, a, w in zip(("dq", "dk", "dv"), got, oracle.attention_bwd(d, q, k, v, o_in, dO)):
+        check(host(a), w, "bf16", name)
 
 
 def _torch_attention_fp32(q, k, v, dO, causal, scale):

@@ -78,6 +78,8 @@ DMA_LIN += [(129, 136, 128), (1576, 768, 3072), (8200, 328, 264), (4001, 152, 20
 # the generic engine's column of ones; operands of 5 to 22 MB on whole 8s of tiles
 # (each XCD its tiles of all splits) and on 36 tiles.
 DMA_LIN += [(16390, 256, 264), (16384, 1024, 128), (8200, 128, 136), (2056, 1024, 1024), (4096, 768, 768)]
+# output rows that are not whole 16 bytes, stored one element at a time
+DMA_LIN += [(300, 64, 333), (260, 136, 130)]
 
 
 def _edge(idx, n):
@@ -110,6 +112,24 @@ def test_linear_bf16_tile_shapes(ops, oracle, m, kin, nout, accumulate):
     _, rdw, rdb = oracle.linear_bwd(np.ascontiguousarray(dy[:, outs]), x, np.ascontiguousarray(w[outs]))
     check(host(dw)[outs], dw0[outs] + rdw, dt, "dw rows")
     check(host(db)[outs], db0[outs] + rdb, dt, "db rows")
+
+
+@pytest.mark.parametrize("relu_input", [False, True])
+def test_linear_bf16_dx_off_alignment(ops, relu_input):
+    """dx (and with relu_input its mask x) one element past a 16-byte boundary:
+    the same bits as at one."""
+    torch.manual_seed(3)
+    x, w, dy = (torch.randn(s, device="cuda").bfloat16() for s in ((300, 136), (264, 136), (300, 264)))
+
+    def shifted(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+
+    want = ops.linear_bwd(dy, x, w, need_dw=False, need_db=False, relu_input=relu_input)[0]
+    xs = shifted(x) if relu_input else x
+    got = ops.linear_bwd(dy, xs, w, dx=shifted(torch.zeros_like(x)), need_dw=False, need_db=False, relu_input=relu_input)[0]
+    assert got.data_ptr() % 16 == 2 and torch.equal(got, want)
+    got = ops.linear_bwd(dy, xs, w, need_dw=False, need_db=False, relu_input=relu_input)[0]
+    assert torch.equal(got, want)
 
 
 # The FC layer's ReLU in the GEMM epilogues: forward y = relu(x·wᵀ + b), and
@@ -216,7 +236,7 @@ CONV = [
     (2, 32, 70, 70, 32, 3, 3, 1, 1, 1),
     (4, 32, 8, 8, 32, 1, 1, 1, 0, 1),
     (1, 128, 8, 8, 64, 3, 3, 2, 1, 1),
-    (2, 32, 40, 40, 256, 3, 3, 2, 1, 1),       # one channel chunk: the bf16 forward takes the tap kernel unsplit
+    (2, 32, 40, 40, 256, 3, 3, 2, 1, 1),       # one channel chunk, several blocks of output channels
     (3, 3, 30, 26, 64, 7, 7, 2, 3, 1),         # stem forward kernel: odd output sizes, tiles across images
     (1, 16, 66, 70, 64, 3, 3, 1, 1, 1),        # tap weight gradient at stride 1 (rows wider than the 3x3 kernel's)
 ]
@@ -351,6 +371,7 @@ CONV_LINES = [
     (2, 24, 8, 8, 32, 3, 3, 2, 1, 1), (2, 24, 9, 8, 32, 3, 3, 2, 1, 1),
     (8, 256, 6, 6, 512, 3, 3, 2, 1, 1), (5, 256, 8, 8, 512, 3, 3, 2, 1, 1),
     (8, 256, 16, 16, 512, 3, 3, 2, 1, 1), (9, 256, 16, 16, 512, 3, 3, 2, 1, 1),
+    (21, 72, 56, 56, 136, 3, 3, 2, 1, 1), (64, 128, 56, 56, 256, 3, 3, 2, 1, 1),   # 128-column tiles, ragged and whole
 ]
 
 

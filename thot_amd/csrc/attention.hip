@@ -1576,7 +1576,7 @@ int bwd_ns(nott_ctx ctx, const nott_attn_desc* d, const AttnParams& p, const voi
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_dq_kernel<T, NS, EXACT>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_q);
     // fp32: rowsum(do∘o) from o; bf16: the dq pass forms it exactly and runs first.
-    if (!EXACT)
+    if constexpr (!EXACT)
         hipLaunchKernelGGL(attn_dsum_kernel<T>, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, ctx->stream,
                            static_cast<const T*>(o), static_cast<const T*>(dO), dsum, rows, p);
     hipLaunchKernelGGL((attn_dq_kernel<T, NS, EXACT>), dim3(bh, (unsigned)p.nqb), dim3(kThreads), lds_q, ctx->stream,

@@ -823,9 +823,11 @@ int rows_wgrad(nott_ctx ctx, const nott_conv2d_desc* d, int64_t p, int64_t q, co
     const int64_t taps = d->r * d->s;
     const int64_t M = d->k, N = taps * d->c, K = d->n * p * q;
     const int64_t tiles = ceil_div(M, BM) * ceil_div(N, 128), nkb = ceil_div(K, BK);
-    // Splits: the 128×128 tile's estimate in gemm_dma.hpp's plan, and 0.04 µs a
-    // split for the sum over a small result's partials ([16, 96, 40, 40], 1×1, 96
-    // outputs: 25 µs at 64 splits, 30 at 200); at most kMaxPixels pixels each.
+    // Splits: rounds of workgroups × (stages × a stage + 3.2 µs), the partials' write
+    // and read, and 0.04 µs a split for the sum over a small result's partials ([16,
+    // 96, 40, 40], 1×1, 96 outputs: 25 µs at 64 splits, 30 at 200); at most kMaxPixels
+    // pixels each.  A stage is 0.6 to 1.2 µs in bf16 (loads), 2.1 in fp32: its MFMAs
+    // alone are 128·128·32 multiply-adds at 128 a cycle, 1.7 µs at 2.4 GHz.
     int64_t stages = 0;
     float best = 0.f;
     for (int64_t s = 1; s <= std::max<int64_t>(ctx->num_cu, ceil_div(K, kMaxPixels)); ++s) {
