@@ -51,15 +51,15 @@ TRAFFIC = {
     ("conv_bwd", "f32", "wgrad"): 385.08e6,    # conv3x3_wgrad + conv3x3_wgrad_reduce
     ("conv_bwd", "bf16", "dgrad"): 182.82e6,
     ("conv_bwd", "bf16", "wgrad"): 230.20e6,
-    ("ln_bwd", "f32", "all"): 206.31e6,        # ln_bwd_kernel + col_reduce_grouped_kernel
-    ("ln_bwd", "bf16", "all"): 105.54e6,
+    ("ln_bwd", "f32", "all"): 206.30e6,        # ln_bwd_kernel + col_reduce_grouped_kernel
+    ("ln_bwd", "bf16", "all"): 105.51e6,
     ("adamw", "f32", "all"): 2799.95e6,
     ("adamw", "bf16", "all"): 2200.00e6,
     ("xent", "f32", "all"): 4200.27e6,         # xent_count_kernel + xent_rows_vec_kernel
     ("xent", "bf16", "all"): 2101.67e6,
-    ("mha_bwd", "bf16", "out_proj"): 194.04e6,   # dA GEMM + dW_o split GEMM + reduce
-    ("mha_bwd", "bf16", "attention"): 241.85e6,  # attn_dq64 + attn_dkdv64
-    ("mha_bwd", "bf16", "in_proj"): 480.57e6,    # dX GEMM + dW_qkv split GEMM + reduce
+    ("mha_bwd", "bf16", "out_proj"): 156.17e6,   # dA GEMM + dW_o split GEMM + reduce
+    ("mha_bwd", "bf16", "attention"): 239.05e6,  # attn_dq32 + attn_dkdv32
+    ("mha_bwd", "bf16", "in_proj"): 367.88e6,    # dX GEMM + dW_qkv split GEMM + reduce
 }
 
 

@@ -285,12 +285,13 @@ int nott_layernorm_bwd(nott_ctx ctx, nott_dtype dtype, int64_t rows, int64_t d,
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
  * Same arguments and results as nott_layernorm_bwd (the same kernels); the
  * dgamma/dbeta column partials live in a static 16 MiB device array, one per
- * GPU, instead of the context workspace.  That bounds the problem.  On the
- * vector path (d <= 2048 and a multiple of 8 bf16 / 4 fp32 elements, every
- * row pointer 16-byte aligned) the partials take 2·16·ceil(d/16)·4 bytes for
- * each of at most (number of CUs) blocks, at most 4 MiB on a 256-CU MI355X,
- * so every row count fits.  Otherwise the generic path needs 8·d·rows bytes
- * (rows·d <= 2^21 elements).  Larger problems return NOTT_ERR_UNSUPPORTED
+ * GPU, instead of the context workspace.  That bounds the problem.  Rows of
+ * d <= 2048, a multiple of 8 bf16 / 4 fp32 elements, with every row pointer
+ * 16-byte aligned, are taken at any count: the partials are 2·16·ceil(d/16)·4
+ * bytes for each of at most (number of CUs) blocks, at most 4 MiB on a 256-CU
+ * MI355X.  Others are taken up to 8·d·rows <= 16 MiB (rows·d <= 2^21), which
+ * is what rows past 16384 columns need; up to 16384 columns the partials are
+ * per block as above and smaller.  Larger problems return NOTT_ERR_UNSUPPORTED
  * with the sizes in the message.  Every call on a GPU
  * shares that GPU's array: calls that overlap on one GPU (two streams, two
  * contexts) race.  The partials are written in full before they are read,

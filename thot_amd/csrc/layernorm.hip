@@ -12,7 +12,8 @@
 // and dy stay in VGPRs, the row sums are DPP wave reductions (and one LDS
 // exchange where several waves share a row), and every lane keeps running
 // dγ / dβ sums for its columns over the rows it takes.  Blocks write per-block
-// column partials; a second kernel reduces them (deterministic order).
+// column partials; a second kernel reduces them (deterministic order).  Longer
+// rows: a block per row, three passes over it, partials per row.
 #include "common.hpp"
 
 #include <mutex>
